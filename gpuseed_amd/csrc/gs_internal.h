@@ -96,11 +96,10 @@ struct PersistCold {
   uint4* dyn_items;
   uint4* dyn_meta;
   uint32_t* dyn_link;
-  uint32_t* dyn_ready;
-  uint32_t* dyn_ctl;
+  uint32_t* reserved;
   uint4* wmeta;
   uint32_t* wlink;
-  uint32_t seg_tasks, epoch;
+  uint32_t seg_tasks, pad;
 };
 constexpr uint32_t kCounterBytes = 32;   // four 64-bit counters
 constexpr uint32_t kColdBytes = 256;     // PersistCold, after the counters
@@ -120,7 +119,7 @@ struct PersistParams {
   uint32_t* nR;
   uint4* seg_meta;           // per item of a segmented read: {emitted, first b, last b, flags}
   uint32_t* seg_link;        // per item of a segmented read: first piece split off it, or ~0
-  uint32_t* queue;           // work-queue counter
+  uint32_t* queue;           // [0] the next item to hand out, [1] pieces reserved
   uint64_t* counters;        // optional: [0] table reads, [1] occ entry reads, [2] direct-extension reads,
                              // [3] tandem-table reads
   uint32_t direct_min;       // size-1 steps before a task reads the text (0: no direct extension)
@@ -128,14 +127,9 @@ struct PersistParams {
   uint4* dyn_items;          // pieces {read, strand, first task, tasks}
   uint4* dyn_meta;           // per piece, as seg_meta
   uint32_t* dyn_link;        // per piece: the next piece in task order, or ~0
-  uint32_t* dyn_ready;       // per piece: == epoch once its entry is written (cleared per launch)
-  uint32_t* dyn_ctl;         // [0] pieces reserved, [64] next piece to claim, [kRunBase + kRunStride * i]
-                             // items running, counter i of kRunSlots (kDynCtlWords words)
   uint4* wmeta;              // per whole-read stream (2 * read + strand) that was split
   uint32_t* wlink;
-  uint32_t dyn_cap, split_work, split_tasks, epoch;
-  uint32_t split_below;           // split only while fewer items than this run (set at launch)
-  uint32_t refill_group;          // idle lanes of a wave that trigger a refill (set at launch)
+  uint32_t dyn_cap, split_work, split_tasks;
   uint32_t tandem;                // tandem jumps: largest period (0: off; needs the index's tandem table)
 };
 
@@ -161,36 +155,18 @@ struct JoinParams {
 };
 
 constexpr uint32_t kSplitStream = 0xFFFFFFFFu;  // nF/nR of a whole-read stream left for join_whole
-// Work splitting by default only in batches of at most this many items per
-// lane of the persistent grid: on the 3.1 Gbp index, 80,000 150 bp reads
-// (0.6 items per lane) 7.5 ms with splitting, 11 ms without; 160,000 (1.2 per
-// lane) 18.8 and 10.7 ms; 10,000 mixed-length reads (1.6 per lane) 7.5 and
-// 6.2 ms.
-constexpr uint32_t kSplitItemsPerLane = 1;
-// Split thresholds for reads held whole in the LDS window (memory operations,
-// task ends); the options' values apply when smaller.  A launch of 10,000
-// 150 bp reads on the 3.1 Gbp index: 8.8 ms with the defaults of long reads
-// (2048, 8), 3.7 ms with (128, 4), 3.6 ms with (64, 2); 40,000 reads: 8.8,
-// 4.9 and 9.7 ms.  Long reads' segments keep the options' values: with
-// (128, 4) for every item a mixed-length launch of 10,000 reads took 12.9
-// against 9.3 ms.
-constexpr uint32_t kSplitWorkWhole = 128;
-constexpr uint32_t kSplitTasksWhole = 4;
-// The running-items count of work splitting, spread over kRunSlots counters
-// 128 bytes apart: waves add to counter (wave mod kRunSlots), readers sum
-// them.  One counter, folded once per wave and iteration, serialised every
-// wave's atomics on one address: 10,000 mixed-length reads took 9.1 ms per
-// launch with splitting on against 6.3 ms with it off.
-constexpr uint32_t kRunBase = 128, kRunStride = 32, kRunSlots = 16;
-constexpr uint32_t kDynCtlWords = kRunBase + kRunStride * kRunSlots;
-// Waves that wait for split-off pieces once they have nothing to do: one in
-// kPollerEvery (about one per CU); the others leave at their first poll
-// that finds no piece.  On the 3.1 Gbp index, 80,000 150 bp reads: 8.0 ->
-// 7.0 ms per launch; 2,000 mixed-length reads: 4.5 -> 3.8 ms.  (Forced on
-// in a launch of 2,000,000 150 bp reads, 15 items per lane, splitting after
-// 128 operations makes it twice as long, 51 against 23 ms: the pieces start
-// without size records; the default keeps it off at that size.)
-constexpr uint32_t kPollerEvery = 16;
+// Work splitting (take_pieces): a lane gives half of its task ends away after
+// kSplitWork memory operations (at once in a launch of fewer items than
+// lanes), while it has at least 2 * kSplitTasks of them left, and once
+// kSplitIdle lanes of its wave are idle (any idle lane, in a small launch).
+constexpr uint32_t kSplitWork = 64;
+constexpr uint32_t kSplitTasks = 4;
+constexpr uint32_t kSplitIdle = 32;
+// Pieces a launch can split off (36 bytes each): 8 per item, at least 65,536,
+// at most 2^20; beyond that items go on whole.
+__host__ inline uint32_t piece_cap(uint64_t n_items) {
+  return (uint32_t)(n_items >= (1u << 17) ? 1u << 20 : (n_items < 8192 ? 65536 : 8 * n_items));
+}
 constexpr uint32_t kRefillGroup = 12;           // idle lanes of a wave that trigger a refill
                                                 // (2.5M 150 bp reads, 3.1 Gbp index, an early
                                                 // form of the kernel: 1 lane 72.5 ms, 4: 58.0 ms,

@@ -21,24 +21,19 @@
 //  * text chunks are compared by the whole wave, one loading lane at a time;
 //  * work splitting: the cost of a stream is heavy-tailed (in young repeat
 //    families interval sizes shrink at every step, so distance-1 pruning
-//    never stops a task and each task walks far).  Once the main queue is
-//    exhausted and fewer items run than half the lanes, an item that has used
-//    split_work memory operations since it started or last split, and still
-//    has at least 2 * split_tasks task ends to do (for reads held whole in
-//    the LDS window at most kSplitWorkWhole and kSplitTasksWhole), hands half
-//    of them to an
-//    overflow queue, which idle lanes take (a piece starts without size
-//    records, so splitting while every lane is busy would only add work);
-//    the join kernels put the pieces back in task order and settle the
-//    SMEM filter at their boundaries, as for the segments of long reads.
-//    A split keeps the upper half of the remaining task ends in the lane
-//    (with its size records) and pushes the lower half as one piece, which
-//    may split again; pieces are chained in task order.  Lanes never wait
-//    for one another: a piece is written by the lane that reserved it in the
-//    same iteration, a lane that claimed a piece whose entry is not visible
-//    yet checks again next iteration, and a lane leaves once the main queue
-//    is exhausted, no piece is left to claim and no item is running anywhere
-//    (so no piece can appear any more).
+//    never stops a task and each task walks far), and a launch ends with its
+//    longest items.  Once the queue is exhausted, the idle lanes of a wave
+//    take the lower half of the task ends that a busy lane of the same wave
+//    still has to do, with its code window and size records (copied in LDS:
+//    records of larger task ends prune smaller ones exactly as in one lane).
+//    Pieces split again, so a wave's remaining work spreads over its 64
+//    lanes within a few iterations; nothing is shared between waves, polled
+//    or waited for.  The join kernels put the pieces back in task order and
+//    settle the SMEM filter at their boundaries, as for the segments of long
+//    reads: pieces are chained in task order.
+//  * a launch of fewer items than lanes gives every wave its share of them
+//    at once (one item per wave at first, if there are fewer than waves) and
+//    splits them from the start.
 #include <algorithm>
 #include <type_traits>
 
@@ -91,12 +86,19 @@ __device__ __forceinline__ uint4 slot_chunk(uint4 v) {
   return make_uint4((uint32_t)rv, (uint32_t)(rv >> 32), __builtin_bitreverse32(fb), 0u);
 }
 
-__device__ __forceinline__ uint32_t load_acquire(const uint32_t* p) {
-  return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void store_release(uint32_t* p, uint32_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+// index of the n-th set bit of m (n < popcount(m))
+__device__ __forceinline__ uint32_t nth_bit(uint64_t m, uint32_t n) {
+  uint32_t at = 0;
+#pragma unroll
+  for (uint32_t w = 32; w; w >>= 1) {
+    const uint32_t c = (uint32_t)__popcll(m & ((1ull << w) - 1ull));
+    if (n >= c) {
+      n -= c;
+      at += w;
+      m >>= w;
+    }
+  }
+  return at;
 }
 
 // The persistent kernel's arguments: what its loop reads on every
@@ -108,7 +110,7 @@ struct PersistArgs {
   const gs::PersistCold* cold;
   uint32_t* queue;
   uint64_t n_items;
-  uint32_t k, smem, direct_min, dyn_cap, split_work, split_tasks, split_below, refill_group, tandem;
+  uint32_t k, smem, direct_min, dyn_cap, split_work, split_tasks, split_idle, refill_group, take, tandem;
 };
 
 // Waves per SIMD the register allocation must allow: 4 for the 4-bit
@@ -168,28 +170,11 @@ seed_persistent(PersistArgs P) {
   const uint32_t L2_0 = P.X.L2[0], L2_1 = P.X.L2[1], L2_2 = P.X.L2[2], L2_3 = P.X.L2[3];
   const uint32_t primary = P.X.primary;
   const uint64_t n_items = P.n_items;
-  // three control words, 256 bytes apart (separate cache lines and channels):
-  // pieces reserved by splitting lanes, the next piece to claim, items being
-  // processed
   const gs::PersistCold* const C = P.cold;
-  auto reserved = [&]() __attribute__((always_inline)) { return C->dyn_ctl; };
-  auto next_piece = [&]() __attribute__((always_inline)) { return C->dyn_ctl + 64; };
-  // items running: one counter per group of waves (gs::kRunSlots of them,
-  // 128 bytes apart), so that no single address takes every wave's atomics;
-  // a wave adds to its own and reads the total with one load per lane
-  auto run_slot = [&]() __attribute__((always_inline)) -> uint32_t* {
-    const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * BS + threadIdx.x) >> 6);
-    return C->dyn_ctl + gs::kRunBase + gs::kRunStride * (wave % gs::kRunSlots);
-  };
-  auto running_total = [&]() __attribute__((always_inline)) -> uint32_t {
-    uint32_t v = lane < (int)gs::kRunSlots ? __hip_atomic_load(C->dyn_ctl + gs::kRunBase + gs::kRunStride * lane,
-                                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                           : 0u;
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-  };
 
-  bool have = false, finished = false, main_done = false;
+  bool have = false;
+  bool drained = false;  // wave-uniform: the queue has no item left for this wave
+  bool splitting = P.dyn_cap != 0;  // wave-uniform
   int kind = 0;  // 0: a whole read's stream, 1: a segment of a long read, 2: a split-off piece
   uint32_t r = 0, strand = 0, L = 0, nout = 0, last_b = 0;
   // the 22 codes left of the task end e: code(e-1-j) at bits 2j of wcode for
@@ -211,12 +196,6 @@ seed_persistent(PersistArgs P) {
   uint32_t l = 0, u = 0, b = 0, cx = 0;
   int32_t e = 0, x = 0, e_min = 0, w0 = 0;
   uint32_t t0 = 0, first_b = 0, flags = 0, work = 0;
-  uint32_t pending = kNone;                                // claimed piece not visible yet
-  int32_t drun = 0;                                         // items started minus ended this iteration
-  uint32_t poll_wait = 0;                                   // wave-uniform: iterations to the next poll
-  uint32_t fold_wait = 0;                                   // wave-uniform: iterations since the count was folded
-  bool in_tail = false;                                     // wave-uniform: items split (work splitting on)
-  uint32_t backoff = 1;                                     // wave-uniform: sleeps while all lanes wait
   uint32_t link = kNone;                                   // first piece split off this item
   uint32_t item = 0;  // index of the item (or piece) in its list
   int phase = 0;
@@ -311,28 +290,6 @@ seed_persistent(PersistArgs P) {
       (strand ? C->nR : C->nF)[r] = nout;
     }
     have = false;
-    --drun;  // folded into `running` once per wave and iteration
-  };
-  // Hands the lower half of the task ends still to do (e-1 .. e_min) to the
-  // overflow queue as one piece and keeps the upper half, whose size records
-  // this lane holds; the piece is linked right after this item's own tasks
-  // (ahead of pieces split off earlier, which cover later task ends).  False
-  // if the queue is full (then the item goes on whole).
-  auto split = [&]() __attribute__((always_inline)) -> bool {
-    const uint32_t n_rem = (uint32_t)(e - e_min);
-    const uint32_t n_push = n_rem / 2;
-    if (__hip_atomic_load(reserved(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= P.dyn_cap) return false;
-    const uint32_t id = atomicAdd(reserved(), 1u);
-    if (id >= P.dyn_cap) return false;  // reserved past the end: nothing to write, nobody claims it
-    const uint32_t t_first = L - (uint32_t)(e_min + (int32_t)n_push - 1);  // task index of end e_min + n_push - 1
-    C->dyn_items[id] = make_uint4(r, strand, t_first, n_push);
-    C->dyn_link[id] = link;  // initial value: the piece's own successor
-    __threadfence();
-    store_release(C->dyn_ready + id, C->epoch);
-    link = id;
-    e_min += (int32_t)n_push;
-    work = 0;
-    return true;
   };
   // At a task's start: a jump (phase 6, the table entry in tq) while the
   // open stretch reaches kTandemMin codes left of e; with no stretch open,
@@ -406,14 +363,6 @@ seed_persistent(PersistArgs P) {
     phase = 0;
     ext_miss = false;
     ones = 0;
-    // split only in the tail (in_tail: the main queue is exhausted and fewer
-    // items run than half the lanes), so pieces find idle lanes instead of
-    // adding work; reads held whole in the window (and pieces of them) split
-    // sooner: their pieces reload only the read's few code chunks
-    const bool whole = L <= (uint32_t)LMAX;
-    const uint32_t sw = whole ? min(P.split_work, gs::kSplitWorkWhole) : P.split_work;
-    const uint32_t stk = whole ? min(P.split_tasks, gs::kSplitTasksWhole) : P.split_tasks;
-    if (in_tail && work > sw && e - e_min >= 2 * (int32_t)stk) split();
     // the next task end: past those whose windows the last probe found
     // absent (their windows are clean), then past 13-base windows holding a
     // code above 3, jumping below the highest such code at once
@@ -502,15 +451,40 @@ seed_persistent(PersistArgs P) {
     }
     return oc == 1 ? 2 : 3;  // nothing is emitted, so the row is not needed
   };
-  // Loads task ends e_hi .. e_hi - tcount + 1 of stream (r, strand) into the
-  // lane: the LDS code window [w0, top) covers every task's 13-base start.
-  auto start_item = [&](uint32_t tstart, uint32_t tcount, uint32_t link0) __attribute__((always_inline)) {
+  // An item's (or piece's) state for its task ends e_hi .. e_hi - tcount + 1,
+  // its LDS slot in place.
+  auto begin_item = [&](int32_t e_hi, uint32_t tcount, uint32_t link0) __attribute__((always_inline)) {
+    nout = 0;
+    last_b = 0xFFFFFFFFu;
+    first_b = 0xFFFFFFFFu;
+    flags = 0;
+    work = 0;
+    link = link0;  // set before the item can end (a piece whose windows all hold an N ends here)
+    e = e_hi;
+    e_min = e - (int32_t)tcount + 1;
+    load_window(e);
+    have = true;
+    phase = 0;
+    ext_miss = false;
+    ones = 0;
+    probe = false;
+    known_e = -1;
+    known_m = 0;
+    b = (uint32_t)e;
+    tp = 0;
+    need_next = (wbad & kBad13) != 0;
+    if (tandem_on && !need_next) t_start();
+  };
+  // Loads the slot for the tcount task ends from task t0 on of stream
+  // (r, strand): the LDS code window [w0, top) covers every task's 13-base
+  // start.
+  auto load_slot = [&](uint32_t code0) __attribute__((always_inline)) {
     const uint32_t nch = (L + 31) >> 5;
-    gcodes = (uint32_t)C->code_off[r] + strand * nch;
+    gcodes = code0 + strand * nch;
     const uint4* src = P.codes + gcodes;
     uint32_t top;
-    t0 = tstart;
-    if (L <= (uint32_t)LMAX) {  // the whole stream fits the window
+    const bool whole = L <= (uint32_t)LMAX;  // pack_codes wrote its chunks in the slot's form
+    if (whole) {  // the whole stream fits the window
       top = nch << 5;
       w0 = 0;
     } else {
@@ -522,189 +496,158 @@ seed_persistent(PersistArgs P) {
     // q = LMAX/32 - 1 - (c - c0)
     const uint32_t c0 = (uint32_t)w0 >> 5, c1 = top >> 5;
     uint32_t* cw = reinterpret_cast<uint32_t*>(lds + sbase + A_BYTES);
-    const bool whole = L <= (uint32_t)LMAX;  // pack_codes wrote its chunks in the slot's form
-    for (uint32_t c = c0; c < c1; ++c) {
-      uint4 v = src[c];
-      if (!whole) v = slot_chunk(v);
-      const uint32_t q = (uint32_t)(LMAX / 32 - 1) - (c - c0);
-      cw[2 * q] = v.x;
-      cw[2 * q + 1] = v.y;
-      cw[CW + q] = v.z;
+    // all of the window's chunks are loaded before the first is used: one
+    // memory latency per item (a wave refills about every seven iterations)
+    uint4 v[LMAX / 32];
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)(LMAX / 32); ++i)
+      if (c0 + i < c1) v[i] = src[c0 + i];
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)(LMAX / 32); ++i) {
+      if (c0 + i < c1) {
+        if (!whole) v[i] = slot_chunk(v[i]);
+        const uint32_t q = (uint32_t)(LMAX / 32 - 1) - i;
+        cw[2 * q] = v[i].x;
+        cw[2 * q + 1] = v[i].y;
+        cw[CW + q] = v[i].z;
+      }
     }
     cw[CW - 2] = 0;
     cw[CW - 1] = 0;
     cw[CW + BW - 1] = 0xFFFFFFFFu;  // left of the read start (a segment's reads left of w0 go to device memory)
     const uint32_t za = ((top - (uint32_t)w0) * (uint32_t)RB / 8 + 15) >> 4;
     for (uint32_t c = 0; c < za; ++c) *reinterpret_cast<uint4*>(lds + sbase + 16 * c) = make_uint4(0, 0, 0, 0);
-    out = C->cand + 2 * C->task_off[r];
-    nout = 0;
-    last_b = 0xFFFFFFFFu;
-    first_b = 0xFFFFFFFFu;
-    flags = 0;
-    work = 0;
-    link = link0;  // set before the item can end (a piece whose windows all hold an N ends here)
-    e = (int32_t)(L - t0);
-    e_min = e - (int32_t)tcount + 1;
-    load_window(e);
-    have = true;
-    ++drun;
-    phase = 0;
-    ext_miss = false;
-    ones = 0;
-    probe = false;
-    known_e = -1;
-    known_m = 0;
-    b = (uint32_t)e;
-    tp = 0;
-    need_next = (wbad & kBad13) != 0;  // no work done yet, so this never splits
-    if (tandem_on && !need_next) t_start();
   };
-  auto start_main = [&](uint64_t it) __attribute__((always_inline)) {
+  // The item `it` of the queue into this lane; its number of task ends, 0 if
+  // it has none.
+  auto load_main = [&](uint64_t it) __attribute__((always_inline)) -> uint32_t {
     item = (uint32_t)it;
     const uint64_t v = C->items[it];
     r = (uint32_t)v;
     strand = (uint32_t)(v >> 32) & 1u;
     const uint32_t seg = (uint32_t)(v >> 33);
     L = C->lens[r];
+    const uint32_t code0 = (uint32_t)C->code_off[r];
+    out = C->cand + 2 * C->task_off[r];
     if (L < k) {
       (strand ? C->nR : C->nF)[r] = 0;
-      return;
+      return 0;
     }
-    // one call site of start_item for both kinds (it is long)
-    uint32_t ts = 0, tc = L - k + 1;
+    t0 = 0;
+    uint32_t tc = L - k + 1;
     kind = 0;
     if (L > (uint32_t)LMAX) {
       kind = 1;
-      ts = seg * C->seg_tasks;
-      tc = min(C->seg_tasks, L - k + 1 - ts);
+      t0 = seg * C->seg_tasks;
+      tc = min(C->seg_tasks, tc - t0);
     }
-    start_item(ts, tc, kNone);
+    load_slot(code0);
+    return tc;
   };
-  auto start_piece = [&](uint32_t id) __attribute__((always_inline)) {
-    const uint4 d = C->dyn_items[id];
-    const uint32_t lk = C->dyn_link[id];
-    item = id;
+  // the lanes that can give work away, if enough lanes are idle to take it
+  auto can_give = [&]() __attribute__((always_inline)) -> uint64_t {
+    if ((uint32_t)__popcll(__ballot(!have)) < P.split_idle) return 0;
+    return __ballot(have && work >= P.split_work && e - e_min >= 2 * (int32_t)P.split_tasks);
+  };
+  // Idle lanes of a wave whose queue is exhausted take work from its busy
+  // lanes (why: a launch ended with its slowest items, alone in their waves
+  // at 2-4 us per operation; 1,000,000 150 bp reads on the 3.1 Gbp index
+  // spent 12 of 18 ms so, 64 reads on a 100 Mbp index all of their 2.4 ms;
+  // with this, 7.4 and 0.25 ms): each of the first n busy lanes that have used split_work memory
+  // operations since they started or last split, and still have at least
+  // 2 * split_tasks task ends after the current one, gives the lower half of
+  // them to an idle lane, as a piece linked right after its own tasks (ahead
+  // of pieces split off earlier, which cover later task ends).  The piece
+  // starts from the giving lane's slot: its codes, and its size records,
+  // which come from larger task ends and so prune the piece's as they would
+  // prune the lane's own.  Returns the taken piece's task ends, 0 for a lane
+  // that takes none.  Every lane of the wave takes part.
+  auto take_pieces = [&]() __attribute__((always_inline)) -> uint32_t {
+    const uint64_t giving = can_give();
+    if (!giving) return 0;
+    const uint64_t idle = __ballot(!have);
+    const uint32_t n_rem = (uint32_t)(e - e_min);  // of a lane that gives
+    uint32_t n = min((uint32_t)__popcll(idle), (uint32_t)__popcll(giving));
+    uint32_t id0 = 0;
+    if (lane == 0) id0 = atomicAdd(C->reserved, n);
+    id0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)id0);
+    if (id0 + n > P.dyn_cap) {  // no room for more pieces: items go on whole
+      splitting = false;
+      n = id0 < P.dyn_cap ? P.dyn_cap - id0 : 0u;
+    }
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint32_t rank = (uint32_t)__popcll((have ? giving : idle) & below);
+    const bool give = ((giving >> lane) & 1u) && rank < n;
+    const bool get = !have && rank < n;
+    const uint32_t n_push = n_rem >> 1;
+    const int from = get ? (int)nth_bit(giving, rank) : lane;
+    const uint32_t g_r = __shfl(r, from), g_strand = __shfl(strand, from), g_L = __shfl(L, from);
+    const int32_t g_emin = __shfl(e_min, from), g_w0 = __shfl(w0, from);
+    const uint32_t g_push = __shfl(n_push, from), g_link = __shfl(link, from), g_codes = __shfl(gcodes, from);
+    const uint64_t g_out = __shfl((uint64_t)out, from);
+    if (give) {
+      link = id0 + rank;
+      e_min += (int32_t)n_push;
+      work = 0;
+    }
+    if (!get) return 0;
+    r = g_r;
+    strand = g_strand;
+    L = g_L;
+    w0 = g_w0;
+    gcodes = g_codes;
+    out = reinterpret_cast<uint4*>(g_out);
+    link = g_link;
     kind = 2;
-    r = d.x;
-    strand = d.y;
-    L = C->lens[r];
-    start_item(d.z, d.w, lk);  // pieces split off this one go in front of its successor
+    item = id0 + rank;
+    t0 = L - (uint32_t)(g_emin + (int32_t)g_push - 1);  // task index of end e_min + n_push - 1
+    C->dyn_items[item] = make_uint4(r, strand, t0, g_push);
+    const uint4* src = reinterpret_cast<const uint4*>(lds + ((threadIdx.x & ~63u) + (uint32_t)from) * SLOT);
+    uint4* dst = reinterpret_cast<uint4*>(lds + sbase);
+#pragma unroll
+    for (int q = 0; q < SLOT / 16; ++q) dst[q] = src[q];
+    return g_push;
   };
-  // items started minus items ended since the wave's last fold, one atomic
-  // per wave every 32 iterations, and at once when the wave has no item
-  // (its count is then final); a split pushes its pieces (and fences) before
-  // its item ends.  A wave's folded total never falls below zero (its items'
-  // starts are folded no later than their ends), and a count that lags only
-  // delays the split trigger or keeps waiting lanes polling a little longer.
-  auto fold_running = [&]() __attribute__((always_inline)) {
-    if ((++fold_wait & 31u) && __ballot(have) != 0) return;
-    // the split trigger's state for the wave: the main queue is exhausted (a
-    // lane of the wave found it so) and fewer items run than split_below
-    const uint32_t total = running_total();
-    in_tail = __ballot(main_done) != 0 && total < P.split_below;
-    if (__ballot(drun != 0) == 0) return;
-    int d = drun;
-    drun = 0;
-    for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
-    if (lane == 0 && d) atomicAdd(run_slot(), (uint32_t)d);
-  };
-  // overflow queue, polled by one lane per wave: claims pieces for the
-  // wave's idle lanes with one CAS, or finds that none can come any more.
-  // Relaxed loads only (an early exit is always safe: a lane that splits
-  // its item takes its own pieces if nobody else does).
-  auto poll_pieces = [&]() __attribute__((always_inline)) {
-    const bool idle = !have && !finished && main_done && pending == kNone;
-    const uint64_t idlemask = __ballot(idle);
-    if (!idlemask) return;
-    if (poll_wait) {
-      --poll_wait;
-      return;
-    }
-    const int leader = __ffsll((unsigned long long)idlemask) - 1;
-    uint32_t got = 0, first = 0, none = 0, empty = 0;
-    if (lane == leader) {
-      const uint32_t nx = __hip_atomic_load(next_piece(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const uint32_t rs = __hip_atomic_load(reserved(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const uint32_t lim = rs < P.dyn_cap ? rs : P.dyn_cap;
-      if (nx < lim) {
-        const uint32_t want = min((uint32_t)__popcll(idlemask), lim - nx);
-        if (atomicCAS(next_piece(), nx, nx + want) == nx) {
-          got = want;
-          first = nx;
-        }
-      } else {
-        empty = 1;
-      }
-    }
-    got = __shfl(got, leader);
-    first = __shfl(first, leader);
-    // nothing to claim: a poller wave (one in kPollerEvery) reads the running
-    // count, which decides whether any piece can still come; the others
-    // leave at once, so that the waiting waves' loads of the few control
-    // lines stay rare (every wave polling them slowed the items still
-    // running 2.4 times)
-    if (__shfl(empty, leader)) {
-      const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * BS + threadIdx.x) >> 6);
-      if (wave % gs::kPollerEvery != 0 || running_total() == 0) none = 1;
-    }
-    if (idle) {
-      const uint32_t rank = (uint32_t)__popcll(idlemask & ((1ull << lane) - 1ull));
-      if (rank < got)
-        pending = first + rank;
-      else if (none)
-        finished = true;
-    }
-    poll_wait = got ? 0u : 256u;  // waves with busy lanes poll rarely
-  };
-  // a claimed piece starts once its entry is visible
-  auto take_pending = [&]() __attribute__((always_inline)) {
-    if (pending == kNone || have) return;
-    if (__hip_atomic_load(C->dyn_ready + pending, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != C->epoch) return;
-    __threadfence();
-    const uint32_t id = pending;
-    pending = kNone;
-    start_piece(id);
-  };
-
   while (true) {
-    // lanes without an item take the next one of the main queue
-    const bool need = !have && !finished && !main_done;
-    const uint64_t needmask = __ballot(need);
-    // refills go in groups: the whole wave runs the refill path (code copy,
-    // record clear, first pattern) whenever any lane takes it, so idle lanes
-    // wait until refill_group of them are idle or the wave has no work
-    if (needmask && ((uint32_t)__popcll(needmask) >= P.refill_group || __ballot(have) == 0)) {
-      const int leader = __ffsll((unsigned long long)needmask) - 1;
-      uint32_t base = 0;
-      if (lane == leader) base = atomicAdd(P.queue, (uint32_t)__popcll(needmask));
-      base = __shfl(base, leader);
-      if (need) {
-        const uint64_t it = (uint64_t)base + __popcll(needmask & ((1ull << lane) - 1ull));
-        if (it >= n_items) {
-          main_done = true;
-          if (!P.dyn_cap) finished = true;
+    // lanes without an item take the next one of the queue
+    uint32_t fresh = 0;  // task ends of the item or piece this lane starts now
+    uint32_t fresh_link = kNone;
+    if (!drained) {
+      const bool need = !have;
+      const uint64_t needmask = __ballot(need);
+      // refills go in groups: the whole wave runs the refill path (code copy,
+      // record clear, first pattern) whenever any lane takes it, so idle lanes
+      // wait until refill_group of them are idle or the wave has no work
+      if (needmask && ((uint32_t)__popcll(needmask) >= P.refill_group || needmask == ~0ull)) {
+        uint32_t base, cnt;
+        if (P.take) {  // a small launch: this wave's share of the items, once
+          cnt = P.take;
+          base = __builtin_amdgcn_readfirstlane((blockIdx.x * BS + threadIdx.x) >> 6) * cnt;
+          drained = true;
         } else {
-          start_main(it);
+          cnt = (uint32_t)__popcll(needmask);
+          base = 0;
+          if (lane == 0) base = atomicAdd(P.queue, cnt);
+          base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+          drained = (uint64_t)base + cnt >= n_items;
         }
+        const uint32_t rank = (uint32_t)__popcll(needmask & ((1ull << lane) - 1ull));
+        const uint64_t it = (uint64_t)base + rank;
+        if (need && rank < cnt && it < n_items) fresh = load_main(it);
       }
+    } else if (splitting) {
+      fresh = take_pieces();
+      fresh_link = link;
     }
-    if (P.dyn_cap) {
-      poll_pieces();
-      take_pending();
-    }
+    if (fresh) begin_item((int32_t)(L - t0), fresh, kind == 2 ? fresh_link : kNone);
     const int op = have && !need_next ? (phase == 0 ? 1 : (phase == 1 ? 2 : phase)) : 0;
-    if (__ballot(op != 0 || need_next) == 0) {
-      if (P.dyn_cap) fold_running();
-      if (__ballot(!finished) == 0) break;
-      // the whole wave waits for pieces: back off (about 3 us per sleep, up to 16)
-      for (uint32_t i = 0; i < backoff; ++i) __builtin_amdgcn_s_sleep(127);
-      backoff = backoff < 16 ? 2 * backoff : 16;
-      poll_wait = 0;
+    if (__ballot(have) == 0) {
+      if (drained) break;
       continue;
     }
-    backoff = 1;
-    // One memory operation per lane: a 16-byte load (and for op 2 perhaps a
-    // second one).  The 1-, 4- and 8-byte items (pair byte, suffix-array and
+    // One memory operation per lane that is not stepping backward (phase 1,
+    // below): a 16-byte load, for a pair probe perhaps two.  The 1-, 4- and
+    // 8-byte items (pair byte, suffix-array and
     // inverse words, recorded intervals) come from the aligned 16 bytes that
     // hold them, `sub` saying which part: one load instruction and address
     // for every kind, the same single random access each.
@@ -713,8 +656,6 @@ seed_persistent(PersistArgs P) {
     uint32_t sub = 0, sub2 = 0;
     bool pair_read = false;  // op 1 reads the pair byte instead of a table entry
     bool dual = false;       // and a second one
-    uint32_t i1 = 0, i2 = 0, b1 = 0, b2 = 0;
-    bool have1 = false;
     uint32_t tlen = gs::kPrecalc, tidx = (uint32_t)wcode & 0x3FFFFFFu;  // table lookup: pattern length and entry
     uint32_t pbit = 64;  // presence bit of the clean 3 bases left of an extended window (64: none)
     if (op == 1) {
@@ -746,17 +687,6 @@ seed_persistent(PersistArgs P) {
       }
       n_table += dual ? 2 : 1;
       work += dual ? 2 : 1;
-    } else if (op == 2) {
-      const uint32_t r1 = l - 1u;
-      have1 = r1 != 0xFFFFFFFFu;
-      i2 = u - (u >= primary ? 1u : 0u);
-      b2 = gs::div96(i2);
-      i1 = have1 ? r1 - (r1 >= primary ? 1u : 0u) : 0u;
-      b1 = gs::div96(i1);
-      a1 = P.X.occ + (size_t)b2 * 4 + cx;
-      if (have1 && b1 != b2) a2 = P.X.occ + (size_t)b1 * 4 + cx;
-      n_occ += a2 ? 2 : 1;
-      work += a2 ? 2 : 1;
     } else if (op == 3) {  // the suffix-array word of row l (arrays padded to 16 bytes)
       a1 = reinterpret_cast<const uint4*>(P.X.sa_full) + (l >> 2);
       sub = l & 3u;
@@ -852,9 +782,7 @@ seed_persistent(PersistArgs P) {
       }
     }
 
-    // the new interval: a table entry (op 1) or one backward step (op 2);
-    // both then share one copy of the task logic, so a wave whose lanes are
-    // in different phases runs it once
+    // the new interval: a table entry (op 1 or 6)
     uint32_t nl = 0, nu = 0, nb = 0;
     bool absent = false;  // the clean (tlen + 3)-base window does not occur
     if (op == 1) {
@@ -867,13 +795,6 @@ seed_persistent(PersistArgs P) {
         nu = (tidx & 1u) ? d1.w : d1.y;
       }
       nb = (uint32_t)e - tlen;
-    } else if (op == 2) {
-      const uint32_t o2 = gs::rank_in_entry(d1, i2 - b2 * gs::kBlockBases);
-      const uint32_t o1 = have1 ? gs::rank_in_entry(d2, i1 - b1 * gs::kBlockBases) : 0u;
-      const uint32_t base = pick4(cx, L2_0, L2_1, L2_2, L2_3);
-      nl = base + o1 + 1u;
-      nu = base + o2;
-      nb = (uint32_t)x;
     } else if (op == 6) {  // the entry's interval of length m = d1.z
       nl = d1.x;
       nu = d1.y;
@@ -944,7 +865,7 @@ seed_persistent(PersistArgs P) {
         else
           res = rout == 1 ? 2 : 3;
       }
-    } else if (op != 0) {
+    } else if (op == 1 || op == 6) {
       // a tandem entry whose repeat occurs for fewer than 13 bases ends the
       // task as a 13-mer table miss would
       if (nl > nu || (op == 6 && d1.z < (uint32_t)gs::kPrecalc)) {
@@ -958,7 +879,7 @@ seed_persistent(PersistArgs P) {
         if (op == 1 && tlen > gs::kPrecalc && k < tlen)
           ext_miss = true;
         else
-          res = op == 2 ? 2 : 1;
+          res = 1;
         if (pair_on && op == 1 && pbit < 64) probe = true;  // an absent clean 19-base window
       } else if (absent) {
         res = 1;  // the same holds for an absent clean (tlen + 3)-base window with k >= tlen + 3
@@ -966,7 +887,6 @@ seed_persistent(PersistArgs P) {
       } else {
         // a present clean 19-base window (a jump's window occurs too)
         if (pair_on && ((op == 1 && pbit < 64) || op == 6)) probe = false;
-        if (op == 2) ones = nl == nu ? ones + 1u : 0u;
         l = nl;
         u = nu;
         b = nb;
@@ -980,10 +900,62 @@ seed_persistent(PersistArgs P) {
         }
       }
     }
-    if (prep) {
-      phase = 1;
-      res = prepare_x();
-      if (res == 0) try_direct();
+    // Backward steps (phase 1), in a loop of their own: one or two occ entries
+    // of one 64-byte block group, the new interval, its size record and the
+    // next base.  It goes round again while at least half of the lanes with
+    // an item still step (the others wait), unless the wave's idle lanes
+    // could take work: a round costs about a quarter of the instructions of
+    // the whole body, and in the tail of a launch, where few lanes have
+    // items and most of them step, the body's instructions decide.  Kernel
+    // time against one step per turn of the body: 1,000,000 150 bp reads on
+    // the 3.1 Gbp index 8.2 -> 7.4 ms, 60,000 uneven reads 7.8 -> 7.0 ms,
+    // 10,000,000 reads 58.7 -> 57.6 ms (going on down to a quarter of the
+    // lanes: 7.7, 6.8 and 58.8; down to three quarters: 7.5, 6.9 and 58.0).
+    for (uint32_t round = 0;; ++round) {
+      if (prep) {
+        prep = false;
+        phase = 1;
+        res = prepare_x();
+        if (res == 0) try_direct();
+      }
+      const bool step = have && !need_next && res == 0 && phase == 1;
+      const uint64_t stepping = __ballot(step);
+      if (!stepping) break;
+      if (round) {
+        if (2 * __popcll(stepping) < __popcll(__ballot(have))) break;
+        if (drained && splitting && can_give()) break;
+      }
+      if (step) {
+        const uint32_t r1 = l - 1u;
+        const bool have1 = r1 != 0xFFFFFFFFu;
+        const uint32_t i2 = u - (u >= primary ? 1u : 0u);
+        const uint32_t b2 = gs::div96(i2);
+        const uint32_t i1 = have1 ? r1 - (r1 >= primary ? 1u : 0u) : 0u;
+        const uint32_t b1 = gs::div96(i1);
+        const bool two = have1 && b1 != b2;
+        const uint4 d2 = P.X.occ[(size_t)b2 * 4 + cx];
+        uint4 d1 = d2;
+        if (two) d1 = P.X.occ[(size_t)b1 * 4 + cx];
+        n_occ += two ? 2 : 1;
+        work += two ? 2 : 1;
+        const uint32_t base = pick4(cx, L2_0, L2_1, L2_2, L2_3);
+        const uint32_t nl = base + (have1 ? gs::rank_in_entry(d1, i1 - b1 * gs::kBlockBases) : 0u) + 1u;
+        const uint32_t nu = base + gs::rank_in_entry(d2, i2 - b2 * gs::kBlockBases);
+        if (nl > nu) {
+          res = 2;
+        } else {
+          ones = nl == nu ? ones + 1u : 0u;
+          l = nl;
+          u = nu;
+          b = (uint32_t)x;
+          if (prune_at((int32_t)b, u - l + 1u)) {
+            res = 1;
+          } else {
+            x = (int32_t)b - 1;
+            prep = true;
+          }
+        }
+      }
     }
     if (res >= 2) finish_task();
     if (res == 3 && P.smem)
@@ -994,7 +966,6 @@ seed_persistent(PersistArgs P) {
       need_next = false;
       next_task();
     }
-    if (P.dyn_cap) fold_running();
   }
   if (C->counters) {
     // wave totals, one atomic per wave
@@ -1152,11 +1123,6 @@ __global__ void __launch_bounds__(256) pack_codes_long(const uint8_t* __restrict
   }
 }
 
-__global__ void zero_words(uint32_t* __restrict__ p, uint32_t n) {
-  const uint32_t i = blockIdx.x * 64 + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
 template <typename AT, int LMAX, int BS>
 int grid_t(unsigned* grid) {
   int dev = 0, per_cu = 0;
@@ -1170,8 +1136,13 @@ int grid_t(unsigned* grid) {
   return GS_OK;
 }
 
-// one thread: the launch's cold fields into their device slot
-__global__ void write_cold(gs::PersistCold c, gs::PersistCold* dst) { *dst = c; }
+// one wave, before every launch: the cold fields into their device slot, the
+// queue, the pieces reserved and the counters cleared
+__global__ void __launch_bounds__(64) set_up_launch(gs::PersistCold c, gs::PersistCold* dst, uint32_t* queue) {
+  if (threadIdx.x == 0) *dst = c;
+  if (threadIdx.x < 2) queue[threadIdx.x] = 0;  // the next item, the pieces reserved
+  if (threadIdx.x < gs::kCounterBytes / 4) reinterpret_cast<uint32_t*>(c.counters)[threadIdx.x] = 0;
+}
 
 template <typename AT, int LMAX, int BS>
 int launch_t(const gs::PersistParams& P, unsigned grid, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
@@ -1189,14 +1160,12 @@ int launch_t(const gs::PersistParams& P, unsigned grid, hipStream_t st, hipEvent
   c.dyn_items = P.dyn_items;
   c.dyn_meta = P.dyn_meta;
   c.dyn_link = P.dyn_link;
-  c.dyn_ready = P.dyn_ready;
-  c.dyn_ctl = P.dyn_ctl;
+  c.reserved = P.queue + 1;
   c.wmeta = P.wmeta;
   c.wlink = P.wlink;
   c.seg_tasks = P.seg_tasks;
-  c.epoch = P.epoch;
   gs::PersistCold* dst = reinterpret_cast<gs::PersistCold*>(reinterpret_cast<uint8_t*>(P.counters) + gs::kCounterBytes);
-  hipLaunchKernelGGL(write_cold, dim3(1), dim3(1), 0, st, c, dst);
+  hipLaunchKernelGGL(set_up_launch, dim3(1), dim3(64), 0, st, c, dst, P.queue);
   PersistArgs A;
   A.X = P.X;
   A.codes = P.codes;
@@ -1209,8 +1178,24 @@ int launch_t(const gs::PersistParams& P, unsigned grid, hipStream_t st, hipEvent
   A.dyn_cap = P.dyn_cap;
   A.split_work = P.split_work;
   A.split_tasks = P.split_tasks;
-  A.split_below = grid * (uint32_t)BS / 2;  // half the lanes of the launch
   A.refill_group = gs::kRefillGroup;
+  A.split_idle = gs::kSplitIdle;
+  A.take = 0;
+  constexpr uint32_t kWaves = BS / 64;  // per workgroup
+  if (P.n_items <= (uint64_t)grid * BS) {
+    // fewer items than lanes: each wave takes its share at once, one item per
+    // wave if there are fewer items than waves, and only as many workgroups
+    // start as have items
+    const uint32_t waves = grid * kWaves;
+    A.take = (uint32_t)((P.n_items + waves - 1) / waves);
+    if (!A.take) A.take = 1;
+    const uint32_t used = (uint32_t)((P.n_items + A.take - 1) / A.take);
+    grid = (used + kWaves - 1) / kWaves;
+    if (!grid) grid = 1;
+    A.split_idle = 1;
+  } else if (!A.split_work) {
+    A.split_work = gs::kSplitWork;
+  }
   A.tandem = P.tandem;
   if (e0 && hipEventRecord(e0, st) != hipSuccess) return GS_EHIP;
   hipLaunchKernelGGL((seed_persistent<AT, LMAX, BS>), dim3(grid), dim3(BS), 0, st, A);
@@ -1267,13 +1252,7 @@ int persistent_grid(int variant, int wg, unsigned* grid) {
 int launch_persistent(const PersistParams& P, int variant, int wg, unsigned grid, hipStream_t st, hipEvent_t e0,
                       hipEvent_t e1) {
   if (!grid) return GS_EINVAL;
-  hipLaunchKernelGGL(zero_words, dim3(1), dim3(64), 0, st, P.queue, 1u);
-  if (P.dyn_cap) {  // an empty overflow queue: no piece reserved, claimed or written
-    hipLaunchKernelGGL(zero_words, dim3((gs::kDynCtlWords + 63) / 64), dim3(64), 0, st, P.dyn_ctl, gs::kDynCtlWords);
-    hipLaunchKernelGGL(zero_words, dim3((P.dyn_cap + 63) / 64), dim3(64), 0, st, P.dyn_ready, P.dyn_cap);
-  }
   if (!P.counters) return GS_EINVAL;  // its buffer also holds the launch's PersistCold
-  hipLaunchKernelGGL(zero_words, dim3(1), dim3(64), 0, st, (uint32_t*)P.counters, 8u);
   constexpr int L = kPersistLmax;
   switch (variant * 1000 + (wg ? wg : 128)) {
     case 64: return launch_t<uint8_t, L, 64>(P, grid, st, e0, e1);

@@ -793,7 +793,7 @@ struct gs_batch {
   DevBuf bases, offs, lens, toff, batch, cand, nF, nR, ns, np, soff, poff, tiles, tot, seeds, rows, scratch;
   DevBuf codes, code_off, queue, counters;  // persistent kernel
   DevBuf items, seg_meta, long_reads, item0, item_tmp;  // item_tmp: counts and scans of the item plan
-  DevBuf seg_link, dyn_items, dyn_meta, dyn_link, dyn_ready, dyn_ctl, wmeta, wlink;  // work splitting
+  DevBuf seg_link, dyn_items, dyn_meta, dyn_link, wmeta, wlink;  // work splitting
   uint64_t code_chunks = 0, n_items = 0;
   uint32_t n_long = 0, seg_tasks = 64, dyn_cap = 0;
   uint64_t n_seeds = 0, n_pos = 0;
@@ -997,8 +997,7 @@ static int ensure_buffers(gs_batch* B, uint64_t span, uint64_t n, uint64_t tasks
       B->seg_link.ensure(n_long ? 4 * n_items : 16) ||
       (dyn_cap &&
        (B->dyn_items.ensure(16ull * dyn_cap) || B->dyn_meta.ensure(16ull * dyn_cap) ||
-        B->dyn_link.ensure(4ull * dyn_cap) || B->dyn_ready.ensure(4ull * dyn_cap) ||
-        B->dyn_ctl.ensure(4ull * gs::kDynCtlWords) || B->wmeta.ensure(32 * nr1) || B->wlink.ensure(8 * nr1))))
+        B->dyn_link.ensure(4ull * dyn_cap) || B->wmeta.ensure(32 * nr1) || B->wlink.ensure(8 * nr1))))
     return GS_ENOMEM;
   return GS_OK;
 }
@@ -1010,7 +1009,7 @@ int gs::batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_
   // every read and long-read segment is an item of each strand; a read has
   // at most as many tasks as bases and code chunks as 32-base spans (+1)
   const uint64_t items = 2 * (reads + bases / seg_tasks + 1);
-  const uint32_t dyn = (uint32_t)std::min<uint64_t>(16u << 20, std::max<uint64_t>(65536, items));
+  const uint32_t dyn = gs::piece_cap(items);
   int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, 0xFFFFFFFFu, dyn);
   if (!rc && bases > (4u << 20)) {  // the pinned chunks of staged uploads
     const size_t ch = std::min<uint64_t>(bases, kStageChunk);
@@ -1108,20 +1107,8 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P) {
   B->n_seeds = B->n_pos = 0;
   B->ran = false;
   const uint64_t n = P.n_reads, nr1 = n + 1;
-  // Work splitting pays where the tail of a launch is a large share of it:
-  // batches of at most kSplitItemsPerLane work items per lane of the
-  // persistent grid (in larger batches the tail is amortised and keeping
-  // the overflow queue live costs more than it saves).  An explicit
-  // split_tasks turns it on whatever the batch size.
-  bool split_on = P.opts.split_tasks != 0xFFFF && P.opts.kernel != 0;
-  if (split_on && P.opts.split_tasks == 0) {
-    unsigned grid = 0;
-    const int wg = P.opts.wg ? P.opts.wg : 128;
-    if (gs::persistent_grid(P.opts.kernel >= 1 ? P.opts.kernel - 1 : 0, wg, &grid) != GS_OK || !grid ||
-        B->n_items > (uint64_t)gs::kSplitItemsPerLane * grid * (uint64_t)wg)
-      split_on = false;
-  }
-  B->dyn_cap = split_on ? (uint32_t)std::min<uint64_t>(16u << 20, std::max<uint64_t>(65536, B->n_items)) : 0u;
+  const bool split_on = P.opts.split_tasks != 0xFFFF && P.opts.kernel != 0;
+  B->dyn_cap = split_on ? gs::piece_cap(B->n_items) : 0u;
   if (ensure_buffers(B, B->span, n, B->tasks, B->code_chunks, B->n_items, B->n_long, B->maxlen, B->dyn_cap))
     return GS_ENOMEM;
   hipStream_t st = B->stream;
@@ -1271,14 +1258,11 @@ static int enqueue_extension(gs_batch* B, const SeedParams& S, int kernel, unsig
   PP.dyn_items = B->dyn_items.as<uint4>();
   PP.dyn_meta = B->dyn_meta.as<uint4>();
   PP.dyn_link = B->dyn_link.as<uint32_t>();
-  PP.dyn_ready = B->dyn_ready.as<uint32_t>();
-  PP.dyn_ctl = B->dyn_ctl.as<uint32_t>();
   PP.wmeta = B->wmeta.as<uint4>();
   PP.wlink = B->wlink.as<uint32_t>();
   PP.dyn_cap = B->dyn_cap;
-  PP.split_tasks = B->opts.split_tasks ? B->opts.split_tasks : 8u;
-  PP.split_work = 64u * (B->opts.split_work ? B->opts.split_work : 32u);
-  PP.epoch = 1;  // dyn_ready is cleared by launch_persistent before every launch
+  PP.split_tasks = B->opts.split_tasks ? B->opts.split_tasks : gs::kSplitTasks;
+  PP.split_work = 64u * B->opts.split_work;  // 0: by the launch's size
   // tandem jumps read the index's tandem table
   const bool tandem = B->opts.tandem != 0xFFFF && B->X->tandem;
   PP.tandem = tandem ? (B->opts.tandem ? std::min<uint32_t>(B->opts.tandem, gs::kTandemMax) : gs::kTandemMax) : 0u;
@@ -1908,6 +1892,12 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
                  o_long = long_scratch ? take(4 * (span + 16)) : 0;
   if (at > kNoAllocBytes) return GS_ERANGE;
   const uint64_t fixed = at;
+  // the pieces of work splitting, where they fit: they are dead once the
+  // streams are joined, and the outputs, written after that, take their place
+  const uint32_t cap = kernel && opts->split_tasks != 0xFFFF ? gs::piece_cap(2ull * n) : 0u;
+  const uint64_t o_ditems = take(16ull * cap), o_dmeta = take(16ull * cap), o_dlink = take(4ull * cap),
+                 o_wmeta = take(32 * nr1), o_wlink = take(8 * nr1);
+  const bool split_on = cap && at <= kNoAllocBytes;
 
   if (X->device < 0 || X->device >= kNoAllocDevices) return GS_EINVAL;
   if (hipSetDevice(X->device) != hipSuccess) return GS_EHIP;
@@ -1933,7 +1923,14 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   B.n_items = kernel ? 2ull * n : 0;
   B.n_long = 0;
   B.seg_tasks = opts->seg_tasks ? opts->seg_tasks : 64u;
-  B.dyn_cap = 0;
+  B.dyn_cap = split_on ? cap : 0u;
+  if (split_on) {
+    B.dyn_items.view(base + o_ditems, 16ull * cap);
+    B.dyn_meta.view(base + o_dmeta, 16ull * cap);
+    B.dyn_link.view(base + o_dlink, 4ull * cap);
+    B.wmeta.view(base + o_wmeta, 32 * nr1);
+    B.wlink.view(base + o_wlink, 8 * nr1);
+  }
   uint64_t h_tot[2] = {0, 0};
   B.h_tot = h_tot;
   B.bases.view(base + o_bases, span + 32);

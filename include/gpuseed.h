@@ -278,13 +278,13 @@ typedef struct {
                        (0 = 64)                                               */
   uint16_t wg;        /* batched kernels: workgroup size 64, 128 or 256 (0 = 128) */
   uint16_t walk_rows; /* suffix-array walk: rows per thread 1, 2 or 4 (0 = 1) */
-  uint16_t split_tasks; /* batched kernels: in the tail of a launch an item
-                       that has used split_work memory operations hands half
-                       of its task ends to an idle lane while at least
-                       2 * split_tasks remain, 1..64; 0 = 8, and only in
-                       batches of at most 4 work items per lane of the
-                       persistent grid; 0xFFFF: no splitting                 */
-  uint16_t split_work;  /* in units of 64 memory operations, 1..0xFFFE (0 = 32) */
+  uint16_t split_tasks; /* batched kernels: once a launch's work queue is
+                       exhausted, an item that has used split_work memory
+                       operations hands half of its task ends to an idle
+                       lane of its wave while at least 2 * split_tasks
+                       remain, 1..64 (0 = 4); 0xFFFF: no splitting           */
+  uint16_t split_work;  /* in units of 64 memory operations, 1..0xFFFE (0 = 1,
+                       and none in a launch of fewer items than lanes)       */
   uint16_t direct_min;  /* batched kernels on an index with gs_index_set_direct:
                        a task reads the text once its interval has kept one
                        row for this many backward steps, 1..64 (0 = 4);

@@ -83,6 +83,8 @@ namespace gs {
 // kernel reads them with scalar loads where it uses them, so that its
 // arguments fit the scalar registers instead of spilling into vector ones.
 struct PersistCold {
+  const uint8_t* bases;    // the batch's bytes and the reads' offsets in them (plain kernel)
+  const uint64_t* offs;
   const uint64_t* code_off;
   const uint32_t* lens;
   const uint64_t* task_off;
@@ -107,6 +109,8 @@ static_assert(sizeof(PersistCold) <= kColdBytes, "PersistCold must fit its slot"
 
 struct PersistParams {
   DevIndex X;
+  const uint8_t* bases;      // plain kernel: the batch's bytes and offsets (32 bytes kept after the last read)
+  const uint64_t* offs;
   const uint4* codes;        // 4-bit virtual codes, per read: forward chunks then reverse chunks
   const uint64_t* code_off;  // per read, in 16-byte chunks
   const uint32_t* lens;
@@ -158,10 +162,16 @@ constexpr uint32_t kSplitStream = 0xFFFFFFFFu;  // nF/nR of a whole-read stream 
 // Work splitting (take_pieces): a lane gives half of its task ends away after
 // kSplitWork memory operations (at once in a launch of fewer items than
 // lanes), while it has at least 2 * kSplitTasks of them left, and once
-// kSplitIdle lanes of its wave are idle (any idle lane, in a small launch).
+// kSplitIdle lanes of its wave are idle (kSplitIdleSmall in such a launch).
+// Measured, kernel ms: idle lanes 8, 16, 24, 32 in small launches: 10,000
+// 150 bp reads on a 100 Mbp index 0.74, 0.80, 0.74, 0.71, 60,000 on the
+// 3.1 Gbp index 1.62, 1.61, 1.68, 1.83; task ends 2, 4, 8: 1.42, 1.68, 2.07
+// and 1000 reads there 0.58, 0.85, 0.86.  In a launch of 1,000,000 reads all
+// of 16-32 idle lanes, 16-64 operations and 1-4 task ends gave 7.2-7.5.
 constexpr uint32_t kSplitWork = 64;
-constexpr uint32_t kSplitTasks = 4;
+constexpr uint32_t kSplitTasks = 2;
 constexpr uint32_t kSplitIdle = 32;
+constexpr uint32_t kSplitIdleSmall = 24;
 // Pieces a launch can split off (36 bytes each): 8 per item, at least 65,536,
 // at most 2^20; beyond that items go on whole.
 __host__ inline uint32_t piece_cap(uint64_t n_items) {
@@ -205,8 +215,8 @@ __host__ __device__ inline uint32_t n_segments(uint32_t L, uint32_t k, uint32_t 
 
 int launch_pack_codes(const uint8_t* bases, const uint64_t* offs, const uint32_t* lens, const uint64_t* code_off,
                       uint32_t n_reads, const uint32_t* long_reads, uint32_t n_long, uint4* codes, hipStream_t st);
-// variant 0: 8-bit size records, 1: 16-bit size records; wg 64, 128 or 256
-// (0 = 128); grid from persistent_grid (called outside any graph capture)
+// variant -1: the plain kernel (wg ignored), 0: 8-bit size records, 1: 16-bit
+// and 2: 4-bit size records; wg 64, 128 or 256 (0 = 128); grid from persistent_grid (called outside any graph capture)
 int persistent_grid(int variant, int wg, unsigned* grid);
 // e0, e1 (optional): recorded on st right before and after seed_persistent
 int launch_persistent(const PersistParams& P, int variant, int wg, unsigned grid, hipStream_t st,
@@ -223,7 +233,7 @@ namespace gs {
 // device when the batch is loaded.
 struct BatchPlan {
   gs_opts opts{};
-  uint32_t seg_tasks = 64, maxlen = 0, next_batch_id = 0;
+  uint32_t seg_tasks = 64, next_batch_id = 0;
   uint64_t n_reads = 0, span = 0, tasks = 0, code_chunks = 0, n_items = 0, n_long = 0;
   std::vector<std::pair<const char*, uint64_t>> pieces;  // bytes uploaded back to back
   std::vector<uint64_t> offs, task_off, code_off;

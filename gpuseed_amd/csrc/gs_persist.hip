@@ -121,7 +121,11 @@ struct PersistArgs {
 template <typename AT>
 constexpr int kMinWaves = std::is_same<AT, Nib>::value ? 4 : 1;
 
-template <typename AT, int LMAX, int BS>
+// PLAIN is the plain kernel (gs_opts.kernel 0): one work item per lane in a
+// launch of as many lanes as items, no queue, and neither pair probes nor
+// direct runs nor tandem jumps.  It reads the batch's bytes instead of packed
+// codes, which its lanes convert as they fill their slots (once per lane).
+template <typename AT, int LMAX, int BS, bool PLAIN>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kMinWaves<AT>)))
 seed_persistent(PersistArgs P) {
   static_assert(LMAX % 32 == 0, "LMAX must be a multiple of 32");
@@ -189,7 +193,7 @@ seed_persistent(PersistArgs P) {
   // was absent; the last probe also answered the windows of the task ends
   // known_e, known_e - 1, ... (their number in bits 4-5 of known_m; bit i
   // set iff the window of known_e - i occurs)
-  const bool pair_on = P.X.pair && P.X.ext_len == 16 && k >= 19;
+  const bool pair_on = !PLAIN && P.X.pair && P.X.ext_len == 16 && k >= 19;
   bool probe = false;
   int32_t known_e = -1;
   uint32_t known_m = 0;
@@ -221,7 +225,7 @@ seed_persistent(PersistArgs P) {
   // size records only prune.  tp 0: no stretch.
   uint32_t tp = 0;
   int32_t tR = 0;
-  const bool tandem_on = P.tandem != 0;
+  const bool tandem_on = !PLAIN && P.tandem != 0;
 
   // code of position i of the stream: the LDS window holds [w0, w0 + LMAX);
   // an extension may run left of it and then reads the 4-bit codes in
@@ -234,6 +238,10 @@ seed_persistent(PersistArgs P) {
       const uint32_t* cw = reinterpret_cast<const uint32_t*>(lds + sbase + A_BYTES);
       if ((cw[CW + (rr >> 5)] >> (rr & 31u)) & 1u) return 4u;
       return (cw[rr >> 4] >> ((rr & 15u) << 1)) & 3u;
+    }
+    if constexpr (PLAIN) {
+      const uint8_t* bytes = C->bases + C->offs[r];
+      return strand ? gs::code_rev(bytes[L - 1 - (uint32_t)i]) : gs::code_fwd(bytes[i]);
     }
     const uint32_t w = reinterpret_cast<const uint32_t*>(P.codes + gcodes + (uint32_t)(i >> 5))[(i >> 3) & 3];
     return (w >> ((i & 7) << 2)) & 15u;
@@ -436,7 +444,7 @@ seed_persistent(PersistArgs P) {
   // suffix array (phase 5) when it is needed: for a candidate that is
   // emitted, or to go on with backward steps past an N.
   auto try_direct = [&]() __attribute__((always_inline)) {
-    if (P.direct_min && l == u && ones >= P.direct_min) {
+    if (!PLAIN && P.direct_min && l == u && ones >= P.direct_min) {
       const int32_t j = x - w0;  // runs stay inside the LDS window
       if (j >= 0 && rec_get(sbase, j) != 1u) phase = 3;
     }
@@ -481,9 +489,8 @@ seed_persistent(PersistArgs P) {
   auto load_slot = [&](uint32_t code0) __attribute__((always_inline)) {
     const uint32_t nch = (L + 31) >> 5;
     gcodes = code0 + strand * nch;
-    const uint4* src = P.codes + gcodes;
     uint32_t top;
-    const bool whole = L <= (uint32_t)LMAX;  // pack_codes wrote its chunks in the slot's form
+    const bool whole = L <= (uint32_t)LMAX;
     if (whole) {  // the whole stream fits the window
       top = nch << 5;
       w0 = 0;
@@ -496,21 +503,27 @@ seed_persistent(PersistArgs P) {
     // q = LMAX/32 - 1 - (c - c0)
     const uint32_t c0 = (uint32_t)w0 >> 5, c1 = top >> 5;
     uint32_t* cw = reinterpret_cast<uint32_t*>(lds + sbase + A_BYTES);
-    // all of the window's chunks are loaded before the first is used: one
-    // memory latency per item (a wave refills about every seven iterations)
-    uint4 v[LMAX / 32];
+    auto put = [&](uint32_t i, uint4 v) __attribute__((always_inline)) {
+      const uint32_t q = (uint32_t)(LMAX / 32 - 1) - i;
+      cw[2 * q] = v.x;
+      cw[2 * q + 1] = v.y;
+      cw[CW + q] = v.z;
+    };
+    if constexpr (PLAIN) {
+      const uint8_t* bytes = C->bases + C->offs[r];
+#pragma unroll 1
+      for (uint32_t c = c0; c < c1; ++c) put(c - c0, slot_chunk(gs::pack_chunk(bytes, L, strand, c)));
+    } else {
+      // all of the window's chunks are loaded before the first is used: one
+      // memory latency per item (a wave refills about every seven iterations)
+      const uint4* src = P.codes + gcodes;
+      uint4 v[LMAX / 32];
 #pragma unroll
-    for (uint32_t i = 0; i < (uint32_t)(LMAX / 32); ++i)
-      if (c0 + i < c1) v[i] = src[c0 + i];
+      for (uint32_t i = 0; i < (uint32_t)(LMAX / 32); ++i)
+        if (c0 + i < c1) v[i] = src[c0 + i];
 #pragma unroll
-    for (uint32_t i = 0; i < (uint32_t)(LMAX / 32); ++i) {
-      if (c0 + i < c1) {
-        if (!whole) v[i] = slot_chunk(v[i]);
-        const uint32_t q = (uint32_t)(LMAX / 32 - 1) - i;
-        cw[2 * q] = v[i].x;
-        cw[2 * q + 1] = v[i].y;
-        cw[CW + q] = v[i].z;
-      }
+      for (uint32_t i = 0; i < (uint32_t)(LMAX / 32); ++i)
+        if (c0 + i < c1) put(i, whole ? v[i] : slot_chunk(v[i]));  // pack_codes wrote whole reads in the slot's form
     }
     cw[CW - 2] = 0;
     cw[CW - 1] = 0;
@@ -527,7 +540,7 @@ seed_persistent(PersistArgs P) {
     strand = (uint32_t)(v >> 32) & 1u;
     const uint32_t seg = (uint32_t)(v >> 33);
     L = C->lens[r];
-    const uint32_t code0 = (uint32_t)C->code_off[r];
+    const uint32_t code0 = PLAIN ? 0u : (uint32_t)C->code_off[r];
     out = C->cand + 2 * C->task_off[r];
     if (L < k) {
       (strand ? C->nR : C->nF)[r] = 0;
@@ -687,20 +700,20 @@ seed_persistent(PersistArgs P) {
       }
       n_table += dual ? 2 : 1;
       work += dual ? 2 : 1;
-    } else if (op == 3) {  // the suffix-array word of row l (arrays padded to 16 bytes)
+    } else if (!PLAIN && op == 3) {  // the suffix-array word of row l (arrays padded to 16 bytes)
       a1 = reinterpret_cast<const uint4*>(P.X.sa_full) + (l >> 2);
       sub = l & 3u;
-    } else if (op == 4) {
+    } else if (!PLAIN && op == 4) {
       a1 = P.X.text + ((tq - 1u) >> 6);  // tq >= 1 whenever phase 4 is entered
-    } else if (op == 5) {  // the inverse word of text position tq
+    } else if (!PLAIN && op == 5) {  // the inverse word of text position tq
       a1 = reinterpret_cast<const uint4*>(P.X.isa) + (tq >> 2);
       sub = tq & 3u;
-    } else if (op == 6) {  // tandem-table entry tq
+    } else if (!PLAIN && op == 6) {  // tandem-table entry tq
       a1 = P.X.tandem + tq;
       ++n_tandem;
       ++work;
     }
-    if (op >= 3 && op <= 5) {
+    if (!PLAIN && op >= 3 && op <= 5) {
       ++n_direct;
       ++work;
     }
@@ -721,7 +734,7 @@ seed_persistent(PersistArgs P) {
     // few wave instructions instead of a loop over 64 positions in one lane.
     uint32_t run_g = 0;  // positions matched (and recorded) by this lane's comparison
     int run_kind = 0;    // 0: all matched; 1: a mismatch, 3: an N at position x - run_g; 4: pruned there
-    {
+    if constexpr (!PLAIN) {
       uint64_t runners = __ballot(op == 4);
       while (runners) {
         const int R = __ffsll((unsigned long long)runners) - 1;
@@ -825,7 +838,7 @@ seed_persistent(PersistArgs P) {
         res = 1;
       else
         probe = false;
-    } else if (op >= 3 && op <= 5) {
+    } else if (!PLAIN && op >= 3 && op <= 5) {
       if (op == 3) {  // the text position of read[b]
         tq = v4;
         if (tq == 0)
@@ -1123,16 +1136,25 @@ __global__ void __launch_bounds__(256) pack_codes_long(const uint8_t* __restrict
   }
 }
 
-template <typename AT, int LMAX, int BS>
+// compute units of the current device (0: the query failed)
+unsigned compute_units() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1)
+    return 0;
+  return (unsigned)n;
+}
+
+template <typename AT, int LMAX, int BS, bool PLAIN = false>
 int grid_t(unsigned* grid) {
-  int dev = 0, per_cu = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return GS_EHIP;
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return GS_EHIP;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, seed_persistent<AT, LMAX, BS>, BS, 0) != hipSuccess ||
+  const unsigned cus = compute_units();
+  int per_cu = 0;
+  if (!cus ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, seed_persistent<AT, LMAX, BS, PLAIN>, BS, 0) !=
+          hipSuccess ||
       per_cu < 1)
     return GS_EHIP;
-  *grid = (unsigned)(per_cu * prop.multiProcessorCount);
+  *grid = (unsigned)per_cu * cus;
   return GS_OK;
 }
 
@@ -1144,9 +1166,11 @@ __global__ void __launch_bounds__(64) set_up_launch(gs::PersistCold c, gs::Persi
   if (threadIdx.x < gs::kCounterBytes / 4) reinterpret_cast<uint32_t*>(c.counters)[threadIdx.x] = 0;
 }
 
-template <typename AT, int LMAX, int BS>
+template <typename AT, int LMAX, int BS, bool PLAIN = false>
 int launch_t(const gs::PersistParams& P, unsigned grid, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
   gs::PersistCold c;
+  c.bases = P.bases;
+  c.offs = P.offs;
   c.code_off = P.code_off;
   c.lens = P.lens;
   c.task_off = P.task_off;
@@ -1180,25 +1204,34 @@ int launch_t(const gs::PersistParams& P, unsigned grid, hipStream_t st, hipEvent
   A.split_tasks = P.split_tasks;
   A.refill_group = gs::kRefillGroup;
   A.split_idle = gs::kSplitIdle;
+  A.tandem = P.tandem;
   A.take = 0;
   constexpr uint32_t kWaves = BS / 64;  // per workgroup
   if (P.n_items <= (uint64_t)grid * BS) {
-    // fewer items than lanes: each wave takes its share at once, one item per
-    // wave if there are fewer items than waves, and only as many workgroups
-    // start as have items
-    const uint32_t waves = grid * kWaves;
-    A.take = (uint32_t)((P.n_items + waves - 1) / waves);
-    if (!A.take) A.take = 1;
+    // Fewer items than lanes: each wave takes its share at once, and only as
+    // many waves start as they need.  One wave per SIMD comes first, one item
+    // each if there are no more, then up to 64 items per wave, then more
+    // waves: the kernel is bound by the instructions that its waves issue, so
+    // that a second wave on a SIMD costs more than lanes that share one.
+    // Kernel time with as many waves as fit against this: 10,000 100 bp reads
+    // on a 1 Mbp index 1.05 -> 0.44 ms, 50,000 and 100,000 150 bp reads on a
+    // 100 Mbp index 2.75 -> 1.31 and (plain kernel) 4.62 -> 2.05 ms, 60,000
+    // on the 3.1 Gbp index 2.72 -> 1.42 ms.
+    const uint64_t simds = std::max(1u, 4 * compute_units());
+    A.take = (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, (P.n_items + simds - 1) / simds));
     const uint32_t used = (uint32_t)((P.n_items + A.take - 1) / A.take);
     grid = (used + kWaves - 1) / kWaves;
     if (!grid) grid = 1;
-    A.split_idle = 1;
-  } else if (!A.split_work) {
-    A.split_work = gs::kSplitWork;
+    A.split_idle = gs::kSplitIdleSmall;
+  } else {
+    if (!A.split_work) A.split_work = gs::kSplitWork;
+    if (PLAIN) {  // one item per lane
+      A.take = 64;
+      grid = (unsigned)((P.n_items + BS - 1) / BS);
+    }
   }
-  A.tandem = P.tandem;
   if (e0 && hipEventRecord(e0, st) != hipSuccess) return GS_EHIP;
-  hipLaunchKernelGGL((seed_persistent<AT, LMAX, BS>), dim3(grid), dim3(BS), 0, st, A);
+  hipLaunchKernelGGL((seed_persistent<AT, LMAX, BS, PLAIN>), dim3(grid), dim3(BS), 0, st, A);
   if (hipGetLastError() != hipSuccess) return GS_EHIP;
   return e1 && hipEventRecord(e1, st) != hipSuccess ? GS_EHIP : GS_OK;
 }
@@ -1235,6 +1268,7 @@ int launch_join(const JoinParams& J, hipStream_t st) {
 // Workgroups that fill every CU at the kernel's occupancy (LDS slots bound it).
 int persistent_grid(int variant, int wg, unsigned* grid) {
   constexpr int L = kPersistLmax;
+  if (variant < 0) return grid_t<Nib, L, 128, true>(grid);
   switch (variant * 1000 + (wg ? wg : 128)) {
     case 64: return grid_t<uint8_t, L, 64>(grid);
     case 128: return grid_t<uint8_t, L, 128>(grid);
@@ -1254,6 +1288,7 @@ int launch_persistent(const PersistParams& P, int variant, int wg, unsigned grid
   if (!grid) return GS_EINVAL;
   if (!P.counters) return GS_EINVAL;  // its buffer also holds the launch's PersistCold
   constexpr int L = kPersistLmax;
+  if (variant < 0) return launch_t<Nib, L, 128, true>(P, grid, st, e0, e1);
   switch (variant * 1000 + (wg ? wg : 128)) {
     case 64: return launch_t<uint8_t, L, 64>(P, grid, st, e0, e1);
     case 128: return launch_t<uint8_t, L, 128>(P, grid, st, e0, e1);

@@ -690,7 +690,7 @@ __global__ void zero_bytes(uint8_t* __restrict__ p, uint32_t n) {
 // segment at most seg_tasks, so the last items a persistent kernel hands
 // out are the small ones.
 
-__device__ __forceinline__ bool read_is_long(uint32_t L, uint32_t k, uint32_t nseg) {
+__host__ __device__ __forceinline__ bool read_is_long(uint32_t L, uint32_t k, uint32_t nseg) {
   return nseg > 1 || (L > gs::kPersistLmax && L >= k);
 }
 
@@ -789,6 +789,9 @@ struct gs_batch {
   hipStream_t stream = nullptr;  // a batch's own stream: batches of one index may run concurrently
   gs_opts opts;
   uint64_t n_reads = 0, span = 0, tasks = 0;
+  // gs_seed_noalloc, where the work items do not fit its array: seed_streams
+  // instead of the persistent kernel (which needs maxlen and the read scratch)
+  bool streams = false;
   uint32_t maxlen = 0;
   DevBuf bases, offs, lens, toff, batch, cand, nF, nR, ns, np, soff, poff, tiles, tot, seeds, rows, scratch;
   DevBuf codes, code_off, queue, counters;  // persistent kernel
@@ -938,7 +941,6 @@ int gs::plan_add(BatchPlan& P, const char* bases, const uint64_t* offsets, const
       ++bid;
       acc = 0;
     }
-    if (L > P.maxlen) P.maxlen = L;
     ++P.n_reads;
     P.code_off.push_back(P.code_chunks);
     P.code_chunks += 2 * ((L + 31) / 32);
@@ -963,8 +965,7 @@ void gs::plan_finish(BatchPlan& P) {
 uint64_t gs::plan_device_bytes(const BatchPlan& P) {
   const uint64_t nr1 = P.n_reads + 1;
   return (P.span + 32) + 16 * (P.code_chunks + 1) + 16 * (2 * P.tasks + 1) + 8 * P.n_items +
-         (P.n_long ? 16 * P.n_items : 0) + 12 * P.n_long + nr1 * (8 * 5 + 4 * 7 + 36) +
-         (P.maxlen > 256 ? 4 * (P.span + 16) : 0);
+         (P.n_long ? 16 * P.n_items : 0) + 12 * P.n_long + nr1 * (8 * 5 + 4 * 7 + 36);
 }
 
 static int batch_events(gs_batch* B) {
@@ -979,10 +980,9 @@ static int batch_events(gs_batch* B) {
 
 // Device buffers of a batch of `span` bases, n reads, `tasks` task slots per
 // strand, `code_chunks` 16-byte code chunks, n_items work items (n_long of
-// them long reads), reads of at most maxlen bases and an overflow queue of
-// dyn_cap pieces; buffers only grow.
+// them long reads) and room for dyn_cap split-off pieces; buffers only grow.
 static int ensure_buffers(gs_batch* B, uint64_t span, uint64_t n, uint64_t tasks, uint64_t code_chunks,
-                          uint64_t n_items, uint64_t n_long, uint32_t maxlen, uint32_t dyn_cap) {
+                          uint64_t n_items, uint64_t n_long, uint32_t dyn_cap) {
   const uint64_t nr1 = n + 1;
   if (B->codes.ensure(16 * (code_chunks + 1)) || B->code_off.ensure(8 * nr1) ||
       B->items.ensure(8 * (n_items + 1)) || B->long_reads.ensure(4 * (n_long + 1)) ||
@@ -992,8 +992,7 @@ static int ensure_buffers(gs_batch* B, uint64_t span, uint64_t n, uint64_t tasks
       B->toff.ensure(8 * nr1) || B->batch.ensure(4 * nr1) || B->cand.ensure(16 * (2 * tasks + 1)) ||
       B->nF.ensure(4 * nr1) || B->nR.ensure(4 * nr1) || B->ns.ensure(4 * nr1) || B->np.ensure(4 * nr1) ||
       B->soff.ensure(8 * nr1) || B->poff.ensure(8 * nr1) || B->tiles.ensure(8 * (nr1 / kScanTile + 2)) ||
-      B->tot.ensure(16) || (maxlen > 256 && B->scratch.ensure(4 * (span + 16))) ||
-      B->queue.ensure(16) || B->counters.ensure(gs::kCounterBytes + gs::kColdBytes) ||
+      B->tot.ensure(16) || B->queue.ensure(16) || B->counters.ensure(gs::kCounterBytes + gs::kColdBytes) ||
       B->seg_link.ensure(n_long ? 4 * n_items : 16) ||
       (dyn_cap &&
        (B->dyn_items.ensure(16ull * dyn_cap) || B->dyn_meta.ensure(16ull * dyn_cap) ||
@@ -1010,7 +1009,7 @@ int gs::batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_
   // at most as many tasks as bases and code chunks as 32-base spans (+1)
   const uint64_t items = 2 * (reads + bases / seg_tasks + 1);
   const uint32_t dyn = gs::piece_cap(items);
-  int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, 0xFFFFFFFFu, dyn);
+  int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, dyn);
   if (!rc && bases > (4u << 20)) {  // the pinned chunks of staged uploads
     const size_t ch = std::min<uint64_t>(bases, kStageChunk);
     if (B->st_a.ensure(ch) || B->st_b.ensure(ch)) rc = GS_ENOMEM;
@@ -1087,6 +1086,25 @@ static int staged_upload(gs_batch* B, char* dst, const std::vector<std::pair<con
   return GS_OK;
 }
 
+// The work items of B's reads, from their lengths on the device.
+static int enqueue_items(gs_batch* B, hipStream_t st) {
+  const uint64_t n = B->n_reads, nr1 = n + 1;
+  uint32_t* cw = B->item_tmp.as<uint32_t>();
+  uint32_t *cs = cw + nr1, *cl = cw + 2 * nr1;
+  uint64_t* ow = reinterpret_cast<uint64_t*>(B->item_tmp.as<uint8_t>() + ((12 * nr1 + 7) & ~7ull));
+  uint64_t *os = ow + nr1, *ol = ow + 2 * nr1;
+  const uint32_t k = (uint32_t)B->opts.k;
+  hipLaunchKernelGGL(item_counts, dim3(grid_for(n, 256)), dim3(256), 0, st, B->lens.as<uint32_t>(), (uint32_t)n, k,
+                     B->seg_tasks, cw, cs, cl);
+  scan_counts(cw, n, ow, B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
+  scan_counts(cs, n, os, B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
+  scan_counts(cl, n, ol, B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
+  hipLaunchKernelGGL(item_fill, dim3(grid_for(n, 256)), dim3(256), 0, st, B->lens.as<uint32_t>(), (uint32_t)n, k,
+                     B->seg_tasks, ow, os, ol, B->items.as<uint64_t>(), B->long_reads.as<uint32_t>(),
+                     B->item0.as<uint64_t>());
+  return hipGetLastError() == hipSuccess ? GS_OK : GS_EHIP;
+}
+
 // Uploads a finished plan into B, reusing B's device buffers where they are
 // large enough.  B's results and any captured graph are dropped.
 int gs::batch_load(gs_batch* B, const BatchPlan& P) {
@@ -1099,7 +1117,6 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P) {
   B->n_reads = P.n_reads;
   B->span = P.span;
   B->tasks = P.tasks;
-  B->maxlen = P.maxlen;
   B->code_chunks = P.code_chunks;
   B->n_items = P.n_items;
   B->n_long = (uint32_t)P.n_long;
@@ -1107,9 +1124,9 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P) {
   B->n_seeds = B->n_pos = 0;
   B->ran = false;
   const uint64_t n = P.n_reads, nr1 = n + 1;
-  const bool split_on = P.opts.split_tasks != 0xFFFF && P.opts.kernel != 0;
+  const bool split_on = P.opts.split_tasks != 0xFFFF;
   B->dyn_cap = split_on ? gs::piece_cap(B->n_items) : 0u;
-  if (ensure_buffers(B, B->span, n, B->tasks, B->code_chunks, B->n_items, B->n_long, B->maxlen, B->dyn_cap))
+  if (ensure_buffers(B, B->span, n, B->tasks, B->code_chunks, B->n_items, B->n_long, B->dyn_cap))
     return GS_ENOMEM;
   hipStream_t st = B->stream;
   if (hipEventRecord(B->ev[0], st) != hipSuccess) return GS_EHIP;
@@ -1122,22 +1139,7 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P) {
        hipMemcpyAsync(B->batch.p, P.rbatch.data(), 4 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
        hipMemcpyAsync(B->code_off.p, P.code_off.data(), 8 * nr1, hipMemcpyHostToDevice, st) != hipSuccess))
     return GS_EHIP;
-  if (n) {  // the work items, from the lengths just uploaded
-    uint32_t* cw = B->item_tmp.as<uint32_t>();
-    uint32_t *cs = cw + nr1, *cl = cw + 2 * nr1;
-    uint64_t* ow = reinterpret_cast<uint64_t*>(B->item_tmp.as<uint8_t>() + ((12 * nr1 + 7) & ~7ull));
-    uint64_t *os = ow + nr1, *ol = ow + 2 * nr1;
-    const uint32_t k = (uint32_t)P.opts.k;
-    hipLaunchKernelGGL(item_counts, dim3(grid_for(n, 256)), dim3(256), 0, st, B->lens.as<uint32_t>(), (uint32_t)n,
-                       k, B->seg_tasks, cw, cs, cl);
-    scan_counts(cw, n, ow, B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
-    scan_counts(cs, n, os, B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
-    scan_counts(cl, n, ol, B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
-    hipLaunchKernelGGL(item_fill, dim3(grid_for(n, 256)), dim3(256), 0, st, B->lens.as<uint32_t>(), (uint32_t)n, k,
-                       B->seg_tasks, ow, os, ol, B->items.as<uint64_t>(), B->long_reads.as<uint32_t>(),
-                       B->item0.as<uint64_t>());
-    if (hipGetLastError() != hipSuccess) return GS_EHIP;
-  }
+  if (n && (rc = enqueue_items(B, st))) return rc;
   if (hipEventRecord(B->ev[1], st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return GS_EHIP;
   float ms = 0;
   (void)hipEventElapsedTime(&ms, B->ev[0], B->ev[1]);
@@ -1226,17 +1228,17 @@ static void fill_params(gs_batch* B, SeedParams& S, PostParams& Q) {
 static int enqueue_extension(gs_batch* B, const SeedParams& S, int kernel, unsigned pgrid, hipStream_t st,
                              hipEvent_t* kev = nullptr) {
   if (!B->n_reads) return GS_OK;
-  if (kernel == 0) {
-    if (kev && hipEventRecord(kev[0], st) != hipSuccess) return GS_EHIP;
+  if (B->streams) {
     if (B->maxlen <= 160)
       launch_seed<uint16_t, 160>(S, st);
     else
       launch_seed<uint16_t, 256>(S, st);
-    if (hipGetLastError() != hipSuccess) return GS_EHIP;
-    return kev && hipEventRecord(kev[1], st) != hipSuccess ? GS_EHIP : GS_OK;
+    return hipGetLastError() == hipSuccess ? GS_OK : GS_EHIP;
   }
   gs::PersistParams PP;
   PP.X = S.X;
+  PP.bases = S.bases;
+  PP.offs = S.offs;
   PP.codes = B->codes.as<uint4>();
   PP.code_off = B->code_off.as<uint64_t>();
   PP.lens = S.lens;
@@ -1289,8 +1291,10 @@ static int enqueue_extension(gs_batch* B, const SeedParams& S, int kernel, unsig
   J.dyn_cap = PP.dyn_cap;
   J.split_tasks = PP.split_tasks;
   J.pad = 0;
-  int rc = gs::launch_pack_codes(S.bases, S.offs, S.lens, PP.code_off, S.n_reads, J.long_reads, B->n_long,
-                                 B->codes.as<uint4>(), st);
+  int rc = GS_OK;
+  if (kernel)  // the plain kernel reads the bytes
+    rc = gs::launch_pack_codes(S.bases, S.offs, S.lens, PP.code_off, S.n_reads, J.long_reads, B->n_long,
+                               B->codes.as<uint4>(), st);
   if (!rc) rc = gs::launch_persistent(PP, kernel - 1, B->opts.wg, pgrid, st, kev ? kev[0] : nullptr,
                                       kev ? kev[1] : nullptr);
   if (!rc) rc = gs::launch_join(J, st);
@@ -1341,7 +1345,7 @@ static int enqueue_walk(gs_batch* B, const SeedParams& S, const PostParams& Q, h
 
 static int persistent_grid_for(gs_batch* B, int kernel, unsigned* grid) {
   *grid = 0;
-  if (kernel == 0 || !B->n_reads) return GS_OK;
+  if (B->streams || !B->n_reads) return GS_OK;
   return gs::persistent_grid(kernel - 1, B->opts.wg, grid);
 }
 
@@ -1856,8 +1860,9 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   if (rc) return rc;
   if (n_reads > 0xFFFFFFFFull / 2) return GS_ERANGE;
   const uint32_t n = (uint32_t)n_reads, k = (uint32_t)opts->k;
+  const uint32_t seg_tasks = opts->seg_tasks ? opts->seg_tasks : 64u;
   // sizes from the lengths alone (one pass, nothing allocated)
-  uint64_t lo = UINT64_MAX, hi = 0, tasks = 0, chunks = 0;
+  uint64_t lo = UINT64_MAX, hi = 0, tasks = 0, chunks = 0, n_items = 0, n_long = 0;
   uint32_t maxlen = 0;
   for (uint32_t i = 0; i < n; ++i) {
     const uint32_t L = lens[i];
@@ -1865,39 +1870,59 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
     if (offsets[i] + L > hi) hi = offsets[i] + L;
     tasks += L >= k ? L - k + 1 : 0;
     chunks += 2 * ((L + 31) / 32);
+    const uint32_t nseg = gs::n_segments(L, k, seg_tasks);
+    if (read_is_long(L, k, nseg)) ++n_long;
+    n_items += 2ull * nseg;
     if (L > maxlen) maxlen = L;
   }
   if (hi < lo) lo = hi = 0;
   const uint64_t span = hi - lo, nr1 = (uint64_t)n + 1;
-  // the persistent kernel takes reads held whole in its LDS window; a call
-  // with longer reads runs the plain kernel (the same output)
-  const int kernel = opts->kernel != 0 && maxlen <= gs::kPersistLmax ? opts->kernel : 0;
-  const bool long_scratch = kernel == 0 && maxlen > 256;
 
-  // slices of the scratch array, in order; outputs (seed records, rows) come
-  // after the counts are known
+  // Slices of the scratch array, in order.  What a call may hold is set by
+  // its first layout: reads of at most 160 bases with a batched kernel need
+  // their codes and two work items each, every other call the plain kernel
+  // seed_streams, which needs none, but for reads of more than 256 bases a
+  // size record per base and strand; the outputs come after that.
   uint64_t at = 0;
   auto take = [&](uint64_t bytes) {
     const uint64_t o = at;
     at = align256(at + bytes);
     return o;
   };
+  const bool short_batched = opts->kernel != 0 && maxlen <= gs::kPersistLmax;
+  const bool long_scratch = !short_batched && maxlen > 256;
   const uint64_t o_bases = take(span + 32), o_offs = take(8 * nr1), o_lens = take(4 * nr1),
-                 o_toff = take(8 * nr1), o_batch = take(4 * nr1), o_code_off = take(8 * nr1),
-                 o_items = kernel ? take(8 * (2 * (uint64_t)n + 1)) : 0,
-                 o_codes = kernel ? take(16 * (chunks + 1)) : 0, o_cand = take(16 * (2 * tasks + 1)),
+                 o_toff = take(8 * nr1), o_batch = take(4 * nr1), o_cand = take(16 * (2 * tasks + 1)),
                  o_nF = take(4 * nr1), o_nR = take(4 * nr1), o_ns = take(4 * nr1), o_np = take(4 * nr1),
                  o_soff = take(8 * nr1), o_poff = take(8 * nr1), o_tiles = take(8 * (nr1 / kScanTile + 2)),
-                 o_tot = take(16), o_queue = take(16), o_counters = take(gs::kCounterBytes + gs::kColdBytes),
-                 o_long = long_scratch ? take(4 * (span + 16)) : 0;
+                 o_tot = take(16), o_queue = take(16), o_counters = take(gs::kCounterBytes + gs::kColdBytes);
+  const uint64_t common = at;
+  const uint64_t o_code_off = take(8 * nr1), o_long = long_scratch ? take(4 * (span + 16)) : 0;
+  if (short_batched) {
+    take(16ull * n + 8);
+    take(16 * (chunks + 1));
+  }
   if (at > kNoAllocBytes) return GS_ERANGE;
   const uint64_t fixed = at;
-  // the pieces of work splitting, where they fit: they are dead once the
-  // streams are joined, and the outputs, written after that, take their place
-  const uint32_t cap = kernel && opts->split_tasks != 0xFFFF ? gs::piece_cap(2ull * n) : 0u;
+  // What runs: the kernel that gs_seed would run, if its buffers fit too
+  // (work items, segments of long reads; a call of reads longer than 160
+  // bases takes the place of the size records for them), else seed_streams.
+  // Everything from `out_at` on is dead once the streams are joined, and the
+  // outputs, written after that, take its place (out_at <= fixed: the list of
+  // long reads is no larger than the code offsets).
+  at = common;
+  const uint64_t o_long_reads = take(4 * (n_long + 1)), out_at = at;
+  const uint64_t o_code_off2 = take(8 * nr1);
+  const bool kernel_codes = opts->kernel != 0;
+  const uint64_t o_items = take(8 * (n_items + 1)), o_codes = kernel_codes ? take(16 * (chunks + 1)) : 0,
+                 o_item_tmp = n_long ? take(36 * nr1 + 8) : 0,
+                 o_item0 = take(8 * (n_long + 1)), o_seg_meta = n_long ? take(16 * n_items) : 0;
+  const bool streams = at > kNoAllocBytes;
+  const uint32_t cap = streams || opts->split_tasks == 0xFFFF ? 0u : gs::piece_cap(n_items);
   const uint64_t o_ditems = take(16ull * cap), o_dmeta = take(16ull * cap), o_dlink = take(4ull * cap),
-                 o_wmeta = take(32 * nr1), o_wlink = take(8 * nr1);
+                 o_wmeta = take(32 * nr1), o_wlink = take(8 * nr1), o_seg_link = n_long ? take(4 * n_items) : 0;
   const bool split_on = cap && at <= kNoAllocBytes;
+  const int kernel = streams ? 0 : opts->kernel;
 
   if (X->device < 0 || X->device >= kNoAllocDevices) return GS_EINVAL;
   if (hipSetDevice(X->device) != hipSuccess) return GS_EHIP;
@@ -1920,16 +1945,28 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   B.tasks = tasks;
   B.maxlen = maxlen;
   B.code_chunks = chunks;
-  B.n_items = kernel ? 2ull * n : 0;
-  B.n_long = 0;
-  B.seg_tasks = opts->seg_tasks ? opts->seg_tasks : 64u;
+  B.streams = streams;
+  B.n_items = streams ? 0 : n_items;
+  B.n_long = streams ? 0 : (uint32_t)n_long;
+  B.seg_tasks = seg_tasks;
   B.dyn_cap = split_on ? cap : 0u;
+  if (!streams) {
+    B.items.view(base + o_items, 8 * (n_items + 1));
+    if (kernel_codes) B.codes.view(base + o_codes, 16 * (chunks + 1));
+    B.long_reads.view(base + o_long_reads, 4 * (n_long + 1));
+    B.item0.view(base + o_item0, 8 * (n_long + 1));
+    if (n_long) {
+      B.item_tmp.view(base + o_item_tmp, 36 * nr1 + 8);
+      B.seg_meta.view(base + o_seg_meta, 16 * n_items);
+    }
+  }
   if (split_on) {
     B.dyn_items.view(base + o_ditems, 16ull * cap);
     B.dyn_meta.view(base + o_dmeta, 16ull * cap);
     B.dyn_link.view(base + o_dlink, 4ull * cap);
     B.wmeta.view(base + o_wmeta, 32 * nr1);
     B.wlink.view(base + o_wlink, 8 * nr1);
+    if (n_long) B.seg_link.view(base + o_seg_link, 4 * n_items);
   }
   uint64_t h_tot[2] = {0, 0};
   B.h_tot = h_tot;
@@ -1938,11 +1975,7 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   B.lens.view(base + o_lens, 4 * nr1);
   B.toff.view(base + o_toff, 8 * nr1);
   B.batch.view(base + o_batch, 4 * nr1);
-  B.code_off.view(base + o_code_off, 8 * nr1);
-  if (kernel) {
-    B.items.view(base + o_items, 8 * (2 * (uint64_t)n + 1));
-    B.codes.view(base + o_codes, 16 * (chunks + 1));
-  }
+  B.code_off.view(base + (streams ? o_code_off : o_code_off2), 8 * nr1);
   B.cand.view(base + o_cand, 16 * (2 * tasks + 1));
   B.nF.view(base + o_nF, 4 * nr1);
   B.nR.view(base + o_nR, 4 * nr1);
@@ -1954,7 +1987,7 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   B.tot.view(base + o_tot, 16);
   B.queue.view(base + o_queue, 16);
   B.counters.view(base + o_counters, gs::kCounterBytes + gs::kColdBytes);
-  if (long_scratch) B.scratch.view(base + o_long, 4 * (span + 16));
+  if (streams && long_scratch) B.scratch.view(base + o_long, 4 * (span + 16));
 
   // inputs, then the plan on the device
   if ((span && hipMemcpyAsync(B.bases.p, bases + lo, span, hipMemcpyHostToDevice, st) != hipSuccess) ||
@@ -1965,12 +1998,13 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   if (n) {
     hipLaunchKernelGGL(noalloc_prepare, dim3(grid_for(n, 256)), dim3(256), 0, st, B.offs.as<uint64_t>(),
                        B.lens.as<uint32_t>(), n, lo, k, B.ns.as<uint32_t>(), B.np.as<uint32_t>(),
-                       kernel ? B.items.as<uint64_t>() : (uint64_t*)nullptr);
+                       streams || n_long ? (uint64_t*)nullptr : B.items.as<uint64_t>());
     scan_counts(B.ns.as<uint32_t>(), n, B.toff.as<uint64_t>(), B.tiles.as<uint64_t>(), B.tot.as<uint64_t>(), st);
     scan_counts(B.np.as<uint32_t>(), n, B.code_off.as<uint64_t>(), B.tiles.as<uint64_t>(),
                 B.tot.as<uint64_t>() + 1, st);
     hipLaunchKernelGGL(noalloc_batch_ids, dim3(1), dim3(64), 0, st, B.lens.as<uint32_t>(), n,
                        opts->batch_bases ? opts->batch_bases : 1000000u, B.batch.as<uint32_t>());
+    if (n_long && !streams && (rc = enqueue_items(&B, st))) return rc;
   }
   if (hipGetLastError() != hipSuccess) return GS_EHIP;
 
@@ -1986,8 +2020,9 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   const uint64_t n_seeds = n ? h_tot[0] : 0, n_pos = n ? h_tot[1] : 0;
   out->n_seeds = n_seeds;
   out->n_pos = n_pos;
-  const uint64_t o_seeds = fixed, o_rows = align256(o_seeds + sizeof(gs_seed_rec) * (n_seeds + 1));
-  if (o_rows + 4 * (n_pos + 1) > kNoAllocBytes) return GS_ERANGE;
+  const uint64_t seeds_bytes = align256(sizeof(gs_seed_rec) * (n_seeds + 1));
+  if (fixed + seeds_bytes + 4 * (n_pos + 1) > kNoAllocBytes) return GS_ERANGE;
+  const uint64_t o_seeds = streams ? fixed : out_at, o_rows = o_seeds + seeds_bytes;
   if (n_seeds > out->seeds_cap || n_pos > out->pos_cap || (n_seeds && !out->seeds) || (n_pos && !out->pos))
     return GS_ERANGE;  // n_seeds and n_pos say what the call needs
   B.n_seeds = n_seeds;

@@ -998,52 +998,114 @@ seed_persistent(PersistArgs P) {
   }
 }
 
-// One piece of a stream (its task ends from t0 on, `m` = {candidates,
-// first finished b, last finished b, flags}) moved next to the stream's
-// earlier pieces; K candidates so far, LB = left end of the last finished
-// task so far.  A piece filters its own tasks in the lane, but its first
-// finished task had no predecessor there: it survives iff its left end is
-// smaller than LB (finish_task, 991-1018).  Candidate i moves from t0 + i to
-// K + i - drop (counted from the end the strand's region is packed against),
-// never toward a higher source index, so a candidate's destination is a
-// source that was read before it: moving `width` consecutive candidates at
-// once (all reads of a group before its writes) keeps that order.  width is
-// 1 for one thread, 64 for a wave whose lanes hold the same K and LB.
-__device__ __forceinline__ void join_piece(uint4* out, uint32_t ntask, uint32_t strand, uint32_t t0, uint4 m,
-                                           uint32_t smem, uint32_t& K, uint32_t& LB, uint32_t lane = 0,
-                                           uint32_t width = 1) {
-  const uint32_t drop = (smem && (m.w & 1u) && !(m.y < LB)) ? 1u : 0u;
-  for (uint32_t i0 = drop; i0 < m.x; i0 += width) {
-    const uint32_t i = i0 + lane;
-    if (i < m.x) {
-      if (strand == 0)
-        out[ntask - 1 - K - (i - drop)] = out[ntask - 1 - t0 - i];
-      else
-        out[ntask + K + (i - drop)] = out[ntask + t0 + i];
+// Joins the next pieces of a stream, one per lane in task order (`t0` its
+// first task, `m` = {candidates, first finished b, last finished b, flags},
+// all 0 in a lane without one), behind the K candidates joined so far; LB is
+// the left end of the last finished task so far.  Every lane of the wave
+// takes part.
+//
+// A piece filtered its own tasks, but its first finished task had no
+// predecessor there: it survives iff its left end is smaller than that of the
+// last finished task before it (finish_task, 991-1018), which is in the
+// nearest lane below with a finished task, or LB.  Candidate i of a piece
+// moves from t0 + i to its place behind the earlier ones (counted from the
+// end the strand's region is packed against).  The lanes move 128 candidates
+// at a time in output order, whatever pieces they come from (a segment of 64
+// task ends holds one or two): a destination is never above its source, and
+// sources increase, so no write of a round reaches a source of a later one.
+__device__ __forceinline__ void join_lanes(uint4* out, uint32_t ntask, uint32_t strand, uint32_t t0, uint4 m,
+                                           uint32_t smem, uint32_t& K, uint32_t& LB) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint64_t fin = __ballot((m.w & 2u) != 0);
+  const uint64_t before = fin & ((1ull << lane) - 1ull);
+  const uint32_t prev = __shfl(m.z, before ? 63 - __clzll((long long)before) : 0);
+  const uint32_t drop = (smem && (m.w & 1u) && !(m.y < (before ? prev : LB))) ? 1u : 0u;
+  const uint32_t n = m.x - drop;
+  uint32_t inc = n;  // candidates of the lanes up to this one
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t t = __shfl_up(inc, d);
+    if (lane >= (uint32_t)d) inc += t;
+  }
+  const uint32_t total = __shfl(inc, 63);
+  const uint32_t first = t0 + drop - (inc - n);  // output o of this piece comes from first + o
+  for (uint32_t o0 = 0; o0 < total; o0 += 128) {
+    uint4 c[2];
+#pragma unroll
+    for (uint32_t q = 0; q < 2; ++q) {
+      const uint32_t o = o0 + 64 * q + lane;
+      uint32_t p = 0;  // the lane whose piece holds output o
+#pragma unroll
+      for (uint32_t w = 32; w; w >>= 1)
+        if (__shfl(inc, (int)(p + w - 1)) <= o) p += w;
+      const uint32_t at = __shfl(first, (int)(p & 63u)) + o;
+      if (o < total) c[q] = strand == 0 ? out[ntask - 1 - at] : out[ntask + at];
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < 2; ++q) {
+      const uint32_t o = o0 + 64 * q + lane;
+      if (o < total) {
+        if (strand == 0)
+          out[ntask - 1 - K - o] = c[q];
+        else
+          out[ntask + K + o] = c[q];
+      }
     }
   }
-  K += m.x - drop;
-  if (m.w & 2u) LB = m.z;
+  K += total;
+  if (fin) LB = __shfl(m.z, 63 - __clzll((long long)fin));
 }
 
-// the pieces linked after an item, in task order (at most dyn_cap of them)
-__device__ __forceinline__ void join_chain(const gs::JoinParams& J, uint4* out, uint32_t ntask, uint32_t strand,
-                                           uint32_t link, uint32_t& K, uint32_t& LB, uint32_t lane = 0,
-                                           uint32_t width = 1) {
-  for (uint32_t guard = 0; link != kNone && guard < J.dyn_cap; ++guard) {
-    join_piece(out, ntask, strand, J.dyn_items[link].z, J.dyn_meta[link], J.smem, K, LB, lane, width);
+// pieces of one stream in task order, in LDS: at least the longest chain
+// (an item has at most kPersistLmax task ends) and its item
+constexpr uint32_t kJoinList = 192;
+static_assert(kJoinList > gs::kPersistLmax && kJoinList > gs::kSegTasksMax, "an item's pieces must fit the list");
+struct JoinList {
+  uint4 meta[kJoinList];
+  uint32_t t0[kJoinList];
+};
+
+__device__ __forceinline__ void join_list(const JoinList& list, uint32_t n, uint4* out, uint32_t ntask,
+                                          uint32_t strand, uint32_t smem, uint32_t& K, uint32_t& LB) {
+  const uint32_t lane = threadIdx.x & 63;
+  for (uint32_t i0 = 0; i0 < n; i0 += 64) {
+    const uint32_t i = i0 + lane;
+    const bool v = i < n;
+    join_lanes(out, ntask, strand, v ? list.t0[i] : 0u, v ? list.meta[i] : make_uint4(0, 0, 0, 0), smem, K, LB);
+  }
+}
+
+// writes an item and the pieces chained behind it to the list from `at` on
+__device__ __forceinline__ void list_chain(const gs::JoinParams& J, JoinList& list, uint32_t at, uint32_t t0, uint4 m,
+                                           uint32_t link, uint32_t n) {
+  for (uint32_t i = 0;; ++i) {
+    list.t0[at + i] = t0;
+    list.meta[at + i] = m;
+    if (i + 1 >= n) break;
+    m = J.dyn_meta[link];
+    t0 = J.dyn_items[link].z;
     link = J.dyn_link[link];
   }
 }
 
-// Streams of long reads, one wave per stream at a time (a 20 kbp read has
-// about 20,000 candidates per strand to move): segments in order, each
-// followed by the chain of pieces split off it; every lane follows the same
-// metadata and the lanes move 64 candidates at a time.  A fixed grid of
-// waves takes the streams in turn (a workgroup per four streams left the
-// launch bound by workgroup dispatch), and the metadata of 64 segments is
-// loaded at once, one segment per lane, then read from the lanes in order.
+__device__ __forceinline__ uint32_t chain_length(const gs::JoinParams& J, uint32_t link) {
+  uint32_t n = 0;
+  while (link != kNone && n + 1 < kJoinList) {
+    ++n;
+    link = J.dyn_link[link];
+  }
+  return n;
+}
+
+// Streams of long reads, one wave per stream at a time, a fixed grid of waves
+// taking the streams in turn: 64 segments at once, each followed by the chain
+// of pieces split off it.  The chains of the 64 segments are followed at
+// once, one per lane, into a list in LDS (a stream's segments and chains
+// followed one after another took 0.9 of 1.6 ms of a launch of 300 uneven
+// reads on the 3.1 Gbp index, whose pieces are small and many).
 __global__ void __launch_bounds__(256) join_segments(gs::JoinParams J) {
+  __shared__ JoinList lists[4];
+  JoinList& list = lists[threadIdx.x >> 6];
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t n_streams = 2ull * J.n_long, n_waves = gridDim.x * 4ull;
   for (uint64_t t = blockIdx.x * 4ull + (threadIdx.x >> 6); t < n_streams; t += n_waves) {
@@ -1058,36 +1120,90 @@ __global__ void __launch_bounds__(256) join_segments(gs::JoinParams J) {
     for (uint32_t g0 = 0; g0 < nseg; g0 += 64) {
       uint4 mine = make_uint4(0, 0, 0, 0);
       uint32_t link = kNone;
-      if (g0 + lane < nseg) {
+      const bool v = g0 + lane < nseg;
+      if (v) {
         const uint64_t it = i0 + 2 * (uint64_t)(g0 + lane);
         mine = J.seg_meta[it];
         if (J.dyn_cap) link = J.seg_link[it];
       }
-      const uint32_t ng = min(64u, nseg - g0);
-      for (uint32_t j = 0; j < ng; ++j) {
-        const uint4 m = make_uint4(__shfl(mine.x, j), __shfl(mine.y, j), __shfl(mine.z, j), __shfl(mine.w, j));
-        const uint32_t lk = __shfl(link, j);
-        join_piece(out, ntask, strand, (g0 + j) * S, m, J.smem, K, LB, lane, 64);
-        if (J.dyn_cap) join_chain(J, out, ntask, strand, lk, K, LB, lane, 64);
+      const uint32_t t0 = (g0 + lane) * S;
+      if (__ballot(link != kNone) == 0) {
+        join_lanes(out, ntask, strand, t0, mine, J.smem, K, LB);
+        continue;
+      }
+      const uint32_t n = v ? 1 + chain_length(J, link) : 0u;
+      uint32_t inc = n;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t a = __shfl_up(inc, d);
+        if (lane >= (uint32_t)d) inc += a;
+      }
+      uint32_t base = 0;  // pieces of the lanes done
+      const uint32_t all = __shfl(inc, 63);
+      while (base < all) {  // as many whole chains as fit the list
+        const bool in = n && inc > base && inc - base <= kJoinList;
+        if (in) list_chain(J, list, inc - n - base, t0, mine, link, n);
+        const uint64_t taken = __ballot(in);
+        const uint32_t upto = __shfl(inc, 63 - __clzll((long long)taken));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        join_list(list, upto - base, out, ntask, strand, J.smem, K, LB);
+        __builtin_amdgcn_wave_barrier();
+        base = upto;
       }
     }
     if (lane == 0) (strand ? J.nR : J.nF)[r] = K;
   }
 }
 
-// Whole-read streams that were split (one thread per stream of the batch;
-// the others were final already).
-__global__ void __launch_bounds__(256) join_whole(gs::JoinParams J) {
+// Whole-read streams that were split (the others were final already), one
+// wave per stream of the batch.
+__global__ void __launch_bounds__(256) join_whole_wave(gs::JoinParams J) {
+  __shared__ JoinList lists[4];
+  JoinList& list = lists[threadIdx.x >> 6];
+  const uint64_t t = blockIdx.x * 4ull + (threadIdx.x >> 6);
+  if (t >= 2ull * J.n_reads) return;
+  const uint32_t r = (uint32_t)(t >> 1), strand = (uint32_t)(t & 1);
+  uint32_t* const n_out = strand ? J.nR : J.nF;
+  if (n_out[r] != gs::kSplitStream) return;
+  const uint32_t ntask = J.lens[r] - J.k + 1;
+  const uint32_t link = J.wlink[t];
+  const uint32_t n = 1 + chain_length(J, link);
+  if ((threadIdx.x & 63) == 0) list_chain(J, list, 0, 0, J.wmeta[t], link, n);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  uint32_t K = 0, LB = 0xFFFFFFFFu;
+  join_list(list, n, J.cand + 2 * J.task_off[r], ntask, strand, J.smem, K, LB);
+  if ((threadIdx.x & 63) == 0) n_out[r] = K;
+}
+
+// The same, one thread per stream: candidate by candidate, each piece in
+// order (join_lanes' rules).
+__global__ void __launch_bounds__(256) join_whole_thread(gs::JoinParams J) {
   const uint64_t t = blockIdx.x * 256ull + threadIdx.x;
   if (t >= 2ull * J.n_reads) return;
   const uint32_t r = (uint32_t)(t >> 1), strand = (uint32_t)(t & 1);
   uint32_t* const n_out = strand ? J.nR : J.nF;
   if (n_out[r] != gs::kSplitStream) return;
   const uint32_t ntask = J.lens[r] - J.k + 1;
-  uint4* out = J.cand + 2 * J.task_off[r];
-  uint32_t K = 0, LB = 0xFFFFFFFFu;
-  join_piece(out, ntask, strand, 0, J.wmeta[t], J.smem, K, LB);
-  join_chain(J, out, ntask, strand, J.wlink[t], K, LB);
+  uint4* const out = J.cand + 2 * J.task_off[r];
+  uint32_t K = 0, LB = 0xFFFFFFFFu, t0 = 0, link = J.wlink[t];
+  uint4 m = J.wmeta[t];
+  for (uint32_t guard = 0; guard < kJoinList; ++guard) {
+    const uint32_t drop = (J.smem && (m.w & 1u) && !(m.y < LB)) ? 1u : 0u;
+    for (uint32_t i = drop; i < m.x; ++i) {
+      if (strand == 0)
+        out[ntask - 1 - K - (i - drop)] = out[ntask - 1 - t0 - i];
+      else
+        out[ntask + K + (i - drop)] = out[ntask + t0 + i];
+    }
+    K += m.x - drop;
+    if (m.w & 2u) LB = m.z;
+    if (link == kNone) break;
+    m = J.dyn_meta[link];
+    t0 = J.dyn_items[link].z;
+    link = J.dyn_link[link];
+  }
   n_out[r] = K;
 }
 
@@ -1259,8 +1375,15 @@ int launch_join(const JoinParams& J, hipStream_t st) {
                        st, J);
   }
   if (J.dyn_cap && J.n_reads) {
-    const uint64_t threads = 2ull * J.n_reads;
-    hipLaunchKernelGGL(join_whole, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, J);
+    // A wave per stream up to 16,384 streams, where nearly all were split and
+    // their chains' latency counts (64 reads: 36 -> 25 us); a thread per
+    // stream beyond, where few were (600,000 streams: 76 us, with waves that
+    // look at 37 streams each 167 us).
+    const uint64_t streams = 2ull * J.n_reads;
+    if (streams <= 16384)
+      hipLaunchKernelGGL(join_whole_wave, dim3((unsigned)((streams + 3) / 4)), dim3(256), 0, st, J);
+    else
+      hipLaunchKernelGGL(join_whole_thread, dim3((unsigned)((streams + 255) / 256)), dim3(256), 0, st, J);
   }
   return hipGetLastError() == hipSuccess ? GS_OK : GS_EHIP;
 }

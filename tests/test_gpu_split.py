@@ -86,3 +86,42 @@ def test_noalloc_splits_like_gs_seed(g, case, smem):
             for kw in (dict(), dict(split_tasks=1), dict(split_tasks=g.NO_SPLIT)):
                 say("noalloc smem=%d reads=%d %s" % (smem, n, kw))
                 assert same(g.seed_noalloc(X, arrays, k=19, smem=smem, kernel=3, **kw), want), (n, kw)
+
+
+@pytest.mark.parametrize("n", [8192, 8193])
+def test_joins_on_both_sides_of_the_wave_per_stream_rule(g, case, n):
+    """16,384 streams and two more."""
+    base = g.pack_reads(case["short"])
+    pick = np.random.default_rng(n).integers(0, len(base[2]), n)
+    arrays = (base[0], base[1][pick], base[2][pick])
+    with g.Index(case["prefix"]) as X:
+        for smem in (True, False):
+            want = g.seed(X, arrays=arrays, k=17, smem=smem, kernel=3, split_tasks=g.NO_SPLIT)
+            assert same(g.seed(X, arrays=arrays, k=17, smem=smem, kernel=3, split_tasks=1), want), smem
+
+
+@pytest.mark.parametrize("seg_tasks", [1, 2, 40, 112])
+def test_joins_of_segments_and_their_pieces(g, case, seg_tasks):
+    """Reads of 63, 64, 65 and 129 segments (one lane each, 64 at a time), and
+    of many short ones; every segment split as far as it goes, so that 64
+    chains do not fit the join's list at once."""
+    import oracle_bind as ob
+    rng = random.Random(seg_tasks)
+    k = 15
+    text = "".join(case["longer"][i].decode() for i in range(40)).replace("N", "A")
+    reads = []
+    for nseg in (63, 64, 65, 129):
+        L = min(nseg * seg_tasks + k - 1, len(text) - 1)
+        p = rng.randrange(0, len(text) - L)
+        reads.append(text[p:p + L].encode())
+    reads += case["longer"][:8]
+    ox = ob.Index(case["prefix"])
+    with g.Index(case["prefix"]) as X:
+        for smem in (True, False):
+            want, _ = ob.seed(ox, reads, k, smem=smem, prune=1)
+            want = [[(x, y, l, u, list(p)) for (x, y, l, u, p) in r] for r in want]
+            for kw in (dict(split_tasks=1), dict(split_tasks=g.NO_SPLIT), dict(kernel=0, split_tasks=1)):
+                kw.setdefault("kernel", 3)
+                say("seg_tasks=%d smem=%d %s" % (seg_tasks, smem, kw))
+                assert g.seed(X, reads, k=k, smem=smem, seg_tasks=seg_tasks, **kw).as_lists() == want, kw
+    ox.close()

@@ -412,102 +412,156 @@ __device__ uint2 mem_skip(const PostParams& P, uint32_t r, int rev, uint32_t i) 
   return skip;
 }
 
-// One lane per read.  Count pass (write == false): seeds and positions per
-// read.  Write pass: seed records and suffix-array rows at the scanned offsets,
-// merged by qbeg with forward entries first on ties (the stable segmented sort
-// at 1233 and 3570).
-// One entry of the merged lists: its seed record and rows (write pass), or
-// only its counts; the seeds and positions it adds.
-template <bool WRITE>
-__device__ __forceinline__ void finalize_entry(const PostParams& P, uint32_t r, const ReadLists& Ls, int rev,
-                                               uint32_t i, uint64_t so, uint64_t po, uint32_t& ns,
-                                               uint32_t& np) {
-  const uint4 en = rev ? Ls.R[i] : Ls.F[i];
-  const uint32_t sz = isize(en);
-  uint32_t cnt = P.smem ? sz : mem_count(Ls, rev, i);
-  if (cnt == 0) return;
-  if (P.max_occ && sz > P.max_occ) cnt = 0;
-  if (WRITE) {
-    gs_seed_rec rec;
-    rec.qbeg = en.x;
-    rec.qend = en.y;
-    rec.l = en.z;
-    rec.u = en.w;
-    rec.n_pos = cnt;
-    rec.pad = 0;
-    P.seeds[so + ns] = rec;
-    if (cnt) {
-      uint2 skip = make_uint2(1, 0);
-      if (!P.smem) skip = mem_skip(P, r, rev, i);
-      uint32_t row = en.z, got = 0;
-      while (got < cnt) {
-        if (row < skip.x || row > skip.y) P.rows[po + np + got++] = row;
-        ++row;
-      }
-    }
-  }
-  ++ns;
-  np += cnt;
-}
-
-// the next entry of the merge: forward entries first on ties of qbeg
+// the next entry of the merge: forward entries first on ties of qbeg (the
+// stable segmented sort at 1233 and 3570)
 __device__ __forceinline__ bool take_forward(const ReadLists& Ls, uint32_t a, uint32_t z) {
   return z >= Ls.nR || (a < Ls.nF && Ls.F[a].x <= (Ls.R[z].x & 0x7FFFFFFFu));
 }
 
-template <bool WRITE>
-__global__ void __launch_bounds__(256) finalize_reads(PostParams P) {
-  const uint32_t r = blockIdx.x * 256 + threadIdx.x;
-  if (r >= P.n_reads) return;
-  if (P.lens[r] > P.long_min && P.lens[r] >= P.k) return;  // finalize_long's (the reads of long_reads)
-  const ReadLists Ls = lists_of(P, r);
-  uint32_t ns = 0, np = 0;
-  uint64_t so = WRITE ? P.seed_off[r] : 0, po = WRITE ? P.pos_off[r] : 0;
-  uint32_t a = 0, z = 0;
-  while (a < Ls.nF || z < Ls.nR) {
-    const bool takeF = take_forward(Ls, a, z);
-    finalize_entry<WRITE>(P, r, Ls, takeF ? 0 : 1, takeF ? a++ : z++, so, po, ns, np);
-  }
-  if (!WRITE) {
-    P.nseeds[r] = ns;
-    P.npos[r] = np;
+// A lane's part of the merged entries of read r: `left` of them, from forward
+// entry a and reverse entry z on.
+struct Part {
+  ReadLists Ls;
+  uint32_t r, a, z, left;
+};
+
+// The entry at the part's front: its list and index, its interval, and the
+// rows it reports (none for an entry that is no seed, `seed` false; none for
+// a seed over max_occ).
+struct Entry {
+  uint4 en;
+  uint32_t i, cnt;
+  int rev;
+  bool seed;
+};
+
+__device__ __forceinline__ Entry take_entry(const PostParams& P, Part& p) {
+  Entry e;
+  e.rev = take_forward(p.Ls, p.a, p.z) ? 0 : 1;
+  e.i = e.rev ? p.z++ : p.a++;
+  --p.left;
+  e.en = e.rev ? p.Ls.R[e.i] : p.Ls.F[e.i];
+  const uint32_t sz = isize(e.en);
+  e.cnt = P.smem ? sz : mem_count(p.Ls, e.rev, e.i);
+  e.seed = e.cnt != 0;
+  if (P.max_occ && sz > P.max_occ) e.cnt = 0;
+  return e;
+}
+
+// Row i of the rows from z on that are not in [skip.x, skip.y].
+__device__ __forceinline__ uint32_t nth_row(uint32_t z, uint2 skip, uint32_t i) {
+  if (skip.x > skip.y || z > skip.y) return z + i;
+  const uint32_t before = skip.x > z ? skip.x - z : 0u;
+  return i < before ? z + i : skip.y + 1u + (i - before);
+}
+
+// seeds and positions of the part's entries
+__device__ __forceinline__ void count_part(const PostParams& P, Part p, uint32_t& ns, uint32_t& np) {
+  ns = np = 0;
+  while (p.left) {
+    const Entry e = take_entry(P, p);
+    ns += e.seed ? 1u : 0u;
+    np += e.cnt;
   }
 }
 
-// Reads longer than long_min bases (thousands of entries each): one wave per
-// read.  Lane l takes positions [l*T/64, (l+1)*T/64) of the merged order of
-// the T = nF + nR entries; its starting split between the two lists is found
-// by binary search on the merge path (the number a of forward entries among
-// the first d merged is the smallest a at which forward entry a does not come
-// before reverse entry d-a-1).  The count pass sums the lanes' seeds and
-// positions; the write pass counts first, scans the lanes' counts for their
-// output offsets, then merges its part again and writes.
-template <bool WRITE>
-__global__ void __launch_bounds__(256) finalize_long(PostParams P) {
-  const uint32_t w = blockIdx.x * 4 + (threadIdx.x >> 6);
+// Writes the seed records of the lanes' parts from so on, and their rows from
+// po on.  The lanes take an entry each per turn and then write the rows of
+// all of them together, 64 at a time whatever entry they are of: one seed may
+// report as many rows as max_occ allows, or the whole of a repeat, and a lane
+// writing its own rows kept its wave waiting.  Records and rows, max_occ 500:
+// 300,007 MEM reads of up to 101 bases on a 100 Mbp index 2.09 -> 0.17 ms
+// (with the sharing of kSharedEntries), 100,000 SMEM reads of 150 there 0.15
+// -> 0.03 ms.  Reading the full suffix array here in place of locate_rows'
+// pass was slower (1,000,000 reads on the 3.1 Gbp index 0.30 ms against 0.25,
+// 60,000 uneven reads 0.40 against 0.29): its loads wait a turn each.
+// Every lane of the wave takes part.
+__device__ void write_parts(const PostParams& P, Part p, uint64_t so, uint64_t po) {
   const uint32_t lane = threadIdx.x & 63;
-  if (w >= P.n_long) return;
-  const uint32_t r = P.long_reads[w];
-  const ReadLists Ls = lists_of(P, r);
-  const uint32_t T = Ls.nF + Ls.nR;
+  while (__ballot(p.left != 0)) {
+    uint32_t cnt = 0, z = 0, done = 0;
+    uint2 skip = make_uint2(1, 0);
+    uint64_t dst = po;
+    if (p.left) {
+      const Entry e = take_entry(P, p);
+      if (e.seed) {
+        gs_seed_rec rec;
+        rec.qbeg = e.en.x;
+        rec.qend = e.en.y;
+        rec.l = e.en.z;
+        rec.u = e.en.w;
+        rec.n_pos = e.cnt;
+        rec.pad = 0;
+        P.seeds[so++] = rec;
+        cnt = e.cnt;
+        z = e.en.z;
+        po += cnt;
+        if (cnt && !P.smem) skip = mem_skip(P, p.r, e.rev, e.i);
+      }
+    }
+    while (__ballot(cnt != 0)) {
+      const uint32_t c = cnt < 65536u ? cnt : 65536u;  // of this lane's rows, in this turn
+      uint32_t inc = c;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t t = __shfl_up(inc, d);
+        if (lane >= (uint32_t)d) inc += t;
+      }
+      const uint32_t total = __shfl(inc, 63), first = inc - c;
+      for (uint32_t o0 = 0; o0 < total; o0 += 64) {
+        const uint32_t o = o0 + lane;
+        uint32_t q = 0;  // the lane whose rows hold o
+#pragma unroll
+        for (uint32_t w = 32; w; w >>= 1)
+          if (__shfl(inc, (int)(q + w - 1)) <= o) q += w;
+        q &= 63u;
+        const uint32_t i = o - __shfl(first, (int)q) + __shfl(done, (int)q);
+        const uint2 sk = make_uint2(__shfl(skip.x, (int)q), __shfl(skip.y, (int)q));
+        const uint32_t zq = __shfl(z, (int)q);
+        const uint64_t at = __shfl(dst, (int)q) + i;
+        if (o < total) P.rows[at] = nth_row(zq, sk, i);
+      }
+      done += c;
+      cnt -= c;
+    }
+  }
+}
+
+// Lane l's part of read r when the wave shares it: positions
+// [l*T/64, (l+1)*T/64) of the merged order of the T = nF + nR entries; its
+// starting split between the two lists is found by binary search on the merge
+// path (the number a of forward entries among the first d merged is the
+// smallest a at which forward entry a does not come before reverse entry
+// d-a-1).
+__device__ __forceinline__ Part shared_part(const PostParams& P, uint32_t r) {
+  const uint32_t lane = threadIdx.x & 63;
+  Part p;
+  p.r = r;
+  p.Ls = lists_of(P, r);
+  const uint32_t T = p.Ls.nF + p.Ls.nR;
   const uint32_t d0 = (uint32_t)((uint64_t)T * lane / 64), d1 = (uint32_t)((uint64_t)T * (lane + 1) / 64);
-  uint32_t lo = d0 > Ls.nR ? d0 - Ls.nR : 0, hi = d0 < Ls.nF ? d0 : Ls.nF;
+  uint32_t lo = d0 > p.Ls.nR ? d0 - p.Ls.nR : 0, hi = d0 < p.Ls.nF ? d0 : p.Ls.nF;
   while (lo < hi) {
     const uint32_t a = (lo + hi) >> 1, b = d0 - a;
-    if (b > 0 && Ls.F[a].x <= (Ls.R[b - 1].x & 0x7FFFFFFFu))
+    if (b > 0 && p.Ls.F[a].x <= (p.Ls.R[b - 1].x & 0x7FFFFFFFu))
       lo = a + 1;  // forward entry a is merged before reverse entry b-1
     else
       hi = a;
   }
-  const uint32_t a0 = lo, z0 = d0 - lo;
-  uint32_t ns = 0, np = 0;
-  {
-    uint32_t a = a0, z = z0;
-    for (uint32_t d = d0; d < d1; ++d) {
-      const bool takeF = take_forward(Ls, a, z);
-      finalize_entry<false>(P, r, Ls, takeF ? 0 : 1, takeF ? a++ : z++, 0, 0, ns, np);
-    }
-  }
+  p.a = lo;
+  p.z = d0 - lo;
+  p.left = d1 - d0;
+  return p;
+}
+
+// One read by the whole wave: its counts (WRITE false), or its records and
+// rows, each lane's from the scanned counts of the lanes before it.
+template <bool WRITE>
+__device__ __forceinline__ void finalize_shared(const PostParams& P, uint32_t r) {
+  const uint32_t lane = threadIdx.x & 63;
+  const Part p = shared_part(P, r);
+  uint32_t ns, np;
+  count_part(P, p, ns, np);
   // inclusive scans over the lanes (64-bit positions: a read's rows can
   // exceed 2^32 only through pathological counts, so sum in 64 bits)
   uint64_t sn = ns, sp = np;
@@ -523,15 +577,57 @@ __global__ void __launch_bounds__(256) finalize_long(PostParams P) {
       P.nseeds[r] = (uint32_t)sn;
       P.npos[r] = (uint32_t)sp;
     }
-    return;
+  } else {
+    write_parts(P, p, P.seed_off[r] + (sn - ns), P.pos_off[r] + (sp - np));
   }
-  const uint64_t so = P.seed_off[r] + (sn - ns), po = P.pos_off[r] + (sp - np);
-  uint32_t ws = 0, wp = 0;
-  uint32_t a = a0, z = z0;
-  for (uint32_t d = d0; d < d1; ++d) {
-    const bool takeF = take_forward(Ls, a, z);
-    finalize_entry<true>(P, r, Ls, takeF ? 0 : 1, takeF ? a++ : z++, so, po, ws, wp);
+}
+
+// Reads with more merged entries than this are shared by the wave's lanes
+// (MEM reads in repeats have up to two entries per base; counts and records
+// of 200,000 MEM reads on the 3.1 Gbp index with 8, 16, 24 and 48: 0.68, 0.68,
+// 0.71, 0.84 ms; 1,000,000 SMEM reads with 4, 16: 0.75, 0.43 ms).
+constexpr uint32_t kSharedEntries = 16;
+
+// A lane per read, then the wave together for each of its reads with many
+// entries.  Count pass (WRITE false): seeds and positions per read.  Write
+// pass: seed records and suffix-array rows at the scanned offsets.
+template <bool WRITE>
+__global__ void __launch_bounds__(256) finalize_reads(PostParams P) {
+  const uint32_t r = blockIdx.x * 256 + threadIdx.x;
+  const bool mine = r < P.n_reads && !(P.lens[r] > P.long_min && P.lens[r] >= P.k);  // else finalize_long's
+  Part p;
+  p.r = r;
+  p.a = p.z = p.left = 0;
+  if (mine) {
+    p.Ls = lists_of(P, r);
+    p.left = p.Ls.nF + p.Ls.nR;
   }
+  const uint64_t many = __ballot(p.left > kSharedEntries);
+  const bool own = mine && p.left <= kSharedEntries;
+  if (!own) p.left = 0;
+  if (!WRITE) {
+    uint32_t ns, np;
+    count_part(P, p, ns, np);
+    if (own) {
+      P.nseeds[r] = ns;
+      P.npos[r] = np;
+    }
+  } else {
+    write_parts(P, p, own ? P.seed_off[r] : 0, own ? P.pos_off[r] : 0);
+  }
+  for (uint64_t m = many; m; m &= m - 1) {
+    const uint32_t lead = (uint32_t)(__ffsll((unsigned long long)m) - 1);
+    finalize_shared<WRITE>(P, (uint32_t)__builtin_amdgcn_readlane((int)r, (int)lead));
+  }
+}
+
+// Reads longer than long_min bases (thousands of entries each): one wave per
+// read.
+template <bool WRITE>
+__global__ void __launch_bounds__(256) finalize_long(PostParams P) {
+  const uint32_t w = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= P.n_long) return;
+  finalize_shared<WRITE>(P, P.long_reads[w]);
 }
 
 // ---- exclusive scan of per-read counts into 64-bit offsets ---------------

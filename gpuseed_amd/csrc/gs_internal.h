@@ -228,16 +228,25 @@ int launch_join(const JoinParams& J, hipStream_t st);
 namespace gs {
 
 // The CPU side of a batch (see gs_batch_create): built on any thread, then
-// uploaded by batch_load.  Per read only; the work items of the persistent
-// kernel (n_items of them, n_long reads cut into segments) are written on the
-// device when the batch is loaded.
+// uploaded by batch_load.  Sizes and the sources of the uploads; offsets of
+// tasks and codes, reference-batch ids and work items (n_items of them, n_whole
+// of reads held whole, n_long reads cut into segments) are written on the
+// device when the batch is loaded.  The reads' bytes, and a single group's
+// arrays unless plan_finish copied them, must stay as they are until then.
 struct BatchPlan {
   gs_opts opts{};
-  uint32_t seg_tasks = 64, next_batch_id = 0;
-  uint64_t n_reads = 0, span = 0, tasks = 0, code_chunks = 0, n_items = 0, n_long = 0;
+  uint32_t seg_tasks = 64;
+  uint64_t n_reads = 0, span = 0, tasks = 0, code_chunks = 0, n_items = 0, n_whole = 0, n_long = 0;
   std::vector<std::pair<const char*, uint64_t>> pieces;  // bytes uploaded back to back
-  std::vector<uint64_t> offs, task_off, code_off;
-  std::vector<uint32_t> lens, rbatch;
+  struct Group {  // reads of one source: offsets less lo, plus base, are theirs in the batch
+    const uint64_t* offs;
+    const uint32_t* lens;
+    uint64_t n, lo, base;
+  };
+  std::vector<Group> groups;
+  std::vector<uint32_t> cuts;  // first reads of the second reference batch and those after it
+  std::vector<uint64_t> offs;  // of several groups (plan_finish)
+  std::vector<uint32_t> lens;
 };
 
 int plan_check(const gs_opts* o);
@@ -245,7 +254,7 @@ void plan_reset(BatchPlan& P, const gs_opts& o);
 // appends reads [r0, r1) of one source as a group of their own
 int plan_add(BatchPlan& P, const char* bases, const uint64_t* offsets, const uint32_t* lens, uint64_t r0,
              uint64_t r1);
-void plan_finish(BatchPlan& P);
+void plan_finish(BatchPlan& P, bool copy = false);
 uint64_t plan_device_bytes(const BatchPlan& P);  // device buffers the plan needs, outputs excluded
 // hold: the batch keeps a reference to X (every batch but gs_seed's own,
 // which the index owns and frees)

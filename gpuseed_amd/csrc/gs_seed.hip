@@ -630,10 +630,14 @@ __global__ void __launch_bounds__(256) finalize_long(PostParams P) {
   finalize_shared<WRITE>(P, P.long_reads[w]);
 }
 
-// ---- exclusive scan of per-read counts into 64-bit offsets ---------------
-// Three launches: per-workgroup totals, a single-workgroup scan of those
-// totals, then per-workgroup local scans offset by the scanned totals.  Waves
-// scan with shuffles; the workgroup combines its four wave totals in LDS.
+// ---- exclusive scans of per-read counts into 64-bit offsets --------------
+// Seeds and positions are scanned together, as are the five counts of a
+// batch's plan (below), each in three launches: per-workgroup totals, a
+// single-workgroup scan of those totals, then per-workgroup local scans offset
+// by the scanned totals; in the last one alone where one workgroup holds all
+// the reads.  (One scan of three launches per count made 24 of the 40 launches
+// of a call of 1000 reads.)  Waves scan with shuffles; the workgroup combines
+// its four wave totals in LDS.
 
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 8;  // per thread
@@ -665,48 +669,77 @@ __device__ __forceinline__ uint64_t block_excl_scan(uint64_t v, uint64_t* tot) {
   return before + inc - v;
 }
 
-__global__ void __launch_bounds__(kScanBlock) scan_tile_totals(const uint32_t* __restrict__ in, uint64_t n,
-                                                               uint64_t* __restrict__ tiles) {
-  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
-  uint64_t s = 0;
-  for (int q = 0; q < kScanItems; ++q)
-    if (base + q < n) s += in[base + q];
-  uint64_t tot;
-  block_excl_scan(s, &tot);
-  if (threadIdx.x == 0) tiles[blockIdx.x] = tot;
-}
-
+// NQ rows of ntiles totals, each scanned exclusively in place; row q's total
+// to total[q] (total may be null)
+template <int NQ>
 __global__ void __launch_bounds__(kScanBlock) scan_tiles(uint64_t* __restrict__ tiles, uint64_t ntiles,
                                                          uint64_t* __restrict__ total) {
-  uint64_t carry = 0;
-  for (uint64_t base = 0; base < ntiles; base += kScanBlock) {
-    const uint64_t i = base + threadIdx.x;
-    const uint64_t v = i < ntiles ? tiles[i] : 0;
-    uint64_t tot;
-    const uint64_t ex = block_excl_scan(v, &tot);
-    if (i < ntiles) tiles[i] = carry + ex;
-    carry += tot;
+  for (int q = 0; q < NQ; ++q) {
+    uint64_t* const row = tiles + q * ntiles;
+    uint64_t carry = 0;
+    for (uint64_t base = 0; base < ntiles; base += kScanBlock) {
+      const uint64_t i = base + threadIdx.x;
+      const uint64_t v = i < ntiles ? row[i] : 0;
+      uint64_t tot;
+      const uint64_t ex = block_excl_scan(v, &tot);
+      if (i < ntiles) row[i] = carry + ex;
+      carry += tot;
+    }
+    if (total && threadIdx.x == 0) total[q] = carry;
   }
-  if (threadIdx.x == 0) *total = carry;
 }
 
-__global__ void __launch_bounds__(kScanBlock) scan_apply(const uint32_t* __restrict__ in, uint64_t n,
-                                                         const uint64_t* __restrict__ tiles,
-                                                         uint64_t* __restrict__ out) {
-  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
-  uint32_t v[kScanItems];
+// seeds and positions per read, scanned into their offsets
+struct PairScan {
+  const uint32_t* in[2];
+  uint64_t* out[2];  // n + 1 entries each
+  uint64_t n, ntiles;
+  uint64_t* tiles;  // [2][ntiles]
+  uint64_t* total;  // [2]
+};
+
+// the thread's kScanItems counts from `base` on (sum returned, each in v)
+__device__ __forceinline__ uint64_t load_counts(const uint32_t* __restrict__ in, uint64_t n, uint64_t base,
+                                                uint32_t* v) {
   uint64_t s = 0;
+#pragma unroll
   for (int q = 0; q < kScanItems; ++q) {
     v[q] = base + q < n ? in[base + q] : 0u;
     s += v[q];
   }
-  uint64_t tot;
-  uint64_t run = tiles[blockIdx.x] + block_excl_scan(s, &tot);
-  for (int q = 0; q < kScanItems; ++q) {
-    if (base + q < n) out[base + q] = run;
-    run += v[q];
+  return s;
+}
+
+__global__ void __launch_bounds__(kScanBlock) pair_totals(PairScan S) {
+  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    uint32_t v[kScanItems];
+    uint64_t tot;
+    block_excl_scan(load_counts(S.in[h], S.n, base, v), &tot);
+    if (threadIdx.x == 0) S.tiles[h * S.ntiles + blockIdx.x] = tot;
   }
-  if (base + kScanItems >= n && base < n) out[n] = run;  // the thread holding the last item
+}
+
+__global__ void __launch_bounds__(kScanBlock) pair_apply(PairScan S) {
+  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    uint32_t v[kScanItems];
+    uint64_t tot;
+    uint64_t run = block_excl_scan(load_counts(S.in[h], S.n, base, v), &tot);
+    if (S.ntiles == 1) {
+      if (threadIdx.x == 0) S.total[h] = tot;
+    } else {
+      run += S.tiles[h * S.ntiles + blockIdx.x];
+    }
+#pragma unroll
+    for (int q = 0; q < kScanItems; ++q) {
+      if (base + q < S.n) S.out[h][base + q] = run;
+      run += v[q];
+    }
+    if (base + kScanItems >= S.n && base < S.n) S.out[h][S.n] = run;  // the thread holding the last item
+  }
 }
 
 // ---- suffix-array walk (locate_seeds_gpu, 668-684) -------------------------
@@ -790,41 +823,133 @@ __host__ __device__ __forceinline__ bool read_is_long(uint32_t L, uint32_t k, ui
   return nseg > 1 || (L > gs::kPersistLmax && L >= k);
 }
 
-// per read: items as a whole-read stream, items as segments, 1 if segmented
-__global__ void item_counts(const uint32_t* __restrict__ lens, uint32_t n, uint32_t k, uint32_t seg_tasks,
-                            uint32_t* __restrict__ c_whole, uint32_t* __restrict__ c_seg,
-                            uint32_t* __restrict__ c_long) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t L = lens[i];
-  const uint32_t nseg = gs::n_segments(L, k, seg_tasks);
-  const bool lng = read_is_long(L, k, nseg);
-  c_whole[i] = lng ? 0u : 2u;
-  c_seg[i] = lng ? 2u * nseg : 0u;
-  c_long[i] = lng ? 1u : 0u;
+// The rest of a batch's plan, from the reads' lengths: task and code-chunk
+// offsets, the reads' offsets rebased onto the uploaded bytes, the
+// reference-batch ids that MEM's row skip needs, and the work items (null
+// code_off, items: not needed).
+constexpr uint32_t kInlineCuts = 16;
+struct PlanParams {
+  uint64_t* offs;
+  const uint32_t* lens;
+  uint64_t n, lo;      // lo: subtracted from the offsets
+  uint64_t n_whole;    // items of reads held whole
+  uint32_t k, seg_tasks;
+  // first reads of the second reference batch and of those after it: in `cut`
+  // (at most kInlineCuts), or at `cuts`; batch null: not needed
+  uint32_t* batch;
+  const uint32_t* cuts;
+  uint32_t n_cuts;
+  uint32_t cut[kInlineCuts];
+  uint64_t* toff;      // n + 1 entries, as code_off
+  uint64_t* code_off;
+  uint64_t* items;
+  uint32_t* long_reads;
+  uint64_t* item0;
+  uint64_t* tiles;     // [kPlanSums][ntiles]
+  uint64_t ntiles;
+};
+constexpr int kPlanSums = 5;
+
+// a read's tasks, code chunks, items as a whole-read stream, items as
+// segments, and 1 if it is segmented (0s past the last read)
+__device__ __forceinline__ bool plan_counts(const PlanParams& P, uint64_t i, uint32_t& L, uint32_t* c) {
+#pragma unroll
+  for (int q = 0; q < kPlanSums; ++q) c[q] = 0;
+  L = 0;
+  if (i >= P.n) return false;
+  L = P.lens[i];
+  const uint32_t nseg = gs::n_segments(L, P.k, P.seg_tasks);
+  const bool lng = read_is_long(L, P.k, nseg);
+  c[0] = L >= P.k ? L - P.k + 1 : 0u;
+  c[1] = 2u * (L / 32u + (L % 32u ? 1u : 0u));
+  c[lng ? 3 : 2] = 2u * nseg;
+  c[4] = lng ? 1u : 0u;
+  return lng;
 }
 
-// o_whole, o_seg, o_long: exclusive scans of the counts (n + 1 entries)
-__global__ void item_fill(const uint32_t* __restrict__ lens, uint32_t n, uint32_t k, uint32_t seg_tasks,
-                          const uint64_t* __restrict__ o_whole, const uint64_t* __restrict__ o_seg,
-                          const uint64_t* __restrict__ o_long, uint64_t* __restrict__ items,
-                          uint32_t* __restrict__ long_reads, uint64_t* __restrict__ item0) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t L = lens[i];
-  const uint32_t nseg = gs::n_segments(L, k, seg_tasks);
-  if (!read_is_long(L, k, nseg)) {
-    const uint64_t p = o_whole[i];
-    items[p] = i;
-    items[p + 1] = i | (1ull << 32);
-    return;
+__global__ void __launch_bounds__(kScanBlock) plan_totals(PlanParams P) {
+  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
+  uint64_t s[kPlanSums] = {0, 0, 0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < kScanItems; ++j) {
+    uint32_t L, c[kPlanSums];
+    plan_counts(P, base + j, L, c);
+#pragma unroll
+    for (int q = 0; q < kPlanSums; ++q) s[q] += c[q];
   }
-  const uint64_t j = o_long[i], first = o_whole[n] + o_seg[i];
-  long_reads[j] = i;
-  item0[j] = first;
-  for (uint64_t g = 0; g < nseg; ++g) {
-    items[first + 2 * g] = i | (g << 33);
-    items[first + 2 * g + 1] = i | (1ull << 32) | (g << 33);
+#pragma unroll
+  for (int q = 0; q < kPlanSums; ++q) {
+    uint64_t tot;
+    block_excl_scan(s[q], &tot);
+    if (threadIdx.x == 0) P.tiles[q * P.ntiles + blockIdx.x] = tot;
+  }
+}
+
+__global__ void __launch_bounds__(kScanBlock) plan_apply(PlanParams P) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
+  uint64_t s[kPlanSums] = {0, 0, 0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < kScanItems; ++j) {
+    uint32_t L, c[kPlanSums];
+    plan_counts(P, base + j, L, c);
+#pragma unroll
+    for (int q = 0; q < kPlanSums; ++q) s[q] += c[q];
+  }
+#pragma unroll
+  for (int q = 0; q < kPlanSums; ++q) {
+    uint64_t tot;
+    s[q] = block_excl_scan(s[q], &tot) + (P.ntiles == 1 ? 0 : P.tiles[q * P.ntiles + blockIdx.x]);
+  }
+  for (int j = 0; j < kScanItems; ++j) {
+    const uint64_t i = base + j;
+    uint32_t L, c[kPlanSums];
+    const bool lng = plan_counts(P, i, L, c);
+    const uint64_t first = P.n_whole + s[3];
+    if (i < P.n) {
+      P.toff[i] = s[0];
+      P.offs[i] -= P.lo;
+      if (i + 1 == P.n) P.toff[P.n] = s[0] + c[0];
+      if (P.code_off) {
+        P.code_off[i] = s[1];
+        if (i + 1 == P.n) P.code_off[P.n] = s[1] + c[1];
+      }
+      if (P.batch) {
+        uint32_t id = 0;  // reference batches that start at or before read i
+        if (P.cuts) {
+          uint32_t hi = P.n_cuts;
+          while (id < hi) {
+            const uint32_t mid = (id + hi) >> 1;
+            if (P.cuts[mid] <= i)
+              id = mid + 1;
+            else
+              hi = mid;
+          }
+        } else {
+          for (uint32_t q = 0; q < kInlineCuts; ++q) id += q < P.n_cuts && P.cut[q] <= i ? 1u : 0u;
+        }
+        P.batch[i] = id;
+      }
+      if (P.items) {
+        if (!lng) {
+          P.items[s[2]] = i;
+          P.items[s[2] + 1] = i | (1ull << 32);
+        } else {
+          P.long_reads[s[4]] = (uint32_t)i;
+          P.item0[s[4]] = first;
+        }
+      }
+    }
+    // a long read's items by the whole wave
+    for (uint64_t m = __ballot(lng && P.items); m; m &= m - 1) {
+      const int from = __ffsll((unsigned long long)m) - 1;
+      const uint64_t ri = __shfl((uint64_t)i, from), at = __shfl(first, from);
+      const uint32_t ni = __shfl(c[3], from);
+      for (uint32_t g = lane; g < ni; g += 64)
+        P.items[at + g] = ri | ((uint64_t)(g & 1u) << 32) | ((uint64_t)(g >> 1) << 33);
+    }
+#pragma unroll
+    for (int q = 0; q < kPlanSums; ++q) s[q] += c[q];
   }
 }
 
@@ -858,14 +983,30 @@ struct DevBuf {
   }
 };
 
-int scan_counts(const uint32_t* in, uint64_t n, uint64_t* out, uint64_t* tiles, uint64_t* total,
-                hipStream_t st) {
-  const uint64_t ntiles = (n + kScanTile - 1) / kScanTile;
-  if (ntiles == 0) return GS_OK;
-  hipLaunchKernelGGL(scan_tile_totals, dim3((unsigned)ntiles), dim3(kScanBlock), 0, st, in, n, tiles);
-  hipLaunchKernelGGL(scan_tiles, dim3(1), dim3(kScanBlock), 0, st, tiles, ntiles, total);
-  hipLaunchKernelGGL(scan_apply, dim3((unsigned)ntiles), dim3(kScanBlock), 0, st, in, n, tiles, out);
-  return GS_OK;
+inline uint64_t scan_ntiles(uint64_t n) { return (n + kScanTile - 1) / kScanTile; }
+
+// bytes of the tile totals of either scan over n reads
+inline uint64_t scan_tile_bytes(uint64_t n) { return 8 * kPlanSums * (scan_ntiles(n) + 1); }
+
+void launch_pair_scan(PairScan S, hipStream_t st) {
+  S.ntiles = scan_ntiles(S.n);
+  if (!S.ntiles) return;
+  if (S.ntiles > 1) {
+    hipLaunchKernelGGL(pair_totals, dim3((unsigned)S.ntiles), dim3(kScanBlock), 0, st, S);
+    hipLaunchKernelGGL(scan_tiles<2>, dim3(1), dim3(kScanBlock), 0, st, S.tiles, S.ntiles, S.total);
+  }
+  hipLaunchKernelGGL(pair_apply, dim3((unsigned)S.ntiles), dim3(kScanBlock), 0, st, S);
+}
+
+void launch_plan(PlanParams P, hipStream_t st) {
+  P.ntiles = scan_ntiles(P.n);
+  if (!P.ntiles) return;
+  if (P.ntiles > 1) {
+    hipLaunchKernelGGL(plan_totals, dim3((unsigned)P.ntiles), dim3(kScanBlock), 0, st, P);
+    hipLaunchKernelGGL(scan_tiles<kPlanSums>, dim3(1), dim3(kScanBlock), 0, st, P.tiles, P.ntiles,
+                       (uint64_t*)nullptr);
+  }
+  hipLaunchKernelGGL(plan_apply, dim3((unsigned)P.ntiles), dim3(kScanBlock), 0, st, P);
 }
 
 template <typename AT, int LMAX>
@@ -891,7 +1032,7 @@ struct gs_batch {
   uint32_t maxlen = 0;
   DevBuf bases, offs, lens, toff, batch, cand, nF, nR, ns, np, soff, poff, tiles, tot, seeds, rows, scratch;
   DevBuf codes, code_off, queue, counters;  // persistent kernel
-  DevBuf items, seg_meta, long_reads, item0, item_tmp;  // item_tmp: counts and scans of the item plan
+  DevBuf items, seg_meta, long_reads, item0, cuts;
   DevBuf seg_link, dyn_items, dyn_meta, dyn_link, wmeta, wlink;  // work splitting
   uint64_t code_chunks = 0, n_items = 0;
   uint32_t n_long = 0, seg_tasks = 64, dyn_cap = 0;
@@ -994,74 +1135,67 @@ void gs::plan_reset(BatchPlan& P, const gs_opts& o) {
   P.seg_tasks = o.seg_tasks ? o.seg_tasks : 64u;
 }
 
-// room for `add` more elements, growing geometrically so that many small
-// additions (a server round's chunks) stay linear
-template <typename V>
-static void grow(V& v, size_t add) {
-  const size_t need = v.size() + add;
-  if (need > v.capacity()) v.reserve(std::max(need, 2 * v.capacity()));
-}
-
+// Everything that a batch's sizes need, in one pass over the lengths; what
+// else follows from them is computed on the device (launch_plan).
 int gs::plan_add(BatchPlan& P, const char* bases, const uint64_t* offsets, const uint32_t* lens, uint64_t r0,
                  uint64_t r1) {
   if (r1 <= r0) return GS_OK;
-  const size_t nr = (size_t)(r1 - r0);
-  grow(P.offs, nr);
-  grow(P.lens, nr);
-  grow(P.task_off, nr + 1);
-  grow(P.rbatch, nr);
-  grow(P.code_off, nr + 1);
+  if (P.n_reads + (r1 - r0) > 0xFFFFFFFFull / 2) return GS_ERANGE;
   const uint32_t k = (uint32_t)P.opts.k;
   const uint32_t batch_bases = P.opts.batch_bases ? P.opts.batch_bases : 1000000u;
-  uint64_t lo = UINT64_MAX, hi = 0;
-  for (uint64_t i = r0; i < r1; ++i) {
-    if (offsets[i] < lo) lo = offsets[i];
-    if (offsets[i] + lens[i] > hi) hi = offsets[i] + lens[i];
-  }
-  if (hi < lo) lo = hi = 0;
-  if (P.n_reads + (r1 - r0) > 0xFFFFFFFFull / 2) return GS_ERANGE;
-  const uint64_t base = P.span;
-  if (hi > lo) P.pieces.push_back({bases + lo, hi - lo});
-  P.span += hi - lo;
-  uint64_t acc = 0;
-  uint32_t bid = P.next_batch_id;
+  // a group starts a reference batch of its own
+  if (P.n_reads) P.cuts.push_back((uint32_t)P.n_reads);
+  uint64_t lo = UINT64_MAX, hi = 0, acc = 0, tasks = 0, chunks = 0, whole = 0, items = 0, n_long = 0;
+  bool closed = false;  // the read before this one closed its reference batch
   for (uint64_t i = r0; i < r1; ++i) {
     const uint32_t L = lens[i];
-    P.offs.push_back(offsets[i] - lo + base);
-    P.lens.push_back(L);
-    P.task_off.push_back(P.tasks);
-    P.tasks += L >= k ? L - k + 1 : 0;
-    P.rbatch.push_back(bid);
+    if (closed) P.cuts.push_back((uint32_t)(P.n_reads + (i - r0)));
     acc += L;
-    if (acc >= batch_bases) {  // a batch closes after the read that reaches the limit (2955-2991)
-      ++bid;
-      acc = 0;
-    }
-    ++P.n_reads;
-    P.code_off.push_back(P.code_chunks);
-    P.code_chunks += 2 * ((L + 31) / 32);
+    closed = acc >= batch_bases;  // a batch closes after the read that reaches the limit (2955-2991)
+    if (closed) acc = 0;
+    lo = std::min(lo, offsets[i]);
+    hi = std::max(hi, offsets[i] + L);
+    tasks += L >= k ? L - k + 1 : 0;
+    chunks += 2 * (uint64_t)((L + 31ull) / 32);
     const uint32_t nseg = gs::n_segments(L, k, P.seg_tasks);
-    if (nseg > 1 || (L > gs::kPersistLmax && L >= k)) ++P.n_long;
-    P.n_items += 2ull * nseg;
+    if (read_is_long(L, k, nseg)) {
+      ++n_long;
+      items += 2ull * nseg;
+    } else {
+      whole += 2ull * nseg;
+    }
   }
-  P.next_batch_id = bid + 1;  // the next group starts a batch of its own
-  if (P.n_items > 0xF0000000ull) return GS_ERANGE;
-  return GS_OK;
+  if (hi < lo) lo = hi = 0;
+  if (hi > lo) P.pieces.push_back({bases + lo, hi - lo});
+  P.groups.push_back({offsets + r0, lens + r0, r1 - r0, lo, P.span});
+  P.span += hi - lo;
+  P.n_reads += r1 - r0;
+  P.tasks += tasks;
+  P.code_chunks += chunks;
+  P.n_whole += whole;
+  P.n_items += whole + items;
+  P.n_long += n_long;
+  return P.n_items > 0xF0000000ull ? GS_ERANGE : GS_OK;
 }
 
-// Closes the per-read offset arrays; the work items (whole-read streams
-// first, then the segments of long reads, so that the last items a
-// persistent kernel hands out are small) are written on the device by
-// batch_load.
-void gs::plan_finish(BatchPlan& P) {
-  P.task_off.push_back(P.tasks);
-  P.code_off.push_back(P.code_chunks);
+// The reads' offsets and lengths as they are uploaded: the caller's own
+// arrays where there is one group of reads and the plan need not outlive the
+// call (copy false), else copies, their offsets rebased onto the groups'
+// bytes, one after another.
+void gs::plan_finish(BatchPlan& P, bool copy) {
+  if (P.groups.size() < 2 && !copy) return;
+  P.offs.reserve(P.n_reads);
+  P.lens.reserve(P.n_reads);
+  for (const auto& g : P.groups) {
+    for (uint64_t i = 0; i < g.n; ++i) P.offs.push_back(g.offs[i] - g.lo + g.base);
+    P.lens.insert(P.lens.end(), g.lens, g.lens + g.n);
+  }
 }
 
 uint64_t gs::plan_device_bytes(const BatchPlan& P) {
   const uint64_t nr1 = P.n_reads + 1;
   return (P.span + 32) + 16 * (P.code_chunks + 1) + 16 * (2 * P.tasks + 1) + 8 * P.n_items +
-         (P.n_long ? 16 * P.n_items : 0) + 12 * P.n_long + nr1 * (8 * 5 + 4 * 7 + 36);
+         (P.n_long ? 16 * P.n_items : 0) + 12 * P.n_long + nr1 * (8 * 5 + 4 * 7);
 }
 
 static int batch_events(gs_batch* B) {
@@ -1082,12 +1216,11 @@ static int ensure_buffers(gs_batch* B, uint64_t span, uint64_t n, uint64_t tasks
   const uint64_t nr1 = n + 1;
   if (B->codes.ensure(16 * (code_chunks + 1)) || B->code_off.ensure(8 * nr1) ||
       B->items.ensure(8 * (n_items + 1)) || B->long_reads.ensure(4 * (n_long + 1)) ||
-      B->item_tmp.ensure(36 * nr1 + 8) ||
       B->item0.ensure(8 * (n_long + 1)) || B->seg_meta.ensure(n_long ? 16 * n_items : 16) ||
       B->bases.ensure(span + 32) || B->offs.ensure(8 * nr1) || B->lens.ensure(4 * nr1) ||
       B->toff.ensure(8 * nr1) || B->batch.ensure(4 * nr1) || B->cand.ensure(16 * (2 * tasks + 1)) ||
       B->nF.ensure(4 * nr1) || B->nR.ensure(4 * nr1) || B->ns.ensure(4 * nr1) || B->np.ensure(4 * nr1) ||
-      B->soff.ensure(8 * nr1) || B->poff.ensure(8 * nr1) || B->tiles.ensure(8 * (nr1 / kScanTile + 2)) ||
+      B->soff.ensure(8 * nr1) || B->poff.ensure(8 * nr1) || B->tiles.ensure(scan_tile_bytes(n)) ||
       B->tot.ensure(16) || B->queue.ensure(16) || B->counters.ensure(gs::kCounterBytes + gs::kColdBytes) ||
       B->seg_link.ensure(n_long ? 4 * n_items : 16) ||
       (dyn_cap &&
@@ -1182,23 +1315,20 @@ static int staged_upload(gs_batch* B, char* dst, const std::vector<std::pair<con
   return GS_OK;
 }
 
-// The work items of B's reads, from their lengths on the device.
-static int enqueue_items(gs_batch* B, hipStream_t st) {
-  const uint64_t n = B->n_reads, nr1 = n + 1;
-  uint32_t* cw = B->item_tmp.as<uint32_t>();
-  uint32_t *cs = cw + nr1, *cl = cw + 2 * nr1;
-  uint64_t* ow = reinterpret_cast<uint64_t*>(B->item_tmp.as<uint8_t>() + ((12 * nr1 + 7) & ~7ull));
-  uint64_t *os = ow + nr1, *ol = ow + 2 * nr1;
-  const uint32_t k = (uint32_t)B->opts.k;
-  hipLaunchKernelGGL(item_counts, dim3(grid_for(n, 256)), dim3(256), 0, st, B->lens.as<uint32_t>(), (uint32_t)n, k,
-                     B->seg_tasks, cw, cs, cl);
-  scan_counts(cw, n, ow, B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
-  scan_counts(cs, n, os, B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
-  scan_counts(cl, n, ol, B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
-  hipLaunchKernelGGL(item_fill, dim3(grid_for(n, 256)), dim3(256), 0, st, B->lens.as<uint32_t>(), (uint32_t)n, k,
-                     B->seg_tasks, ow, os, ol, B->items.as<uint64_t>(), B->long_reads.as<uint32_t>(),
-                     B->item0.as<uint64_t>());
-  return hipGetLastError() == hipSuccess ? GS_OK : GS_EHIP;
+// B's part of a plan on the device (PP: lo, n_whole and the reference batches)
+static void enqueue_plan(gs_batch* B, PlanParams PP, hipStream_t st) {
+  PP.offs = B->offs.as<uint64_t>();
+  PP.lens = B->lens.as<uint32_t>();
+  PP.n = B->n_reads;
+  PP.k = (uint32_t)B->opts.k;
+  PP.seg_tasks = B->seg_tasks;
+  PP.toff = B->toff.as<uint64_t>();
+  PP.code_off = B->streams ? nullptr : B->code_off.as<uint64_t>();
+  PP.items = B->streams ? nullptr : B->items.as<uint64_t>();
+  PP.long_reads = B->long_reads.as<uint32_t>();
+  PP.item0 = B->item0.as<uint64_t>();
+  PP.tiles = B->tiles.as<uint64_t>();
+  launch_plan(PP, st);
 }
 
 // Uploads a finished plan into B, reusing B's device buffers where they are
@@ -1219,7 +1349,7 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P) {
   B->seg_tasks = P.seg_tasks;
   B->n_seeds = B->n_pos = 0;
   B->ran = false;
-  const uint64_t n = P.n_reads, nr1 = n + 1;
+  const uint64_t n = P.n_reads;
   const bool split_on = P.opts.split_tasks != 0xFFFF;
   B->dyn_cap = split_on ? gs::piece_cap(B->n_items) : 0u;
   if (ensure_buffers(B, B->span, n, B->tasks, B->code_chunks, B->n_items, B->n_long, B->dyn_cap))
@@ -1228,14 +1358,31 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P) {
   if (hipEventRecord(B->ev[0], st) != hipSuccess) return GS_EHIP;
   if ((rc = staged_upload(B, B->bases.as<char>(), P.pieces, P.span))) return rc;
   hipLaunchKernelGGL(zero_bytes, dim3(1), dim3(32), 0, st, B->bases.as<uint8_t>() + B->span, 32u);
-  if (n &&
-      (hipMemcpyAsync(B->offs.p, P.offs.data(), 8 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
-       hipMemcpyAsync(B->lens.p, P.lens.data(), 4 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
-       hipMemcpyAsync(B->toff.p, P.task_off.data(), 8 * nr1, hipMemcpyHostToDevice, st) != hipSuccess ||
-       hipMemcpyAsync(B->batch.p, P.rbatch.data(), 4 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
-       hipMemcpyAsync(B->code_off.p, P.code_off.data(), 8 * nr1, hipMemcpyHostToDevice, st) != hipSuccess))
-    return GS_EHIP;
-  if (n && (rc = enqueue_items(B, st))) return rc;
+  if (n) {
+    const bool one = P.offs.empty();
+    const uint64_t* offs = one ? P.groups[0].offs : P.offs.data();
+    const uint32_t* lens = one ? P.groups[0].lens : P.lens.data();
+    PlanParams PP{};
+    PP.lo = one ? P.groups[0].lo : 0;
+    PP.n_whole = P.n_whole;
+    if (!P.opts.smem) {  // only MEM's row skip looks at the reference batches
+      PP.batch = B->batch.as<uint32_t>();
+      PP.n_cuts = (uint32_t)P.cuts.size();
+      if (PP.n_cuts <= kInlineCuts) {
+        std::copy(P.cuts.begin(), P.cuts.end(), PP.cut);
+      } else {
+        if (B->cuts.ensure(4 * P.cuts.size())) return GS_ENOMEM;
+        PP.cuts = B->cuts.as<uint32_t>();
+        if (hipMemcpyAsync(B->cuts.p, P.cuts.data(), 4 * P.cuts.size(), hipMemcpyHostToDevice, st) != hipSuccess)
+          return GS_EHIP;
+      }
+    }
+    if (hipMemcpyAsync(B->offs.p, offs, 8 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
+        hipMemcpyAsync(B->lens.p, lens, 4 * n, hipMemcpyHostToDevice, st) != hipSuccess)
+      return GS_EHIP;
+    enqueue_plan(B, PP, st);
+    if (hipGetLastError() != hipSuccess) return GS_EHIP;
+  }
   if (hipEventRecord(B->ev[1], st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return GS_EHIP;
   float ms = 0;
   (void)hipEventElapsedTime(&ms, B->ev[0], B->ev[1]);
@@ -1402,8 +1549,8 @@ static int enqueue_counts(gs_batch* B, const PostParams& Q, hipStream_t st) {
   if (n) {
     hipLaunchKernelGGL(finalize_reads<false>, dim3(grid_for(n, 256)), dim3(256), 0, st, Q);
     if (Q.n_long) hipLaunchKernelGGL(finalize_long<false>, dim3((Q.n_long + 3) / 4), dim3(256), 0, st, Q);
-    scan_counts(Q.nseeds, n, B->soff.as<uint64_t>(), B->tiles.as<uint64_t>(), B->tot.as<uint64_t>(), st);
-    scan_counts(Q.npos, n, B->poff.as<uint64_t>(), B->tiles.as<uint64_t>(), B->tot.as<uint64_t>() + 1, st);
+    launch_pair_scan({{Q.nseeds, Q.npos}, {B->soff.as<uint64_t>(), B->poff.as<uint64_t>()}, n, 0,
+                      B->tiles.as<uint64_t>(), B->tot.as<uint64_t>()}, st);
     GS_HIP(hipMemcpyAsync(B->h_tot, B->tot.p, 16, hipMemcpyDeviceToHost, st));
   } else {  // no reads: the offset arrays still hold their closing 0
     hipLaunchKernelGGL(zero_bytes, dim3(1), dim3(32), 0, st, B->soff.as<uint8_t>(), 8u);
@@ -1880,24 +2027,6 @@ std::mutex g_scratch_mu;
 void* g_scratch_ptr[kNoAllocDevices];  // device address of `scratch` on each device (null: not looked up)
 int g_scratch_rc[kNoAllocDevices];     // the lookup's result once it has run
 
-// Per read: the offset rebased onto the uploaded span, the task and code
-// chunk counts that the scans turn into offsets, and the two work items of a
-// whole-read stream (items may be null: plain kernel).
-__global__ void noalloc_prepare(uint64_t* __restrict__ offs, const uint32_t* __restrict__ lens, uint32_t n,
-                                uint64_t lo, uint32_t k, uint32_t* __restrict__ ntask,
-                                uint32_t* __restrict__ ncode, uint64_t* __restrict__ items) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t L = lens[i];
-  offs[i] -= lo;
-  ntask[i] = L >= k ? L - k + 1 : 0u;
-  ncode[i] = 2u * ((L + 31u) / 32u);
-  if (items) {
-    items[2ull * i] = i;
-    items[2ull * i + 1] = i | (1ull << 32);
-  }
-}
-
 // Reference-batch id of every read: a batch closes after the read that
 // brings it to batch_bases (seed_gen.cu:2955-2991), a running count with a
 // reset.  One wave: the lanes load 64 lengths at a time and every lane
@@ -1958,16 +2087,28 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   const uint32_t n = (uint32_t)n_reads, k = (uint32_t)opts->k;
   const uint32_t seg_tasks = opts->seg_tasks ? opts->seg_tasks : 64u;
   // sizes from the lengths alone (one pass, nothing allocated)
-  uint64_t lo = UINT64_MAX, hi = 0, tasks = 0, chunks = 0, n_items = 0, n_long = 0;
-  uint32_t maxlen = 0;
+  const uint32_t batch_bases = opts->batch_bases ? opts->batch_bases : 1000000u;
+  uint64_t lo = UINT64_MAX, hi = 0, tasks = 0, chunks = 0, n_items = 0, n_whole = 0, n_long = 0, acc = 0;
+  uint32_t maxlen = 0, n_cuts = 0, cut[kInlineCuts];
+  bool closed = false;  // the read before this one closed its reference batch
   for (uint32_t i = 0; i < n; ++i) {
     const uint32_t L = lens[i];
+    if (closed && n_cuts <= kInlineCuts) {
+      if (n_cuts < kInlineCuts) cut[n_cuts] = i;
+      ++n_cuts;
+    }
+    acc += L;
+    closed = acc >= batch_bases;
+    if (closed) acc = 0;
     if (offsets[i] < lo) lo = offsets[i];
     if (offsets[i] + L > hi) hi = offsets[i] + L;
     tasks += L >= k ? L - k + 1 : 0;
     chunks += 2 * ((L + 31) / 32);
     const uint32_t nseg = gs::n_segments(L, k, seg_tasks);
-    if (read_is_long(L, k, nseg)) ++n_long;
+    if (read_is_long(L, k, nseg))
+      ++n_long;
+    else
+      n_whole += 2ull * nseg;
     n_items += 2ull * nseg;
     if (L > maxlen) maxlen = L;
   }
@@ -1990,8 +2131,9 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   const uint64_t o_bases = take(span + 32), o_offs = take(8 * nr1), o_lens = take(4 * nr1),
                  o_toff = take(8 * nr1), o_batch = take(4 * nr1), o_cand = take(16 * (2 * tasks + 1)),
                  o_nF = take(4 * nr1), o_nR = take(4 * nr1), o_ns = take(4 * nr1), o_np = take(4 * nr1),
-                 o_soff = take(8 * nr1), o_poff = take(8 * nr1), o_tiles = take(8 * (nr1 / kScanTile + 2)),
+                 o_soff = take(8 * nr1), o_poff = take(8 * nr1), o_spare = take(8 * (nr1 / kScanTile + 2)),
                  o_tot = take(16), o_queue = take(16), o_counters = take(gs::kCounterBytes + gs::kColdBytes);
+  (void)o_spare;
   const uint64_t common = at;
   const uint64_t o_code_off = take(8 * nr1), o_long = long_scratch ? take(4 * (span + 16)) : 0;
   if (short_batched) {
@@ -2011,8 +2153,7 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   const uint64_t o_code_off2 = take(8 * nr1);
   const bool kernel_codes = opts->kernel != 0;
   const uint64_t o_items = take(8 * (n_items + 1)), o_codes = kernel_codes ? take(16 * (chunks + 1)) : 0,
-                 o_item_tmp = n_long ? take(36 * nr1 + 8) : 0,
-                 o_item0 = take(8 * (n_long + 1)), o_seg_meta = n_long ? take(16 * n_items) : 0;
+                 o_tiles2 = take(scan_tile_bytes(n)), o_item0 = take(8 * (n_long + 1)), o_seg_meta = n_long ? take(16 * n_items) : 0;
   const bool streams = at > kNoAllocBytes;
   const uint32_t cap = streams || opts->split_tasks == 0xFFFF ? 0u : gs::piece_cap(n_items);
   const uint64_t o_ditems = take(16ull * cap), o_dmeta = take(16ull * cap), o_dlink = take(4ull * cap),
@@ -2051,10 +2192,7 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
     if (kernel_codes) B.codes.view(base + o_codes, 16 * (chunks + 1));
     B.long_reads.view(base + o_long_reads, 4 * (n_long + 1));
     B.item0.view(base + o_item0, 8 * (n_long + 1));
-    if (n_long) {
-      B.item_tmp.view(base + o_item_tmp, 36 * nr1 + 8);
-      B.seg_meta.view(base + o_seg_meta, 16 * n_items);
-    }
+    if (n_long) B.seg_meta.view(base + o_seg_meta, 16 * n_items);
   }
   if (split_on) {
     B.dyn_items.view(base + o_ditems, 16ull * cap);
@@ -2079,7 +2217,9 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   B.np.view(base + o_np, 4 * nr1);
   B.soff.view(base + o_soff, 8 * nr1);
   B.poff.view(base + o_poff, 8 * nr1);
-  B.tiles.view(base + o_tiles, 8 * (nr1 / kScanTile + 2));
+  // the scans' tile totals: with seed_streams in place of the code offsets it
+  // does not read (40 bytes per 2048 reads, 8 per read)
+  B.tiles.view(base + (streams ? o_code_off : o_tiles2), scan_tile_bytes(n));
   B.tot.view(base + o_tot, 16);
   B.queue.view(base + o_queue, 16);
   B.counters.view(base + o_counters, gs::kCounterBytes + gs::kColdBytes);
@@ -2092,15 +2232,20 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
     return GS_EHIP;
   hipLaunchKernelGGL(zero_bytes, dim3(1), dim3(32), 0, st, B.bases.as<uint8_t>() + span, 32u);
   if (n) {
-    hipLaunchKernelGGL(noalloc_prepare, dim3(grid_for(n, 256)), dim3(256), 0, st, B.offs.as<uint64_t>(),
-                       B.lens.as<uint32_t>(), n, lo, k, B.ns.as<uint32_t>(), B.np.as<uint32_t>(),
-                       streams || n_long ? (uint64_t*)nullptr : B.items.as<uint64_t>());
-    scan_counts(B.ns.as<uint32_t>(), n, B.toff.as<uint64_t>(), B.tiles.as<uint64_t>(), B.tot.as<uint64_t>(), st);
-    scan_counts(B.np.as<uint32_t>(), n, B.code_off.as<uint64_t>(), B.tiles.as<uint64_t>(),
-                B.tot.as<uint64_t>() + 1, st);
-    hipLaunchKernelGGL(noalloc_batch_ids, dim3(1), dim3(64), 0, st, B.lens.as<uint32_t>(), n,
-                       opts->batch_bases ? opts->batch_bases : 1000000u, B.batch.as<uint32_t>());
-    if (n_long && !streams && (rc = enqueue_items(&B, st))) return rc;
+    PlanParams PP{};
+    PP.lo = lo;
+    PP.n_whole = n_whole;
+    if (!opts->smem) {
+      if (n_cuts <= kInlineCuts) {
+        PP.batch = B.batch.as<uint32_t>();
+        PP.n_cuts = n_cuts;
+        std::copy(cut, cut + n_cuts, PP.cut);
+      } else {  // no room for the list: a running count on the device
+        hipLaunchKernelGGL(noalloc_batch_ids, dim3(1), dim3(64), 0, st, B.lens.as<uint32_t>(), n, batch_bases,
+                           B.batch.as<uint32_t>());
+      }
+    }
+    enqueue_plan(&B, PP, st);
   }
   if (hipGetLastError() != hipSuccess) return GS_EHIP;
 

@@ -218,7 +218,7 @@ void build_round(gs_server* S, Round& R) {
       return;
     }
   }
-  gs::plan_finish(R.plan);
+  gs::plan_finish(R.plan, true);
   R.device_bytes = gs::plan_device_bytes(R.plan);
 }
 

@@ -31,6 +31,7 @@
 //    every later task would end there too and be filtered out.
 #include <stdlib.h>
 #include <string.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <mutex>
@@ -1009,6 +1010,75 @@ void launch_plan(PlanParams P, hipStream_t st) {
   hipLaunchKernelGGL(plan_apply, dim3((unsigned)P.ntiles), dim3(kScanBlock), 0, st, P);
 }
 
+// Arrays on their way to pinned host memory: copied by one launch, 16 bytes
+// per lane, at the link's rate where they are large.  A copy (and, to pageable
+// memory, a wait) for each of six arrays cost small calls more than their
+// bytes: 64 reads 484 -> 394 us per call, 100,000 plain 5.1 -> 4.45 ms.  Sources are read up to the next 16 bytes
+// (every device buffer and slice here has that room behind it).
+struct GatherParams {
+  struct Segment {
+    uint4* dst;
+    const uint4* src;
+    uint64_t end;  // 16-byte units up to this segment's last
+  } seg[6];
+  int n;
+};
+
+__global__ void __launch_bounds__(256) gather_arrays(GatherParams G) {
+  const uint64_t units = G.seg[G.n - 1].end, step = gridDim.x * 256ull;
+  for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < units; i += step) {
+    uint64_t first = 0;
+    for (int q = 0; q < G.n; ++q) {
+      if (i < G.seg[q].end) {
+        G.seg[q].dst[i - first] = G.seg[q].src[i - first];
+        break;
+      }
+      first = G.seg[q].end;
+    }
+  }
+}
+
+// Result arrays on their way to the caller's memory, laid end to end on 256
+// byte boundaries.
+struct FetchParts {
+  struct Part {
+    void* dst;
+    const void* src;
+    size_t bytes, at;
+  } part[6];
+  int n = 0;
+  size_t total = 0;
+  void add(void* dst, const void* src, size_t bytes) {
+    if (!bytes) return;
+    part[n++] = {dst, src, bytes, total};
+    total += (bytes + 255) & ~(size_t)255;
+  }
+  // f(part, offset in it, bytes, offset in all) for what lies in [a, z)
+  template <typename F>
+  void each(size_t a, size_t z, F&& f) const {
+    for (int i = 0; i < n; ++i) {
+      const Part& p = part[i];
+      const size_t b = std::max(a, p.at), e = std::min(z, p.at + p.bytes);
+      if (b < e) f(p, b - p.at, e - b, b);
+    }
+  }
+  // what lies in [a, z), a multiple of 256, to `stage` with one launch
+  int launch_gather(size_t a, size_t z, char* stage, hipStream_t st) const {
+    GatherParams G;
+    G.n = 0;
+    uint64_t units = 0;
+    each(a, z, [&](const Part& p, size_t o, size_t len, size_t at) {
+      units += (len + 15) / 16;
+      G.seg[G.n++] = {reinterpret_cast<uint4*>(stage + (at - a)),
+                      reinterpret_cast<const uint4*>(static_cast<const char*>(p.src) + o), units};
+    });
+    if (!units) return GS_OK;
+    const unsigned grid = (unsigned)std::min<uint64_t>((units + 255) / 256, 2048);
+    hipLaunchKernelGGL(gather_arrays, dim3(grid), dim3(256), 0, st, G);
+    return hipGetLastError() == hipSuccess ? GS_OK : GS_EHIP;
+  }
+};
+
 template <typename AT, int LMAX>
 void launch_seed(const SeedParams& P, hipStream_t st) {
   const uint64_t lanes = 2ull * P.n_reads;
@@ -1085,9 +1155,24 @@ struct gs_batch {
 static void free_graph(gs_batch* B);
 static void free_host_results(gs_batch* B);
 
-void* gs::result_alloc(size_t bytes) { return malloc(bytes); }
+// Arrays of 4 MB and more on huge pages: the 4 KB page faults of a new array
+// of that size cost more than filling it (107 MB of results, copied by one
+// thread: 28 ms after a replay whose device work takes 11.6 ms).
+void* gs::result_alloc(size_t bytes) {
+  constexpr size_t kHuge = 2u << 20;
+  if (bytes < 2 * kHuge) return malloc(bytes);
+  const size_t whole = (bytes + kHuge - 1) & ~(kHuge - 1);
+  void* p = aligned_alloc(kHuge, whole);
+  if (p) (void)madvise(p, whole, MADV_HUGEPAGE);
+  return p;
+}
 
-constexpr size_t kStageChunk = 64u << 20;  // pinned chunks of staged uploads and downloads
+// Pinned chunks of staged uploads and downloads: two of them, the DMA of one
+// under the host's copy of the other, so at least four chunks in a large copy.
+constexpr size_t kStageChunk = 64u << 20, kStageChunkMin = 8u << 20;
+static size_t stage_chunk(size_t total) {
+  return std::min(total, std::max(kStageChunkMin, std::min(kStageChunk, (total / 4 + 4095) & ~(size_t)4095)));
+}
 
 static void destroy_batch(gs_batch* B) {
   if (!B) return;
@@ -1240,7 +1325,7 @@ int gs::batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_
   const uint32_t dyn = gs::piece_cap(items);
   int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, dyn);
   if (!rc && bases > (4u << 20)) {  // the pinned chunks of staged uploads
-    const size_t ch = std::min<uint64_t>(bases, kStageChunk);
+    const size_t ch = stage_chunk(bases);
     if (B->st_a.ensure(ch) || B->st_b.ensure(ch)) rc = GS_ENOMEM;
   }
   return rc;
@@ -1275,7 +1360,6 @@ static void parallel_parts(size_t len, F&& part) {
 // own staging, one thread at a fraction of the link's rate.
 static int staged_upload(gs_batch* B, char* dst, const std::vector<std::pair<const char*, uint64_t>>& pieces,
                          uint64_t total) {
-  constexpr size_t kChunk = kStageChunk;
   hipStream_t st = B->stream;
   if (total <= (4u << 20)) {  // small: the pieces directly
     uint64_t at = 0;
@@ -1285,7 +1369,7 @@ static int staged_upload(gs_batch* B, char* dst, const std::vector<std::pair<con
     }
     return GS_OK;
   }
-  const size_t ch = std::min<uint64_t>(total, kChunk);
+  const size_t ch = stage_chunk(total);
   if (B->st_a.ensure(ch) || B->st_b.ensure(ch)) return GS_ENOMEM;
   for (auto& e : B->cev)
     if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return GS_EHIP;
@@ -1786,28 +1870,22 @@ extern "C" GS_API int gs_batch_replay(gs_batch* B, gs_batch_stats* stats) {
   return GS_OK;
 }
 
-// Device-to-host copy of `bytes` into pageable memory through two pinned
-// chunks: the DMA of chunk c+1 runs while chunk c is copied out, on several
-// threads when it is large.  Pageable destinations otherwise go through the
-// runtime's own staging at a fraction of the link's rate.
-static int staged_d2h(gs_batch* B, void* dst, const void* src, size_t bytes) {
-  constexpr size_t kChunk = kStageChunk;
+// Device-to-host copy into pageable memory through two pinned chunks: the DMA
+// of chunk c+1 runs while chunk c is copied out, on several threads when it
+// is large.  Pageable destinations otherwise go through the runtime's own
+// staging at a fraction of the link's rate (and one array after another: a
+// call of 1000 reads waited six times).
+static int staged_d2h(gs_batch* B, const FetchParts& P) {
+  if (!P.total) return GS_OK;
   hipStream_t st = B->stream;
-  if (bytes <= (4u << 20))  // small: one plain copy
-    return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st) == hipSuccess &&
-                   hipStreamSynchronize(st) == hipSuccess
-               ? GS_OK
-               : GS_EHIP;
-  const size_t ch = std::min(bytes, kChunk);
-  if (B->st_a.ensure(ch) || B->st_b.ensure(ch)) return GS_ENOMEM;
+  const size_t ch = stage_chunk(P.total), nch = (P.total + ch - 1) / ch;
+  if (B->st_a.ensure(ch) || (nch > 1 && B->st_b.ensure(ch))) return GS_ENOMEM;
   for (auto& e : B->cev)
     if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return GS_EHIP;
   char* stage[2] = {static_cast<char*>(B->st_a.p), static_cast<char*>(B->st_b.p)};
-  const size_t nch = (bytes + ch - 1) / ch;
   auto issue = [&](size_t c) -> bool {
-    const size_t off = c * ch, len = std::min(ch, bytes - off);
-    return hipMemcpyAsync(stage[c & 1], static_cast<const char*>(src) + off, len, hipMemcpyDeviceToHost, st) ==
-               hipSuccess &&
+    const size_t off = c * ch;
+    return P.launch_gather(off, std::min(P.total, off + ch), stage[c & 1], st) == GS_OK &&
            hipEventRecord(B->cev[c & 1], st) == hipSuccess;
   };
   if (!issue(0)) return GS_EHIP;
@@ -1815,24 +1893,13 @@ static int staged_d2h(gs_batch* B, void* dst, const void* src, size_t bytes) {
     // the buffer of chunk c+1 held chunk c-1, already copied out
     if (c + 1 < nch && !issue(c + 1)) return GS_EHIP;
     if (hipEventSynchronize(B->cev[c & 1]) != hipSuccess) return GS_EHIP;
-    const size_t off = c * ch, len = std::min(ch, bytes - off);
-    char* d = static_cast<char*>(dst) + off;
+    const size_t off = c * ch;
     const char* sp = stage[c & 1];
-    constexpr size_t kThreads = 8;
-    const size_t part = (len + kThreads - 1) / kThreads;
-    std::vector<std::thread> th;
-    size_t done = part;  // bytes the helper threads do not cover
-    try {
-      for (size_t t = 1; t < kThreads; ++t) {
-        const size_t a = std::min(len, t * part), z = std::min(len, a + part);
-        th.emplace_back([=] { memcpy(d + a, sp + a, z - a); });
-        done = std::min(len, (t + 1) * part);
-      }
-    } catch (...) {  // no thread to spare: this one copies the rest
-    }
-    memcpy(d, sp, std::min(len, part));
-    if (done < len) memcpy(d + done, sp + done, len - done);
-    for (auto& t : th) t.join();
+    parallel_parts(std::min(ch, P.total - off), [&](size_t a, size_t z) {
+      P.each(off + a, off + z, [&](const FetchParts::Part& p, size_t o, size_t len, size_t at) {
+        memcpy(static_cast<char*>(p.dst) + o, sp + (at - off), len);
+      });
+    });
   }
   return GS_OK;
 }
@@ -1858,28 +1925,35 @@ extern "C" GS_API int gs_batch_fetch(gs_batch* B, gs_result* out) {
     return GS_ENOMEM;
   }
   if (B->graph_fresh) {  // the last replay already downloaded everything
-    memcpy(out->read_nseeds, B->hr_ns, 4 * n);
-    memcpy(out->read_npos, B->hr_np, 4 * n);
+    FetchParts P;
+    P.add(out->read_nseeds, B->hr_ns, 4 * n);
+    P.add(out->read_npos, B->hr_np, 4 * n);
     if (n) {
-      memcpy(out->read_seed_off, B->hr_soff, 8 * nr1);
-      memcpy(out->read_pos_off, B->hr_poff, 8 * nr1);
+      P.add(out->read_seed_off, B->hr_soff, 8 * nr1);
+      P.add(out->read_pos_off, B->hr_poff, 8 * nr1);
     } else {
       out->read_seed_off[0] = out->read_pos_off[0] = 0;
     }
-    memcpy(out->seeds, B->hr_seeds, sizeof(gs_seed_rec) * B->n_seeds);
-    memcpy(out->pos, B->hr_rows, 4 * B->n_pos);
+    P.add(out->seeds, B->hr_seeds, sizeof(gs_seed_rec) * B->n_seeds);
+    P.add(out->pos, B->hr_rows, 4 * B->n_pos);
+    parallel_parts(P.total, [&](size_t a, size_t z) {
+      P.each(a, z, [&](const FetchParts::Part& p, size_t o, size_t len, size_t) {
+        memcpy(static_cast<char*>(p.dst) + o, static_cast<const char*>(p.src) + o, len);
+      });
+    });
     return GS_OK;
   }
   hipEvent_t e0 = B->ev[5], e1 = B->ev[6];
   int rc = GS_OK;
   if (hipEventRecord(e0, st) != hipSuccess) rc = GS_EHIP;
-  // per-read arrays, then seeds and positions, each through the pinned chunks
-  if (!rc && n) rc = staged_d2h(B, out->read_nseeds, B->ns.p, 4 * n);
-  if (!rc && n) rc = staged_d2h(B, out->read_npos, B->np.p, 4 * n);
-  if (!rc) rc = staged_d2h(B, out->read_seed_off, B->soff.p, 8 * nr1);
-  if (!rc) rc = staged_d2h(B, out->read_pos_off, B->poff.p, 8 * nr1);
-  if (!rc && B->n_seeds) rc = staged_d2h(B, out->seeds, B->seeds.p, sizeof(gs_seed_rec) * B->n_seeds);
-  if (!rc && B->n_pos) rc = staged_d2h(B, out->pos, B->rows.p, 4 * B->n_pos);
+  FetchParts P;
+  P.add(out->read_nseeds, B->ns.p, 4 * n);
+  P.add(out->read_npos, B->np.p, 4 * n);
+  P.add(out->read_seed_off, B->soff.p, 8 * nr1);
+  P.add(out->read_pos_off, B->poff.p, 8 * nr1);
+  P.add(out->seeds, B->seeds.p, sizeof(gs_seed_rec) * B->n_seeds);
+  P.add(out->pos, B->rows.p, 4 * B->n_pos);
+  if (!rc) rc = staged_d2h(B, P);
   if (!rc && (hipEventRecord(e1, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess)) rc = GS_EHIP;
   if (rc) {
     gs_result_free(out);
@@ -2023,7 +2097,12 @@ constexpr int kNoAllocDevices = 64;
 
 static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
 
+// Small results of a call leave through pinned memory that is set up with the
+// scratch array (larger ones go straight to the caller's arrays).
+constexpr size_t kNoAllocStage = 1u << 20;
+
 std::mutex g_scratch_mu;
+char* g_scratch_stage[kNoAllocDevices];  // pinned, kNoAllocStage bytes (null: none)
 void* g_scratch_ptr[kNoAllocDevices];  // device address of `scratch` on each device (null: not looked up)
 int g_scratch_rc[kNoAllocDevices];     // the lookup's result once it has run
 
@@ -2070,6 +2149,9 @@ int gs::noalloc_setup(int device) {
     g_scratch_rc[device] = GS_EHIP;
     return GS_EHIP;
   }
+  void* stage = nullptr;
+  if (hipHostMalloc(&stage, kNoAllocStage, hipHostMallocDefault) != hipSuccess) stage = nullptr;
+  g_scratch_stage[device] = static_cast<char*>(stage);
   g_scratch_ptr[device] = p;
   return GS_OK;
 }
@@ -2164,9 +2246,11 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   if (X->device < 0 || X->device >= kNoAllocDevices) return GS_EINVAL;
   if (hipSetDevice(X->device) != hipSuccess) return GS_EHIP;
   uint8_t* base = nullptr;
+  char* stage = nullptr;
   {
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     base = static_cast<uint8_t*>(g_scratch_ptr[X->device]);
+    stage = g_scratch_stage[X->device];
   }
   if (!base) return GS_EHIP;  // the lookup at set-up failed
   hipStream_t st = X->stream;
@@ -2273,14 +2357,23 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   fill_params(&B, S, Q);
   if ((rc = enqueue_write(&B, Q, st))) return rc;
   if ((rc = enqueue_walk(&B, S, Q, st))) return rc;
-  if ((n && (hipMemcpyAsync(out->read_nseeds, B.ns.p, 4ull * n, hipMemcpyDeviceToHost, st) != hipSuccess ||
-             hipMemcpyAsync(out->read_npos, B.np.p, 4ull * n, hipMemcpyDeviceToHost, st) != hipSuccess)) ||
-      hipMemcpyAsync(out->read_seed_off, B.soff.p, 8 * nr1, hipMemcpyDeviceToHost, st) != hipSuccess ||
-      hipMemcpyAsync(out->read_pos_off, B.poff.p, 8 * nr1, hipMemcpyDeviceToHost, st) != hipSuccess ||
-      (n_seeds && hipMemcpyAsync(out->seeds, B.seeds.p, sizeof(gs_seed_rec) * n_seeds, hipMemcpyDeviceToHost,
-                                 st) != hipSuccess) ||
-      (n_pos && hipMemcpyAsync(out->pos, B.rows.p, 4 * n_pos, hipMemcpyDeviceToHost, st) != hipSuccess))
-    return GS_EHIP;
+  FetchParts P;
+  P.add(out->read_nseeds, B.ns.p, 4ull * n);
+  P.add(out->read_npos, B.np.p, 4ull * n);
+  P.add(out->read_seed_off, B.soff.p, 8 * nr1);
+  P.add(out->read_pos_off, B.poff.p, 8 * nr1);
+  P.add(out->seeds, B.seeds.p, sizeof(gs_seed_rec) * n_seeds);
+  P.add(out->pos, B.rows.p, 4 * n_pos);
+  const bool staged = stage && P.total <= kNoAllocStage;
+  if (staged) {
+    if ((rc = P.launch_gather(0, P.total, stage, st))) return rc;
+  } else {
+    for (int i = 0; i < P.n; ++i)
+      if (hipMemcpyAsync(P.part[i].dst, P.part[i].src, P.part[i].bytes, hipMemcpyDeviceToHost, st) != hipSuccess)
+        return GS_EHIP;
+  }
   GS_HIP(hipStreamSynchronize(st));
+  if (staged)
+    for (int i = 0; i < P.n; ++i) memcpy(P.part[i].dst, stage + P.part[i].at, P.part[i].bytes);
   return GS_OK;
 }

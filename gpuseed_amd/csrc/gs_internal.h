@@ -259,7 +259,7 @@ uint64_t plan_device_bytes(const BatchPlan& P);  // device buffers the plan need
 // hold: the batch keeps a reference to X (every batch but gs_seed's own,
 // which the index owns and frees)
 gs_batch* batch_new(gs_index* X, bool hold = true);
-int batch_load(gs_batch* B, const BatchPlan& P);
+int batch_load(gs_batch* B, const BatchPlan& P, bool wait = true);
 // Grows B's device buffers for any plan of at most `bases` bases and `reads`
 // reads, so that loading such plans allocates (and synchronises) nothing.
 int batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_tasks);

@@ -696,7 +696,7 @@ struct PairScan {
   uint64_t* out[2];  // n + 1 entries each
   uint64_t n, ntiles;
   uint64_t* tiles;  // [2][ntiles]
-  uint64_t* total;  // [2]
+  uint64_t* total;  // [2], pinned host memory
 };
 
 // the thread's kScanItems counts from `base` on (sum returned, each in v)
@@ -1010,10 +1010,10 @@ void launch_plan(PlanParams P, hipStream_t st) {
   hipLaunchKernelGGL(plan_apply, dim3((unsigned)P.ntiles), dim3(kScanBlock), 0, st, P);
 }
 
-// Arrays on their way to pinned host memory: copied by one launch, 16 bytes
-// per lane, at the link's rate where they are large.  A copy (and, to pageable
+// Arrays on their way to pinned host memory or back: copied by one launch, 16
+// bytes per lane, at the link's rate where they are large.  A copy (and, to pageable
 // memory, a wait) for each of six arrays cost small calls more than their
-// bytes: 64 reads 484 -> 394 us per call, 100,000 plain 5.1 -> 4.45 ms.  Sources are read up to the next 16 bytes
+// bytes: 64 reads 484 -> 394 us per call, 100,000 plain 5.1 -> 4.45 ms.  Arrays are copied up to the next 16 bytes
 // (every device buffer and slice here has that room behind it).
 struct GatherParams {
   struct Segment {
@@ -1038,8 +1038,8 @@ __global__ void __launch_bounds__(256) gather_arrays(GatherParams G) {
   }
 }
 
-// Result arrays on their way to the caller's memory, laid end to end on 256
-// byte boundaries.
+// Device arrays (src) on their way to the caller's memory, laid end to end on
+// 256 byte boundaries.
 struct FetchParts {
   struct Part {
     void* dst;
@@ -1062,15 +1062,21 @@ struct FetchParts {
       if (b < e) f(p, b - p.at, e - b, b);
     }
   }
-  // what lies in [a, z), a multiple of 256, to `stage` with one launch
-  int launch_gather(size_t a, size_t z, char* stage, hipStream_t st) const {
+  // what lies in [a, z), a a multiple of 256, to `stage` with one launch
+  int launch_gather(size_t a, size_t z, char* stage, hipStream_t st) const { return launch(a, z, stage, false, st); }
+  // the other way: from `stage` to the arrays
+  int launch_scatter(size_t a, size_t z, char* stage, hipStream_t st) const { return launch(a, z, stage, true, st); }
+
+ private:
+  int launch(size_t a, size_t z, char* stage, bool scatter, hipStream_t st) const {
     GatherParams G;
     G.n = 0;
     uint64_t units = 0;
     each(a, z, [&](const Part& p, size_t o, size_t len, size_t at) {
       units += (len + 15) / 16;
-      G.seg[G.n++] = {reinterpret_cast<uint4*>(stage + (at - a)),
-                      reinterpret_cast<const uint4*>(static_cast<const char*>(p.src) + o), units};
+      uint4* const device = reinterpret_cast<uint4*>(static_cast<char*>(const_cast<void*>(p.src)) + o);
+      uint4* const host = reinterpret_cast<uint4*>(stage + (at - a));
+      G.seg[G.n++] = {scatter ? device : host, scatter ? host : device, units};
     });
     if (!units) return GS_OK;
     const unsigned grid = (unsigned)std::min<uint64_t>((units + 255) / 256, 2048);
@@ -1100,7 +1106,7 @@ struct gs_batch {
   // instead of the persistent kernel (which needs maxlen and the read scratch)
   bool streams = false;
   uint32_t maxlen = 0;
-  DevBuf bases, offs, lens, toff, batch, cand, nF, nR, ns, np, soff, poff, tiles, tot, seeds, rows, scratch;
+  DevBuf bases, offs, lens, toff, batch, cand, nF, nR, ns, np, soff, poff, tiles, seeds, rows, scratch;
   DevBuf codes, code_off, queue, counters;  // persistent kernel
   DevBuf items, seg_meta, long_reads, item0, cuts;
   DevBuf seg_link, dyn_items, dyn_meta, dyn_link, wmeta, wlink;  // work splitting
@@ -1108,7 +1114,9 @@ struct gs_batch {
   uint32_t n_long = 0, seg_tasks = 64, dyn_cap = 0;
   uint64_t n_seeds = 0, n_pos = 0;
   bool ran = false;
-  hipEvent_t ev[7] = {};
+  hipEvent_t ev[6] = {};
+  hipEvent_t fev[2] = {};  // around a fetch's copies
+  hipEvent_t lev[2] = {};  // around the upload and the plan
   hipEvent_t kev[2] = {};  // around the extension kernel's own launch (t_kernel)
   double t_h2d = 0;
   uint64_t* h_tot = nullptr;  // pinned: totals of the count stage
@@ -1184,6 +1192,10 @@ static void destroy_batch(gs_batch* B) {
     if (e) (void)hipEventDestroy(e);
   if (B->h_tot) (void)hipHostFree(B->h_tot);
   for (auto& e : B->ev)
+    if (e) (void)hipEventDestroy(e);
+  for (auto& e : B->lev)
+    if (e) (void)hipEventDestroy(e);
+  for (auto& e : B->fev)
     if (e) (void)hipEventDestroy(e);
   for (auto& e : B->kev)
     if (e) (void)hipEventDestroy(e);
@@ -1287,6 +1299,10 @@ static int batch_events(gs_batch* B) {
   if (!B->stream && hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking) != hipSuccess) return GS_EHIP;
   for (auto& e : B->ev)
     if (!e && hipEventCreate(&e) != hipSuccess) return GS_EHIP;
+  for (auto& e : B->lev)
+    if (!e && hipEventCreate(&e) != hipSuccess) return GS_EHIP;
+  for (auto& e : B->fev)
+    if (!e && hipEventCreate(&e) != hipSuccess) return GS_EHIP;
   for (auto& e : B->kev)
     if (!e && hipEventCreate(&e) != hipSuccess) return GS_EHIP;
   if (!B->h_tot && hipHostMalloc((void**)&B->h_tot, 16, hipHostMallocDefault) != hipSuccess) return GS_ENOMEM;
@@ -1306,7 +1322,7 @@ static int ensure_buffers(gs_batch* B, uint64_t span, uint64_t n, uint64_t tasks
       B->toff.ensure(8 * nr1) || B->batch.ensure(4 * nr1) || B->cand.ensure(16 * (2 * tasks + 1)) ||
       B->nF.ensure(4 * nr1) || B->nR.ensure(4 * nr1) || B->ns.ensure(4 * nr1) || B->np.ensure(4 * nr1) ||
       B->soff.ensure(8 * nr1) || B->poff.ensure(8 * nr1) || B->tiles.ensure(scan_tile_bytes(n)) ||
-      B->tot.ensure(16) || B->queue.ensure(16) || B->counters.ensure(gs::kCounterBytes + gs::kColdBytes) ||
+      B->queue.ensure(16) || B->counters.ensure(gs::kCounterBytes + gs::kColdBytes) ||
       B->seg_link.ensure(n_long ? 4 * n_items : 16) ||
       (dyn_cap &&
        (B->dyn_items.ensure(16ull * dyn_cap) || B->dyn_meta.ensure(16ull * dyn_cap) ||
@@ -1324,9 +1340,9 @@ int gs::batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_
   const uint64_t items = 2 * (reads + bases / seg_tasks + 1);
   const uint32_t dyn = gs::piece_cap(items);
   int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, dyn);
-  if (!rc && bases > (4u << 20)) {  // the pinned chunks of staged uploads
-    const size_t ch = stage_chunk(bases);
-    if (B->st_a.ensure(ch) || B->st_b.ensure(ch)) rc = GS_ENOMEM;
+  if (!rc) {  // the pinned chunks of staged uploads
+    const size_t up = bases + 12 * reads + 1024, ch = stage_chunk(up);
+    if (B->st_a.ensure(ch) || (ch < up && B->st_b.ensure(ch))) rc = GS_ENOMEM;
   }
   return rc;
 }
@@ -1354,50 +1370,78 @@ static void parallel_parts(size_t len, F&& part) {
   for (auto& t : th) t.join();
 }
 
-// The batch's read bytes (the plan's pieces, back to back) to dst through two
-// pinned chunks: the bytes of chunk c+1 are gathered on several threads while
-// chunk c's DMA runs.  Pageable sources otherwise go through the runtime's
-// own staging, one thread at a fraction of the link's rate.
-static int staged_upload(gs_batch* B, char* dst, const std::vector<std::pair<const char*, uint64_t>>& pieces,
-                         uint64_t total) {
-  hipStream_t st = B->stream;
-  if (total <= (4u << 20)) {  // small: the pieces directly
-    uint64_t at = 0;
-    for (const auto& pc : pieces) {
-      if (hipMemcpyAsync(dst + at, pc.first, pc.second, hipMemcpyHostToDevice, st) != hipSuccess) return GS_EHIP;
-      at += pc.second;
-    }
-    return GS_OK;
+// A batch's inputs on their way to the device: the reads' bytes (pieces, back
+// to back, with 32 zero bytes behind them), offsets and lengths, each array on
+// a 256 byte boundary.
+struct UploadParts {
+  struct Source {
+    const char* p;
+    size_t bytes, at;
+  };
+  std::vector<Source> from;  // in the order of `at`
+  FetchParts to;             // src: the device array (dst unused)
+  void source(const void* p, size_t bytes, size_t at) {
+    if (bytes) from.push_back({static_cast<const char*>(p), bytes, at});
   }
-  const size_t ch = stage_chunk(total);
-  if (B->st_a.ensure(ch) || B->st_b.ensure(ch)) return GS_ENOMEM;
+  void array(void* device, const void* p, size_t bytes) {
+    source(p, bytes, to.total);
+    to.add(nullptr, device, bytes);
+  }
+  // bytes [a, z) of the sources to dst
+  void fill(size_t a, size_t z, char* dst) const {
+    size_t lo = 0, hi = from.size();  // the first source that ends past a
+    while (lo < hi) {
+      const size_t mid = (lo + hi) / 2;
+      if (from[mid].at + from[mid].bytes <= a)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    for (; lo < from.size() && from[lo].at < z; ++lo) {
+      const size_t b = std::max(a, from[lo].at), e = std::min(z, from[lo].at + from[lo].bytes);
+      if (b < e) memcpy(dst + (b - a), from[lo].p + (b - from[lo].at), e - b);
+    }
+  }
+};
+
+// Through two pinned chunks: chunk c+1 is filled on several threads while
+// chunk c is copied.  Pageable sources otherwise go through the runtime's own
+// staging, an array after another, on one thread at a fraction of the link's
+// rate.  Up to kScatterMax one launch reads them all (launch_scatter: a call
+// of 10,000 reads 102 -> 70 us); larger ones are copied array by array, which
+// reads host memory faster than that kernel (45 MB: 1.1 ms against 1.4).
+constexpr size_t kScatterMax = 2u << 20;
+static int staged_upload(gs_batch* B, const UploadParts& U) {
+  hipStream_t st = B->stream;
+  const size_t total = U.to.total;
+  if (!total) return GS_OK;
+  const size_t ch = stage_chunk(total), nch = (total + ch - 1) / ch;
+  if (B->st_a.ensure(ch) || (nch > 1 && B->st_b.ensure(ch))) return GS_ENOMEM;
   for (auto& e : B->cev)
     if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return GS_EHIP;
-  std::vector<uint64_t> start(pieces.size() + 1, 0);  // offset of each piece in the batch
-  for (size_t i = 0; i < pieces.size(); ++i) start[i + 1] = start[i] + pieces[i].second;
   char* stage[2] = {static_cast<char*>(B->st_a.p), static_cast<char*>(B->st_b.p)};
-  const size_t nch = (total + ch - 1) / ch;
   for (size_t c = 0; c < nch; ++c) {
-    // the buffer of chunk c held chunk c-2, whose DMA must be done
+    // the buffer of chunk c held chunk c-2, which must have been read
     if (c >= 2 && hipEventSynchronize(B->cev[c & 1]) != hipSuccess) return GS_EHIP;
-    const uint64_t off = c * ch, len = std::min<uint64_t>(ch, total - off);
+    const size_t off = c * ch, len = std::min(ch, total - off);
     char* sp = stage[c & 1];
-    parallel_parts(len, [&](size_t a, size_t z) {
-      uint64_t g = off + a;  // batch offset of the next byte to copy
-      size_t i = std::upper_bound(start.begin(), start.end(), g) - start.begin() - 1;
-      while (g < off + z) {
-        const uint64_t in = g - start[i], n = std::min(pieces[i].second - in, off + z - g);
-        memcpy(sp + (g - off), pieces[i].first + in, n);
-        g += n;
-        ++i;
-      }
-    });
-    if (hipMemcpyAsync(dst + off, sp, len, hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipEventRecord(B->cev[c & 1], st) != hipSuccess)
-      return GS_EHIP;
+    parallel_parts(len, [&](size_t a, size_t z) { U.fill(off + a, off + z, sp + a); });
+    if (total <= kScatterMax) {
+      if (U.to.launch_scatter(off, off + len, sp, st)) return GS_EHIP;
+    } else {
+      bool ok = true;
+      U.to.each(off, off + len, [&](const FetchParts::Part& p, size_t o, size_t m, size_t at) {
+        ok = ok && hipMemcpyAsync(static_cast<char*>(const_cast<void*>(p.src)) + o, sp + (at - off), m,
+                                  hipMemcpyHostToDevice, st) == hipSuccess;
+      });
+      if (!ok) return GS_EHIP;
+    }
+    if (c + 2 < nch && hipEventRecord(B->cev[c & 1], st) != hipSuccess) return GS_EHIP;
   }
   return GS_OK;
 }
+
+static const char kZeros[32] = {0};  // behind the reads' bytes: kernels read whole words of them
 
 // B's part of a plan on the device (PP: lo, n_whole and the reference batches)
 static void enqueue_plan(gs_batch* B, PlanParams PP, hipStream_t st) {
@@ -1415,9 +1459,17 @@ static void enqueue_plan(gs_batch* B, PlanParams PP, hipStream_t st) {
   launch_plan(PP, st);
 }
 
+static void load_time(gs_batch* B) {
+  float ms = 0;
+  (void)hipEventElapsedTime(&ms, B->lev[0], B->lev[1]);
+  B->t_h2d = ms * 1e-3;
+}
+
 // Uploads a finished plan into B, reusing B's device buffers where they are
-// large enough.  B's results and any captured graph are dropped.
-int gs::batch_load(gs_batch* B, const BatchPlan& P) {
+// large enough.  B's results and any captured graph are dropped.  Without
+// `wait` the plan and what it points at must stay as they are until the
+// batch's stream has come this far (load_time then says how long it took).
+int gs::batch_load(gs_batch* B, const BatchPlan& P, bool wait) {
   gs_index* X = B->X;
   if (hipSetDevice(X->device) != hipSuccess) return GS_EHIP;
   int rc = batch_events(B);
@@ -1439,13 +1491,25 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P) {
   if (ensure_buffers(B, B->span, n, B->tasks, B->code_chunks, B->n_items, B->n_long, B->dyn_cap))
     return GS_ENOMEM;
   hipStream_t st = B->stream;
-  if (hipEventRecord(B->ev[0], st) != hipSuccess) return GS_EHIP;
-  if ((rc = staged_upload(B, B->bases.as<char>(), P.pieces, P.span))) return rc;
-  hipLaunchKernelGGL(zero_bytes, dim3(1), dim3(32), 0, st, B->bases.as<uint8_t>() + B->span, 32u);
+  if (hipEventRecord(B->lev[0], st) != hipSuccess) return GS_EHIP;
+  const bool one = P.offs.empty();
+  {
+    UploadParts U;
+    U.from.reserve(P.pieces.size() + 3);
+    size_t at = 0;
+    for (const auto& pc : P.pieces) {
+      U.source(pc.first, pc.second, at);
+      at += pc.second;
+    }
+    U.source(kZeros, sizeof kZeros, at);
+    U.to.add(nullptr, B->bases.p, P.span + sizeof kZeros);
+    if (n) {
+      U.array(B->offs.p, one ? P.groups[0].offs : P.offs.data(), 8 * n);
+      U.array(B->lens.p, one ? P.groups[0].lens : P.lens.data(), 4 * n);
+    }
+    if ((rc = staged_upload(B, U))) return rc;
+  }
   if (n) {
-    const bool one = P.offs.empty();
-    const uint64_t* offs = one ? P.groups[0].offs : P.offs.data();
-    const uint32_t* lens = one ? P.groups[0].lens : P.lens.data();
     PlanParams PP{};
     PP.lo = one ? P.groups[0].lo : 0;
     PP.n_whole = P.n_whole;
@@ -1461,16 +1525,14 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P) {
           return GS_EHIP;
       }
     }
-    if (hipMemcpyAsync(B->offs.p, offs, 8 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
-        hipMemcpyAsync(B->lens.p, lens, 4 * n, hipMemcpyHostToDevice, st) != hipSuccess)
-      return GS_EHIP;
     enqueue_plan(B, PP, st);
     if (hipGetLastError() != hipSuccess) return GS_EHIP;
   }
-  if (hipEventRecord(B->ev[1], st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return GS_EHIP;
-  float ms = 0;
-  (void)hipEventElapsedTime(&ms, B->ev[0], B->ev[1]);
-  B->t_h2d = ms * 1e-3;
+  if (hipEventRecord(B->lev[1], st) != hipSuccess) return GS_EHIP;
+  if (wait) {
+    if (hipStreamSynchronize(st) != hipSuccess) return GS_EHIP;
+    load_time(B);
+  }
   return GS_OK;
 }
 
@@ -1634,8 +1696,7 @@ static int enqueue_counts(gs_batch* B, const PostParams& Q, hipStream_t st) {
     hipLaunchKernelGGL(finalize_reads<false>, dim3(grid_for(n, 256)), dim3(256), 0, st, Q);
     if (Q.n_long) hipLaunchKernelGGL(finalize_long<false>, dim3((Q.n_long + 3) / 4), dim3(256), 0, st, Q);
     launch_pair_scan({{Q.nseeds, Q.npos}, {B->soff.as<uint64_t>(), B->poff.as<uint64_t>()}, n, 0,
-                      B->tiles.as<uint64_t>(), B->tot.as<uint64_t>()}, st);
-    GS_HIP(hipMemcpyAsync(B->h_tot, B->tot.p, 16, hipMemcpyDeviceToHost, st));
+                      B->tiles.as<uint64_t>(), B->h_tot}, st);
   } else {  // no reads: the offset arrays still hold their closing 0
     hipLaunchKernelGGL(zero_bytes, dim3(1), dim3(32), 0, st, B->soff.as<uint8_t>(), 8u);
     hipLaunchKernelGGL(zero_bytes, dim3(1), dim3(32), 0, st, B->poff.as<uint8_t>(), 8u);
@@ -1676,14 +1737,12 @@ static int persistent_grid_for(gs_batch* B, int kernel, unsigned* grid) {
   return gs::persistent_grid(kernel - 1, B->opts.wg, grid);
 }
 
-// Runs the whole device pipeline on an uploaded batch; results stay in HBM.
-extern "C" GS_API int gs_batch_run(gs_batch* B, int kernel_override, gs_batch_stats* stats) {
-  if (!B) return GS_EINVAL;
+// The whole device pipeline on an uploaded batch; results stay in HBM.  kev:
+// record the extension kernel's own time; its end is waited for by the caller.
+static int run_pipeline(gs_batch* B, int kernel, bool kev) {
   gs_index* X = B->X;
   if (hipSetDevice(X->device) != hipSuccess) return GS_EHIP;
   hipStream_t st = B->stream;
-  const int kernel = kernel_override >= 0 ? kernel_override : B->opts.kernel;
-  if (kernel < 0 || kernel > 3) return GS_EINVAL;
   unsigned pgrid = 0;
   int rc = persistent_grid_for(B, kernel, &pgrid);
   if (rc) return rc;
@@ -1692,7 +1751,7 @@ extern "C" GS_API int gs_batch_run(gs_batch* B, int kernel_override, gs_batch_st
   fill_params(B, S, Q);
   B->h_tot[0] = B->h_tot[1] = 0;
   GS_HIP(hipEventRecord(B->ev[0], st));
-  rc = enqueue_extension(B, S, kernel, pgrid, st, B->kev);
+  rc = enqueue_extension(B, S, kernel, pgrid, st, kev ? B->kev : nullptr);
   if (rc) return rc;
   GS_HIP(hipEventRecord(B->ev[1], st));
   rc = enqueue_counts(B, Q, st);
@@ -1711,28 +1770,46 @@ extern "C" GS_API int gs_batch_run(gs_batch* B, int kernel_override, gs_batch_st
   GS_HIP(hipEventRecord(B->ev[4], st));
   if ((rc = enqueue_walk(B, S, Q, st))) return rc;
   GS_HIP(hipEventRecord(B->ev[5], st));
-  GS_HIP(hipStreamSynchronize(st));
   B->ran = true;
   B->graph_fresh = false;
+  return GS_OK;
+}
+
+// times and sizes of a run that has ended
+static void run_stats(gs_batch* B, gs_batch_stats* stats) {
+  float ms[5] = {0, 0, 0, 0, 0};
+  (void)hipEventElapsedTime(&ms[0], B->ev[0], B->ev[1]);
+  (void)hipEventElapsedTime(&ms[1], B->ev[1], B->ev[2]);
+  (void)hipEventElapsedTime(&ms[2], B->ev[3], B->ev[4]);
+  (void)hipEventElapsedTime(&ms[3], B->ev[4], B->ev[5]);
+  (void)hipEventElapsedTime(&ms[4], B->ev[0], B->ev[5]);
+  memset(stats, 0, sizeof(*stats));
+  stats->t_h2d = B->t_h2d;
+  stats->t_seed = ms[0] * 1e-3;
+  stats->t_count = ms[1] * 1e-3;
+  stats->t_write = ms[2] * 1e-3;
+  stats->t_locate = ms[3] * 1e-3;
+  stats->t_total = ms[4] * 1e-3;
+  stats->n_reads = B->n_reads;
+  stats->n_seeds = B->n_seeds;
+  stats->n_pos = B->n_pos;
+}
+
+extern "C" GS_API int gs_batch_run(gs_batch* B, int kernel_override, gs_batch_stats* stats) {
+  if (!B) return GS_EINVAL;
+  const int kernel = kernel_override >= 0 ? kernel_override : B->opts.kernel;
+  if (hipSetDevice(B->X->device) != hipSuccess) return GS_EHIP;
+  if (kernel < 0 || kernel > 3) return GS_EINVAL;
+  const int rc = run_pipeline(B, kernel, true);
+  if (rc) return rc;
+  if (hipStreamSynchronize(B->stream) != hipSuccess) {
+    B->ran = false;
+    return GS_EHIP;
+  }
   if (stats) {
-    float ms[5] = {0, 0, 0, 0, 0};
-    (void)hipEventElapsedTime(&ms[0], B->ev[0], B->ev[1]);
-    (void)hipEventElapsedTime(&ms[1], B->ev[1], B->ev[2]);
-    (void)hipEventElapsedTime(&ms[2], B->ev[3], B->ev[4]);
-    (void)hipEventElapsedTime(&ms[3], B->ev[4], B->ev[5]);
-    (void)hipEventElapsedTime(&ms[4], B->ev[0], B->ev[5]);
-    memset(stats, 0, sizeof(*stats));
-    stats->t_h2d = B->t_h2d;
-    stats->t_seed = ms[0] * 1e-3;
-    stats->t_count = ms[1] * 1e-3;
-    stats->t_write = ms[2] * 1e-3;
-    stats->t_locate = ms[3] * 1e-3;
-    stats->t_total = ms[4] * 1e-3;
+    run_stats(B, stats);
     float kms = 0;
     if (B->n_reads && hipEventElapsedTime(&kms, B->kev[0], B->kev[1]) == hipSuccess) stats->t_kernel = kms * 1e-3;
-    stats->n_reads = B->n_reads;
-    stats->n_seeds = B->n_seeds;
-    stats->n_pos = B->n_pos;
     if (kernel >= 1) {
       uint64_t c[4] = {0, 0, 0, 0};
       if (hipMemcpy(c, B->counters.p, 32, hipMemcpyDeviceToHost) == hipSuccess) {
@@ -1943,7 +2020,7 @@ extern "C" GS_API int gs_batch_fetch(gs_batch* B, gs_result* out) {
     });
     return GS_OK;
   }
-  hipEvent_t e0 = B->ev[5], e1 = B->ev[6];
+  hipEvent_t e0 = B->fev[0], e1 = B->fev[1];
   int rc = GS_OK;
   if (hipEventRecord(e0, st) != hipSuccess) rc = GS_EHIP;
   FetchParts P;
@@ -2058,11 +2135,19 @@ extern "C" GS_API int gs_seed(gs_index* X, const char* bases, const uint64_t* of
   // reused (no allocation, which would synchronise the device, once they fit)
   if (!X->work) X->work = gs::batch_new(X, false);
   gs_batch* B = X->work;
-  if ((rc = gs::batch_load(B, P))) return rc;
-  gs_batch_stats s;
-  rc = gs_batch_run(B, -1, &s);
+  // one stream from upload to fetch, waited for where the host needs the
+  // sizes and the results (a wait after each stage, and the counters' copy,
+  // made 0.1 ms of a call of 10,000 reads)
+  rc = gs::batch_load(B, P, false);
+  if (!rc) rc = run_pipeline(B, B->opts.kernel, false);
   if (!rc) rc = gs_batch_fetch(B, out);
-  if (!rc) {
+  if (rc) {
+    if (B->stream) (void)hipStreamSynchronize(B->stream);  // the caller's arrays may still be read
+    B->ran = false;
+  } else {
+    load_time(B);
+    gs_batch_stats s;
+    run_stats(B, &s);
     out->t_h2d = s.t_h2d;
     out->t_seed = s.t_seed;
     out->t_post = s.t_count + s.t_write;
@@ -2097,12 +2182,13 @@ constexpr int kNoAllocDevices = 64;
 
 static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
 
-// Small results of a call leave through pinned memory that is set up with the
-// scratch array (larger ones go straight to the caller's arrays).
-constexpr size_t kNoAllocStage = 1u << 20;
+// Small inputs and results of a call go through pinned memory that is set up
+// with the scratch array (larger ones are copied from and to the caller's
+// arrays), behind the call's totals.
+constexpr size_t kNoAllocStage = 1u << 20, kNoAllocTotals = 256;
 
 std::mutex g_scratch_mu;
-char* g_scratch_stage[kNoAllocDevices];  // pinned, kNoAllocStage bytes (null: none)
+char* g_scratch_stage[kNoAllocDevices];  // pinned, kNoAllocTotals + kNoAllocStage bytes
 void* g_scratch_ptr[kNoAllocDevices];  // device address of `scratch` on each device (null: not looked up)
 int g_scratch_rc[kNoAllocDevices];     // the lookup's result once it has run
 
@@ -2150,7 +2236,10 @@ int gs::noalloc_setup(int device) {
     return GS_EHIP;
   }
   void* stage = nullptr;
-  if (hipHostMalloc(&stage, kNoAllocStage, hipHostMallocDefault) != hipSuccess) stage = nullptr;
+  if (hipHostMalloc(&stage, kNoAllocTotals + kNoAllocStage, hipHostMallocDefault) != hipSuccess) {
+    g_scratch_rc[device] = GS_EHIP;
+    return GS_EHIP;
+  }
   g_scratch_stage[device] = static_cast<char*>(stage);
   g_scratch_ptr[device] = p;
   return GS_OK;
@@ -2214,8 +2303,9 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
                  o_toff = take(8 * nr1), o_batch = take(4 * nr1), o_cand = take(16 * (2 * tasks + 1)),
                  o_nF = take(4 * nr1), o_nR = take(4 * nr1), o_ns = take(4 * nr1), o_np = take(4 * nr1),
                  o_soff = take(8 * nr1), o_poff = take(8 * nr1), o_spare = take(8 * (nr1 / kScanTile + 2)),
-                 o_tot = take(16), o_queue = take(16), o_counters = take(gs::kCounterBytes + gs::kColdBytes);
+                 o_tot = take(16) /* unused */, o_queue = take(16), o_counters = take(gs::kCounterBytes + gs::kColdBytes);
   (void)o_spare;
+  (void)o_tot;
   const uint64_t common = at;
   const uint64_t o_code_off = take(8 * nr1), o_long = long_scratch ? take(4 * (span + 16)) : 0;
   if (short_batched) {
@@ -2286,7 +2376,9 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
     B.wlink.view(base + o_wlink, 8 * nr1);
     if (n_long) B.seg_link.view(base + o_seg_link, 4 * n_items);
   }
-  uint64_t h_tot[2] = {0, 0};
+  uint64_t* const h_tot = reinterpret_cast<uint64_t*>(stage);
+  stage += kNoAllocTotals;
+  h_tot[0] = h_tot[1] = 0;
   B.h_tot = h_tot;
   B.bases.view(base + o_bases, span + 32);
   B.offs.view(base + o_offs, 8 * nr1);
@@ -2304,17 +2396,28 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   // the scans' tile totals: with seed_streams in place of the code offsets it
   // does not read (40 bytes per 2048 reads, 8 per read)
   B.tiles.view(base + (streams ? o_code_off : o_tiles2), scan_tile_bytes(n));
-  B.tot.view(base + o_tot, 16);
   B.queue.view(base + o_queue, 16);
   B.counters.view(base + o_counters, gs::kCounterBytes + gs::kColdBytes);
   if (streams && long_scratch) B.scratch.view(base + o_long, 4 * (span + 16));
 
   // inputs, then the plan on the device
-  if ((span && hipMemcpyAsync(B.bases.p, bases + lo, span, hipMemcpyHostToDevice, st) != hipSuccess) ||
-      (n && (hipMemcpyAsync(B.offs.p, offsets, 8ull * n, hipMemcpyHostToDevice, st) != hipSuccess ||
-             hipMemcpyAsync(B.lens.p, lens, 4ull * n, hipMemcpyHostToDevice, st) != hipSuccess)))
-    return GS_EHIP;
-  hipLaunchKernelGGL(zero_bytes, dim3(1), dim3(32), 0, st, B.bases.as<uint8_t>() + span, 32u);
+  FetchParts in;
+  in.add(nullptr, B.bases.p, span + sizeof kZeros);
+  in.add(nullptr, B.offs.p, 8ull * n);
+  in.add(nullptr, B.lens.p, 4ull * n);
+  if (in.total <= kNoAllocStage) {
+    if (span) memcpy(stage, bases + lo, span);
+    memcpy(stage + span, kZeros, sizeof kZeros);
+    if (n) memcpy(stage + in.part[1].at, offsets, 8ull * n);
+    if (n) memcpy(stage + in.part[2].at, lens, 4ull * n);
+    if ((rc = in.launch_scatter(0, in.total, stage, st))) return rc;
+  } else {
+    if ((span && hipMemcpyAsync(B.bases.p, bases + lo, span, hipMemcpyHostToDevice, st) != hipSuccess) ||
+        (n && (hipMemcpyAsync(B.offs.p, offsets, 8ull * n, hipMemcpyHostToDevice, st) != hipSuccess ||
+               hipMemcpyAsync(B.lens.p, lens, 4ull * n, hipMemcpyHostToDevice, st) != hipSuccess)))
+      return GS_EHIP;
+    hipLaunchKernelGGL(zero_bytes, dim3(1), dim3(32), 0, st, B.bases.as<uint8_t>() + span, 32u);
+  }
   if (n) {
     PlanParams PP{};
     PP.lo = lo;
@@ -2364,7 +2467,7 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   P.add(out->read_pos_off, B.poff.p, 8 * nr1);
   P.add(out->seeds, B.seeds.p, sizeof(gs_seed_rec) * n_seeds);
   P.add(out->pos, B.rows.p, 4 * n_pos);
-  const bool staged = stage && P.total <= kNoAllocStage;
+  const bool staged = P.total <= kNoAllocStage;
   if (staged) {
     if ((rc = P.launch_gather(0, P.total, stage, st))) return rc;
   } else {

@@ -1167,9 +1167,20 @@ __global__ void __launch_bounds__(256) join_whole_wave(gs::JoinParams J) {
   uint32_t* const n_out = strand ? J.nR : J.nF;
   if (n_out[r] != gs::kSplitStream) return;
   const uint32_t ntask = J.lens[r] - J.k + 1;
-  const uint32_t link = J.wlink[t];
-  const uint32_t n = 1 + chain_length(J, link);
-  if ((threadIdx.x & 63) == 0) list_chain(J, list, 0, 0, J.wmeta[t], link, n);
+  uint32_t n = 0;  // pieces, the whole wave following the chain
+  uint32_t t0 = 0, link = J.wlink[t];
+  uint4 m = J.wmeta[t];
+  while (true) {
+    if ((threadIdx.x & 63) == 0) {
+      list.t0[n] = t0;
+      list.meta[n] = m;
+    }
+    ++n;
+    if (link == kNone || n >= kJoinList) break;
+    m = J.dyn_meta[link];
+    t0 = J.dyn_items[link].z;
+    link = J.dyn_link[link];
+  }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
   uint32_t K = 0, LB = 0xFFFFFFFFu;
@@ -1229,23 +1240,25 @@ __global__ void __launch_bounds__(256) pack_codes(const uint8_t* __restrict__ ba
   codes[code_off[r] + strand * nch + c] = slot_chunk(pack_chunk(bases + offs[r], L, strand, c));
 }
 
-// longer reads: a fixed grid of waves taking the reads in turn, a wave's
-// lanes one chunk each (a workgroup per read left the launch bound by
-// workgroup dispatch: 1.4 M workgroups of about a hundred chunks each)
+// longer reads: a fixed grid of waves taking the reads, or one of their
+// `parts` parts, in turn, a wave's lanes one chunk each (a workgroup per read
+// left the launch bound by workgroup dispatch: 1.4 M workgroups of about a
+// hundred chunks each; a wave per read left a launch of few reads waiting for
+// the longest: 1000 uneven reads 31 -> 11 us)
 __global__ void __launch_bounds__(256) pack_codes_long(const uint8_t* __restrict__ bases,
                                                        const uint64_t* __restrict__ offs,
                                                        const uint32_t* __restrict__ lens,
                                                        const uint64_t* __restrict__ code_off,
                                                        const uint32_t* __restrict__ long_reads, uint32_t n_long,
-                                                       uint4* __restrict__ codes) {
+                                                       uint32_t parts, uint4* __restrict__ codes) {
   const uint32_t lane = threadIdx.x & 63, n_waves = gridDim.x * 4;
-  for (uint32_t w = blockIdx.x * 4 + (threadIdx.x >> 6); w < n_long; w += n_waves) {
-    const uint32_t r = long_reads[w];
+  for (uint64_t w = blockIdx.x * 4 + (threadIdx.x >> 6); w < (uint64_t)n_long * parts; w += n_waves) {
+    const uint32_t r = long_reads[w / parts], part = (uint32_t)(w % parts);
     const uint32_t L = lens[r];
     const uint32_t nch = (L + 31) >> 5;
     const uint8_t* s = bases + offs[r];
     uint4* dst = codes + code_off[r];
-    for (uint32_t q = lane; q < 2 * nch; q += 64) {
+    for (uint32_t q = 64 * part + lane; q < 2 * nch; q += 64 * parts) {
       const uint32_t strand = q >= nch ? 1u : 0u;
       dst[q] = pack_chunk(s, L, strand, q - strand * nch);
     }
@@ -1362,9 +1375,12 @@ int launch_pack_codes(const uint8_t* bases, const uint64_t* offs, const uint32_t
   if (threads)
     hipLaunchKernelGGL(pack_codes, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, bases, offs, lens,
                        code_off, n_reads, codes);
-  if (n_long)
-    hipLaunchKernelGGL(pack_codes_long, dim3(std::min<uint32_t>((n_long + 3) / 4, kHelperGrid)), dim3(256), 0, st,
-                       bases, offs, lens, code_off, long_reads, n_long, codes);
+  if (n_long) {
+    const uint32_t parts = std::min(16u, std::max(1u, 4 * kHelperGrid / n_long));
+    const uint64_t waves = (uint64_t)n_long * parts;
+    hipLaunchKernelGGL(pack_codes_long, dim3((unsigned)std::min<uint64_t>((waves + 3) / 4, kHelperGrid)), dim3(256),
+                       0, st, bases, offs, lens, code_off, long_reads, n_long, parts, codes);
+  }
   return hipGetLastError() == hipSuccess ? GS_OK : GS_EHIP;
 }
 

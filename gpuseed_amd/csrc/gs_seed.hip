@@ -296,6 +296,7 @@ struct PostParams {
   const uint64_t* pos_off;
   gs_seed_rec* seeds;
   uint32_t* rows;
+  uint32_t per_wave;          // reads of a wave of finalize_reads
   uint32_t long_min;          // reads longer than this go to finalize_long
   uint32_t n_long;
   const uint32_t* long_reads;
@@ -466,21 +467,26 @@ __device__ __forceinline__ void count_part(const PostParams& P, Part p, uint32_t
   }
 }
 
+// Entries with at least this many rows have them written by the whole wave.
+constexpr uint32_t kWaveRows = 16;
+
 // Writes the seed records of the lanes' parts from so on, and their rows from
-// po on.  The lanes take an entry each per turn and then write the rows of
-// all of them together, 64 at a time whatever entry they are of: one seed may
-// report as many rows as max_occ allows, or the whole of a repeat, and a lane
-// writing its own rows kept its wave waiting.  Records and rows, max_occ 500:
-// 300,007 MEM reads of up to 101 bases on a 100 Mbp index 2.09 -> 0.17 ms
-// (with the sharing of kSharedEntries), 100,000 SMEM reads of 150 there 0.15
-// -> 0.03 ms.  Reading the full suffix array here in place of locate_rows'
-// pass was slower (1,000,000 reads on the 3.1 Gbp index 0.30 ms against 0.25,
-// 60,000 uneven reads 0.40 against 0.29): its loads wait a turn each.
+// po on.  The lanes take an entry each per turn and write up to kWaveRows - 1
+// rows of it themselves; the rows of an entry with more (as many as max_occ
+// allows, or the whole of a repeat) are written by the wave, 64 at a time,
+// one such entry after another: a lane that wrote them alone kept its wave
+// waiting (300,007 MEM reads of up to 101 bases on a 100 Mbp index, max_occ
+// 500: 2.09 ms), and finding the entry of each row among all lanes' takes 19
+// shuffles per 64 rows (the same reads 0.17 ms, 0.16 with this; 1000 uneven
+// reads 41 -> 17 us, 10,000 MEM reads with every row 82 -> 49 us).
+// Reading the full suffix array here in place of locate_rows' pass was slower
+// (1,000,000 reads on the 3.1 Gbp index 0.30 ms against 0.25, 60,000 uneven
+// reads 0.40 against 0.29): its loads wait a turn each.
 // Every lane of the wave takes part.
 __device__ void write_parts(const PostParams& P, Part p, uint64_t so, uint64_t po) {
   const uint32_t lane = threadIdx.x & 63;
   while (__ballot(p.left != 0)) {
-    uint32_t cnt = 0, z = 0, done = 0;
+    uint32_t cnt = 0, z = 0;
     uint2 skip = make_uint2(1, 0);
     uint64_t dst = po;
     if (p.left) {
@@ -500,30 +506,17 @@ __device__ void write_parts(const PostParams& P, Part p, uint64_t so, uint64_t p
         if (cnt && !P.smem) skip = mem_skip(P, p.r, e.rev, e.i);
       }
     }
-    while (__ballot(cnt != 0)) {
-      const uint32_t c = cnt < 65536u ? cnt : 65536u;  // of this lane's rows, in this turn
-      uint32_t inc = c;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t t = __shfl_up(inc, d);
-        if (lane >= (uint32_t)d) inc += t;
-      }
-      const uint32_t total = __shfl(inc, 63), first = inc - c;
-      for (uint32_t o0 = 0; o0 < total; o0 += 64) {
-        const uint32_t o = o0 + lane;
-        uint32_t q = 0;  // the lane whose rows hold o
-#pragma unroll
-        for (uint32_t w = 32; w; w >>= 1)
-          if (__shfl(inc, (int)(q + w - 1)) <= o) q += w;
-        q &= 63u;
-        const uint32_t i = o - __shfl(first, (int)q) + __shfl(done, (int)q);
-        const uint2 sk = make_uint2(__shfl(skip.x, (int)q), __shfl(skip.y, (int)q));
-        const uint32_t zq = __shfl(z, (int)q);
-        const uint64_t at = __shfl(dst, (int)q) + i;
-        if (o < total) P.rows[at] = nth_row(zq, sk, i);
-      }
-      done += c;
-      cnt -= c;
+    if (cnt < kWaveRows)
+      for (uint32_t i = 0; i < cnt; ++i) P.rows[dst + i] = nth_row(z, skip, i);
+    for (uint64_t m = __ballot(cnt >= kWaveRows); m; m &= m - 1) {
+      const int q = __ffsll((unsigned long long)m) - 1;
+      const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cnt, q);
+      const uint32_t zq = (uint32_t)__builtin_amdgcn_readlane((int)z, q);
+      const uint2 sk = make_uint2((uint32_t)__builtin_amdgcn_readlane((int)skip.x, q),
+                                  (uint32_t)__builtin_amdgcn_readlane((int)skip.y, q));
+      const uint64_t at = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)dst, q) |
+                          ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(dst >> 32), q) << 32);
+      for (uint64_t i = lane; i < c; i += 64) P.rows[at + i] = nth_row(zq, sk, (uint32_t)i);
     }
   }
 }
@@ -589,13 +582,21 @@ __device__ __forceinline__ void finalize_shared(const PostParams& P, uint32_t r)
 // 0.71, 0.84 ms; 1,000,000 SMEM reads with 4, 16: 0.75, 0.43 ms).
 constexpr uint32_t kSharedEntries = 16;
 
+// Reads of a wave: fewer than 64 in small calls, whose few waves otherwise take
+// their reads of many entries one after another (10,000 MEM reads: 157 waves;
+// counts 30 -> 21 us, records with kWaveRows above 82 -> 49 us).
+inline uint32_t reads_per_wave(uint64_t n) {
+  return (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(8, (n + 4095) / 4096));
+}
+
 // A lane per read, then the wave together for each of its reads with many
 // entries.  Count pass (WRITE false): seeds and positions per read.  Write
 // pass: seed records and suffix-array rows at the scanned offsets.
 template <bool WRITE>
 __global__ void __launch_bounds__(256) finalize_reads(PostParams P) {
-  const uint32_t r = blockIdx.x * 256 + threadIdx.x;
-  const bool mine = r < P.n_reads && !(P.lens[r] > P.long_min && P.lens[r] >= P.k);  // else finalize_long's
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t r = (blockIdx.x * 4 + (threadIdx.x >> 6)) * P.per_wave + lane;
+  const bool mine = lane < P.per_wave && r < P.n_reads && !(P.lens[r] > P.long_min && P.lens[r] >= P.k);  // else finalize_long's
   Part p;
   p.r = r;
   p.a = p.z = p.left = 0;
@@ -641,7 +642,7 @@ __global__ void __launch_bounds__(256) finalize_long(PostParams P) {
 // its four wave totals in LDS.
 
 constexpr int kScanBlock = 256;
-constexpr int kScanItems = 8;  // per thread
+constexpr int kScanItems = 8;  // per thread, fewer where one workgroup holds all the reads (ONE_TILE)
 constexpr uint32_t kScanTile = kScanBlock * kScanItems;
 
 __device__ __forceinline__ uint64_t wave_incl_scan(uint64_t v) {
@@ -699,12 +700,13 @@ struct PairScan {
   uint64_t* total;  // [2], pinned host memory
 };
 
-// the thread's kScanItems counts from `base` on (sum returned, each in v)
+// the thread's ITEMS counts from `base` on (sum returned, each in v)
+template <int ITEMS>
 __device__ __forceinline__ uint64_t load_counts(const uint32_t* __restrict__ in, uint64_t n, uint64_t base,
                                                 uint32_t* v) {
   uint64_t s = 0;
 #pragma unroll
-  for (int q = 0; q < kScanItems; ++q) {
+  for (int q = 0; q < ITEMS; ++q) {
     v[q] = base + q < n ? in[base + q] : 0u;
     s += v[q];
   }
@@ -717,29 +719,30 @@ __global__ void __launch_bounds__(kScanBlock) pair_totals(PairScan S) {
   for (int h = 0; h < 2; ++h) {
     uint32_t v[kScanItems];
     uint64_t tot;
-    block_excl_scan(load_counts(S.in[h], S.n, base, v), &tot);
+    block_excl_scan(load_counts<kScanItems>(S.in[h], S.n, base, v), &tot);
     if (threadIdx.x == 0) S.tiles[h * S.ntiles + blockIdx.x] = tot;
   }
 }
 
+template <int ITEMS>
 __global__ void __launch_bounds__(kScanBlock) pair_apply(PairScan S) {
-  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
+  const uint64_t base = (uint64_t)blockIdx.x * kScanBlock * ITEMS + threadIdx.x * ITEMS;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    uint32_t v[kScanItems];
+    uint32_t v[ITEMS];
     uint64_t tot;
-    uint64_t run = block_excl_scan(load_counts(S.in[h], S.n, base, v), &tot);
+    uint64_t run = block_excl_scan(load_counts<ITEMS>(S.in[h], S.n, base, v), &tot);
     if (S.ntiles == 1) {
       if (threadIdx.x == 0) S.total[h] = tot;
     } else {
       run += S.tiles[h * S.ntiles + blockIdx.x];
     }
 #pragma unroll
-    for (int q = 0; q < kScanItems; ++q) {
+    for (int q = 0; q < ITEMS; ++q) {
       if (base + q < S.n) S.out[h][base + q] = run;
       run += v[q];
     }
-    if (base + kScanItems >= S.n && base < S.n) S.out[h][S.n] = run;  // the thread holding the last item
+    if (base + ITEMS >= S.n && base < S.n) S.out[h][S.n] = run;  // the thread holding the last item
   }
 }
 
@@ -886,12 +889,12 @@ __global__ void __launch_bounds__(kScanBlock) plan_totals(PlanParams P) {
   }
 }
 
+template <int ITEMS>
 __global__ void __launch_bounds__(kScanBlock) plan_apply(PlanParams P) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint64_t base = (uint64_t)blockIdx.x * kScanTile + threadIdx.x * kScanItems;
+  const uint64_t base = (uint64_t)blockIdx.x * kScanBlock * ITEMS + threadIdx.x * ITEMS;
   uint64_t s[kPlanSums] = {0, 0, 0, 0, 0};
 #pragma unroll
-  for (int j = 0; j < kScanItems; ++j) {
+  for (int j = 0; j < ITEMS; ++j) {
     uint32_t L, c[kPlanSums];
     plan_counts(P, base + j, L, c);
 #pragma unroll
@@ -902,7 +905,7 @@ __global__ void __launch_bounds__(kScanBlock) plan_apply(PlanParams P) {
     uint64_t tot;
     s[q] = block_excl_scan(s[q], &tot) + (P.ntiles == 1 ? 0 : P.tiles[q * P.ntiles + blockIdx.x]);
   }
-  for (int j = 0; j < kScanItems; ++j) {
+  for (int j = 0; j < ITEMS; ++j) {
     const uint64_t i = base + j;
     uint32_t L, c[kPlanSums];
     const bool lng = plan_counts(P, i, L, c);
@@ -941,17 +944,22 @@ __global__ void __launch_bounds__(kScanBlock) plan_apply(PlanParams P) {
         }
       }
     }
-    // a long read's items by the whole wave
-    for (uint64_t m = __ballot(lng && P.items); m; m &= m - 1) {
-      const int from = __ffsll((unsigned long long)m) - 1;
-      const uint64_t ri = __shfl((uint64_t)i, from), at = __shfl(first, from);
-      const uint32_t ni = __shfl(c[3], from);
-      for (uint32_t g = lane; g < ni; g += 64)
-        P.items[at + g] = ri | ((uint64_t)(g & 1u) << 32) | ((uint64_t)(g >> 1) << 33);
-    }
 #pragma unroll
     for (int q = 0; q < kPlanSums; ++q) s[q] += c[q];
   }
+}
+
+// A long read's items, a wave each (in plan_apply, whose one workgroup holds
+// the reads of a small call, its waves wrote them one read after another: 60
+// of 68 us for 1000 uneven reads).
+__global__ void __launch_bounds__(256) plan_long_items(PlanParams P, uint32_t n_long) {
+  const uint32_t w = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= n_long) return;
+  const uint32_t r = P.long_reads[w];
+  const uint32_t n = 2u * gs::n_segments(P.lens[r], P.k, P.seg_tasks);
+  uint64_t* const out = P.items + P.item0[w];
+  for (uint32_t g = threadIdx.x & 63; g < n; g += 64)
+    out[g] = (uint64_t)r | ((uint64_t)(g & 1u) << 32) | ((uint64_t)(g >> 1) << 33);
 }
 
 // ---- device buffers of one gs_seed call -------------------------------------
@@ -989,6 +997,20 @@ inline uint64_t scan_ntiles(uint64_t n) { return (n + kScanTile - 1) / kScanTile
 // bytes of the tile totals of either scan over n reads
 inline uint64_t scan_tile_bytes(uint64_t n) { return 8 * kPlanSums * (scan_ntiles(n) + 1); }
 
+// The last launch of a scan: with as few items per thread as hold n reads in
+// one workgroup (the threads' serial parts decide there: the plan of 64 reads
+// 9.2 -> 3.3 us, of 1000 13 -> 7.8).
+#define GS_ONE_TILE(kernel, n, tiles, st, ...)                                                   \
+  do {                                                                                           \
+    if ((n) <= kScanBlock)                                                                       \
+      hipLaunchKernelGGL(kernel<1>, dim3(1), dim3(kScanBlock), 0, st, __VA_ARGS__);              \
+    else if ((n) <= 4 * kScanBlock)                                                              \
+      hipLaunchKernelGGL(kernel<4>, dim3(1), dim3(kScanBlock), 0, st, __VA_ARGS__);              \
+    else                                                                                         \
+      hipLaunchKernelGGL(kernel<kScanItems>, dim3((unsigned)(tiles)), dim3(kScanBlock), 0, st,   \
+                         __VA_ARGS__);                                                           \
+  } while (0)
+
 void launch_pair_scan(PairScan S, hipStream_t st) {
   S.ntiles = scan_ntiles(S.n);
   if (!S.ntiles) return;
@@ -996,10 +1018,10 @@ void launch_pair_scan(PairScan S, hipStream_t st) {
     hipLaunchKernelGGL(pair_totals, dim3((unsigned)S.ntiles), dim3(kScanBlock), 0, st, S);
     hipLaunchKernelGGL(scan_tiles<2>, dim3(1), dim3(kScanBlock), 0, st, S.tiles, S.ntiles, S.total);
   }
-  hipLaunchKernelGGL(pair_apply, dim3((unsigned)S.ntiles), dim3(kScanBlock), 0, st, S);
+  GS_ONE_TILE(pair_apply, S.n, S.ntiles, st, S);
 }
 
-void launch_plan(PlanParams P, hipStream_t st) {
+void launch_plan(PlanParams P, uint32_t n_long, hipStream_t st) {
   P.ntiles = scan_ntiles(P.n);
   if (!P.ntiles) return;
   if (P.ntiles > 1) {
@@ -1007,7 +1029,8 @@ void launch_plan(PlanParams P, hipStream_t st) {
     hipLaunchKernelGGL(scan_tiles<kPlanSums>, dim3(1), dim3(kScanBlock), 0, st, P.tiles, P.ntiles,
                        (uint64_t*)nullptr);
   }
-  hipLaunchKernelGGL(plan_apply, dim3((unsigned)P.ntiles), dim3(kScanBlock), 0, st, P);
+  GS_ONE_TILE(plan_apply, P.n, P.ntiles, st, P);
+  if (n_long && P.items) hipLaunchKernelGGL(plan_long_items, dim3((n_long + 3) / 4), dim3(256), 0, st, P, n_long);
 }
 
 // Arrays on their way to pinned host memory or back: copied by one launch, 16
@@ -1456,7 +1479,7 @@ static void enqueue_plan(gs_batch* B, PlanParams PP, hipStream_t st) {
   PP.long_reads = B->long_reads.as<uint32_t>();
   PP.item0 = B->item0.as<uint64_t>();
   PP.tiles = B->tiles.as<uint64_t>();
-  launch_plan(PP, st);
+  launch_plan(PP, B->n_long, st);
 }
 
 static void load_time(gs_batch* B) {
@@ -1606,6 +1629,7 @@ static void fill_params(gs_batch* B, SeedParams& S, PostParams& Q) {
   Q.seeds = B->seeds.as<gs_seed_rec>();
   Q.rows = B->rows.as<uint32_t>();
   // reads longer than the persistent kernel's window are finalized a wave each
+  Q.per_wave = reads_per_wave(B->n_reads);
   Q.long_min = B->n_long ? gs::kPersistLmax : 0xFFFFFFFFu;
   Q.n_long = B->n_long;
   Q.long_reads = B->long_reads.as<uint32_t>();
@@ -1693,7 +1717,7 @@ static int enqueue_extension(gs_batch* B, const SeedParams& S, int kernel, unsig
 static int enqueue_counts(gs_batch* B, const PostParams& Q, hipStream_t st) {
   const uint64_t n = B->n_reads;
   if (n) {
-    hipLaunchKernelGGL(finalize_reads<false>, dim3(grid_for(n, 256)), dim3(256), 0, st, Q);
+    hipLaunchKernelGGL(finalize_reads<false>, dim3(grid_for(n, 4 * Q.per_wave)), dim3(256), 0, st, Q);
     if (Q.n_long) hipLaunchKernelGGL(finalize_long<false>, dim3((Q.n_long + 3) / 4), dim3(256), 0, st, Q);
     launch_pair_scan({{Q.nseeds, Q.npos}, {B->soff.as<uint64_t>(), B->poff.as<uint64_t>()}, n, 0,
                       B->tiles.as<uint64_t>(), B->h_tot}, st);
@@ -1705,7 +1729,7 @@ static int enqueue_counts(gs_batch* B, const PostParams& Q, hipStream_t st) {
 }
 
 static int enqueue_write(gs_batch* B, const PostParams& Q, hipStream_t st) {
-  if (B->n_reads) hipLaunchKernelGGL(finalize_reads<true>, dim3(grid_for(B->n_reads, 256)), dim3(256), 0, st, Q);
+  if (B->n_reads) hipLaunchKernelGGL(finalize_reads<true>, dim3(grid_for(B->n_reads, 4 * Q.per_wave)), dim3(256), 0, st, Q);
   if (Q.n_long) hipLaunchKernelGGL(finalize_long<true>, dim3((Q.n_long + 3) / 4), dim3(256), 0, st, Q);
   return hipGetLastError() == hipSuccess ? GS_OK : GS_EHIP;
 }

@@ -25,14 +25,13 @@ constexpr int kPairCore = 18;       // bases of a pair-table core: its bytes ans
 // reciprocal of 3.
 __device__ __forceinline__ uint32_t div96(uint32_t i) { return __umulhi(i >> 5, 0xAAAAAAABu) >> 1; }
 
-// n low bits set, n in [0, 32]
-__device__ __forceinline__ uint32_t low_mask(uint32_t n) { return n >= 32 ? 0xFFFFFFFFu : ((1u << n) - 1u); }
-
-// count stored in the entry plus the set bits of positions [0, bit] of the block
+// count stored in the entry plus the set bits of positions [0, bit] of the
+// block (bit < 96): the words below bit's own whole, its own shifted so that
+// the bits above `bit` leave (11 instructions)
 __device__ __forceinline__ uint32_t rank_in_entry(uint4 e, uint32_t bit) {
-  const uint32_t r = bit + 1;  // 1..96 positions counted
-  const uint32_t n1 = r > 32 ? r - 32 : 0, n2 = r > 64 ? r - 64 : 0;
-  return e.x + __popc(e.y & low_mask(r)) + __popc(e.z & low_mask(n1)) + __popc(e.w & low_mask(n2));
+  const bool w1 = bit > 31u, w2 = bit > 63u;
+  const uint32_t own = w2 ? e.w : (w1 ? e.z : e.y);
+  return e.x + __popc(w1 ? e.y : 0u) + __popc(w2 ? e.z : 0u) + __popc(own << (~bit & 31u));
 }
 
 struct DevIndex {
@@ -81,9 +80,13 @@ __device__ __forceinline__ void extend(const DevIndex& X, uint32_t c, uint32_t& 
   const bool have1 = r1 != 0xFFFFFFFFu;
   const uint32_t i1 = have1 ? row_to_idx(r1, X.primary) : 0u;
   const uint32_t b1 = div96(i1);
+  const bool two = have1 && b1 != b2;
   const uint4 e2 = X.occ[(size_t)b2 * 4 + c];
-  uint4 e1 = e2;
-  if (have1 && b1 != b2) e1 = X.occ[(size_t)b1 * 4 + c];
+  uint4 e1 = make_uint4(0, 0, 0, 0);
+  if (two) e1 = X.occ[(size_t)b1 * 4 + c];
+  // opaque: or e2 is waited for, as e1's default, before e1 is loaded
+  asm volatile("" : "+v"(e1.x), "+v"(e1.y), "+v"(e1.z), "+v"(e1.w));
+  if (!two) e1 = e2;
   const uint32_t o2 = rank_in_entry(e2, i2 - b2 * kBlockBases);
   const uint32_t o1 = have1 ? rank_in_entry(e1, i1 - b1 * kBlockBases) : 0u;
   const uint32_t base = X.L2[c];

@@ -45,9 +45,15 @@ namespace {
 // from its first template argument: Nib, uint8_t or uint16_t)
 struct Nib {};
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ uint32_t pick4(uint32_t c, uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3) {
-  return c == 0 ? a0 : (c == 1 ? a1 : (c == 2 ? a2 : a3));
+  const uint32_t lo = c & 1u ? a1 : a0, hi = c & 1u ? a3 : a2;
+  return c & 2u ? hi : lo;
 }
+
+// __ballot without the trip of the predicate through a vector register
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 // workgroups (of four waves) of the helper kernels that take reads or
@@ -171,7 +177,9 @@ seed_persistent(PersistArgs P) {
   };
   const int lane = threadIdx.x & 63;
   const uint32_t k = P.k;
-  const uint32_t L2_0 = P.X.L2[0], L2_1 = P.X.L2[1], L2_2 = P.X.L2[2], L2_3 = P.X.L2[3];
+  // in vector registers: a select between scalar ones becomes branches
+  uint32_t L2_0 = P.X.L2[0], L2_1 = P.X.L2[1], L2_2 = P.X.L2[2], L2_3 = P.X.L2[3];
+  asm volatile("" : "+v"(L2_0), "+v"(L2_1), "+v"(L2_2), "+v"(L2_3));
   const uint32_t primary = P.X.primary;
   const uint64_t n_items = P.n_items;
   const gs::PersistCold* const C = P.cold;
@@ -231,14 +239,15 @@ seed_persistent(PersistArgs P) {
   // an extension may run left of it and then reads the 4-bit codes in
   // device memory (only in segments of long reads: a read held whole has
   // w0 = 0, and its chunks are stored in the slot's form)
+  auto slot_code = [&](int32_t j) __attribute__((always_inline)) -> uint32_t {  // position w0 + j
+    const uint32_t rr = (uint32_t)(LMAX - 1 - j);
+    const uint32_t* cw = reinterpret_cast<const uint32_t*>(lds + sbase + A_BYTES);
+    const uint32_t bad = (cw[CW + (rr >> 5)] >> (rr & 31u)) & 1u;
+    return ((cw[rr >> 4] >> ((rr & 15u) << 1)) & 3u) | (bad << 2);
+  };
   auto code = [&](int32_t i) __attribute__((always_inline)) -> uint32_t {
     const int32_t j = i - w0;
-    if (j >= 0) {
-      const uint32_t rr = (uint32_t)(LMAX - 1 - j);
-      const uint32_t* cw = reinterpret_cast<const uint32_t*>(lds + sbase + A_BYTES);
-      if ((cw[CW + (rr >> 5)] >> (rr & 31u)) & 1u) return 4u;
-      return (cw[rr >> 4] >> ((rr & 15u) << 1)) & 3u;
-    }
+    if (j >= 0) return slot_code(j);
     if constexpr (PLAIN) {
       const uint8_t* bytes = C->bases + C->offs[r];
       return strand ? gs::code_rev(bytes[L - 1 - (uint32_t)i]) : gs::code_fwd(bytes[i]);
@@ -559,8 +568,8 @@ seed_persistent(PersistArgs P) {
   };
   // the lanes that can give work away, if enough lanes are idle to take it
   auto can_give = [&]() __attribute__((always_inline)) -> uint64_t {
-    if ((uint32_t)__popcll(__ballot(!have)) < P.split_idle) return 0;
-    return __ballot(have && work >= P.split_work && e - e_min >= 2 * (int32_t)P.split_tasks);
+    if ((uint32_t)__popcll(ballot(!have)) < P.split_idle) return 0;
+    return ballot(have && work >= P.split_work && e - e_min >= 2 * (int32_t)P.split_tasks);
   };
   // Idle lanes of a wave whose queue is exhausted take work from its busy
   // lanes (why: a launch ended with its slowest items, alone in their waves
@@ -578,7 +587,7 @@ seed_persistent(PersistArgs P) {
   auto take_pieces = [&]() __attribute__((always_inline)) -> uint32_t {
     const uint64_t giving = can_give();
     if (!giving) return 0;
-    const uint64_t idle = __ballot(!have);
+    const uint64_t idle = ballot(!have);
     const uint32_t n_rem = (uint32_t)(e - e_min);  // of a lane that gives
     uint32_t n = min((uint32_t)__popcll(idle), (uint32_t)__popcll(giving));
     uint32_t id0 = 0;
@@ -627,7 +636,7 @@ seed_persistent(PersistArgs P) {
     uint32_t fresh_link = kNone;
     if (!drained) {
       const bool need = !have;
-      const uint64_t needmask = __ballot(need);
+      const uint64_t needmask = ballot(need);
       // refills go in groups: the whole wave runs the refill path (code copy,
       // record clear, first pattern) whenever any lane takes it, so idle lanes
       // wait until refill_group of them are idle or the wave has no work
@@ -654,7 +663,7 @@ seed_persistent(PersistArgs P) {
     }
     if (fresh) begin_item((int32_t)(L - t0), fresh, kind == 2 ? fresh_link : kNone);
     const int op = have && !need_next ? (phase == 0 ? 1 : (phase == 1 ? 2 : phase)) : 0;
-    if (__ballot(have) == 0) {
+    if (ballot(have) == 0) {
       if (drained) break;
       continue;
     }
@@ -717,9 +726,10 @@ seed_persistent(PersistArgs P) {
       ++n_direct;
       ++work;
     }
-    uint4 d1 = make_uint4(0, 0, 0, 0);
+    // both in flight before either is waited for (with d1 as the second's
+    // default the first load was waited for, to be copied, before the second)
+    uint4 d1 = make_uint4(0, 0, 0, 0), d2 = make_uint4(0, 0, 0, 0);
     if (a1) d1 = *a1;
-    uint4 d2 = d1;
     if (a2) d2 = *a2;
     // ops 3 and 5: word `sub`; the pair byte: byte `sub`
     const uint32_t word = pick4(pair_read ? sub >> 2 : sub, d1.x, d1.y, d1.z, d1.w);
@@ -735,7 +745,7 @@ seed_persistent(PersistArgs P) {
     uint32_t run_g = 0;  // positions matched (and recorded) by this lane's comparison
     int run_kind = 0;    // 0: all matched; 1: a mismatch, 3: an N at position x - run_g; 4: pruned there
     if constexpr (!PLAIN) {
-      uint64_t runners = __ballot(op == 4);
+      uint64_t runners = ballot(op == 4);
       while (runners) {
         const int R = __ffsll((unsigned long long)runners) - 1;
         runners &= runners - 1;
@@ -762,9 +772,9 @@ seed_persistent(PersistArgs P) {
           const uint32_t t = tp - (uint32_t)lane;
           tb = (pick4((t >> 4) & 3u, t0, t1, t2, t3) >> ((t & 15u) << 1)) & 3u;
         }
-        const uint64_t bad = __ballot(valid && cc != tb);  // a code above 3 never equals a base
-        const uint64_t nmask = __ballot(valid && cc > 3);
-        const uint64_t prn = __ballot(valid && cc == tb && rec == 1u);
+        const uint64_t bad = ballot(valid && cc != tb);  // a code above 3 never equals a base
+        const uint64_t nmask = ballot(valid && cc > 3);
+        const uint64_t prn = ballot(valid && cc == tb && rec == 1u);
         const uint32_t fb = bad ? (uint32_t)__ffsll((unsigned long long)bad) - 1u : 64u;
         const uint32_t fp = prn ? (uint32_t)__ffsll((unsigned long long)prn) - 1u : 64u;
         uint32_t g = fb < fp ? fb : fp;  // the first event, 64 if none
@@ -924,6 +934,12 @@ seed_persistent(PersistArgs P) {
     // the 3.1 Gbp index 8.2 -> 7.4 ms, 60,000 uneven reads 7.8 -> 7.0 ms,
     // 10,000,000 reads 58.7 -> 57.6 ms (going on down to a quarter of the
     // lanes: 7.7, 6.8 and 58.8; down to three quarters: 7.5, 6.9 and 58.0).
+    // What a step waits for is one memory latency: both entries are in flight
+    // at once, and the record and the next code are read from LDS meanwhile
+    // (one entry after the other, then the record, then the code: 64 reads
+    // on a 100 Mbp index 255 us, with this 161; 1000 uneven reads there 727
+    // -> 628 us, 1,000,000 on the 3.1 Gbp index 7.04 -> 6.5 ms, 60,000 uneven
+    // ones 6.9 -> 6.55 ms).
     for (uint32_t round = 0;; ++round) {
       if (prep) {
         prep = false;
@@ -932,28 +948,35 @@ seed_persistent(PersistArgs P) {
         if (res == 0) try_direct();
       }
       const bool step = have && !need_next && res == 0 && phase == 1;
-      const uint64_t stepping = __ballot(step);
+      const uint64_t stepping = ballot(step);
       if (!stepping) break;
       if (round) {
-        if (2 * __popcll(stepping) < __popcll(__ballot(have))) break;
+        if (2 * __popcll(stepping) < __popcll(ballot(have))) break;
         if (drained && splitting && can_give()) break;
       }
       if (step) {
-        const uint32_t r1 = l - 1u;
-        const bool have1 = r1 != 0xFFFFFFFFu;
+        // rows l - 1 (l >= 1: an interval of a string is never that of the
+        // empty one) and u
         const uint32_t i2 = u - (u >= primary ? 1u : 0u);
         const uint32_t b2 = gs::div96(i2);
-        const uint32_t i1 = have1 ? r1 - (r1 >= primary ? 1u : 0u) : 0u;
+        const uint32_t i1 = l - 1u - (l > primary ? 1u : 0u);
         const uint32_t b1 = gs::div96(i1);
-        const bool two = have1 && b1 != b2;
-        const uint4 d2 = P.X.occ[(size_t)b2 * 4 + cx];
-        uint4 d1 = d2;
-        if (two) d1 = P.X.occ[(size_t)b1 * 4 + cx];
+        const bool two = b1 != b2;
+        const u32x4* const occ = reinterpret_cast<const u32x4*>(P.X.occ) + cx;
+        u32x4 d2 = occ[(size_t)b2 * 4], d1 = {0, 0, 0, 0};
+        // while they are read: the size record at x and the next position's
+        // code (of the window's lowest positions where x lies left of it)
+        const int32_t j = x - w0, jr = j < 0 ? 0 : j, jn = j < 1 ? 0 : j - 1;
+        const uint32_t rec = rec_get(sbase, jr), next = slot_code(jn);
+        if (two) d1 = occ[(size_t)b1 * 4];
+        // opaque: or d2 is waited for, as d1's default, before d1 is loaded
+        asm volatile("" : "+v"(d1));
+        if (!two) d1 = d2;
         n_occ += two ? 2 : 1;
         work += two ? 2 : 1;
         const uint32_t base = pick4(cx, L2_0, L2_1, L2_2, L2_3);
-        const uint32_t nl = base + (have1 ? gs::rank_in_entry(d1, i1 - b1 * gs::kBlockBases) : 0u) + 1u;
-        const uint32_t nu = base + gs::rank_in_entry(d2, i2 - b2 * gs::kBlockBases);
+        const uint32_t nl = base + gs::rank_in_entry(make_uint4(d1.x, d1.y, d1.z, d1.w), i1 - b1 * gs::kBlockBases) + 1u;
+        const uint32_t nu = base + gs::rank_in_entry(make_uint4(d2.x, d2.y, d2.z, d2.w), i2 - b2 * gs::kBlockBases);
         if (nl > nu) {
           res = 2;
         } else {
@@ -961,11 +984,18 @@ seed_persistent(PersistArgs P) {
           l = nl;
           u = nu;
           b = (uint32_t)x;
-          if (prune_at((int32_t)b, u - l + 1u)) {
+          --x;
+          const uint32_t size = nu - nl + 1u, sv = size >= SAT ? SAT : size;
+          if (j >= 0 && size < SAT && rec == sv) {  // as prune_at
             res = 1;
           } else {
-            x = (int32_t)b - 1;
-            prep = true;
+            if (j >= 0) rec_set(sbase, jr, sv);
+            if (j > 0 && next <= 3) {  // as prepare_x
+              cx = next;
+              try_direct();
+            } else {
+              prep = true;
+            }
           }
         }
       }

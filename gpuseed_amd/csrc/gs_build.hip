@@ -43,10 +43,13 @@ inline unsigned grid_for(uint64_t n, unsigned bs) { return (unsigned)((n + bs - 
 
 constexpr int kKeyChars = 21;
 
+// also sets *bad if a code is above 3 (a loop over the codes on the host took
+// 2 ms for 5 Mbp)
 __global__ void make_keys(const uint8_t* __restrict__ T, uint64_t n, uint64_t* __restrict__ keys,
-                          uint32_t* __restrict__ vals) {
+                          uint32_t* __restrict__ vals, uint64_t* __restrict__ bad) {
   const uint64_t i = blockIdx.x * 256ull + threadIdx.x;
   if (i > n) return;
+  if (i < n && T[i] > 3) *bad = 1;
   uint64_t key = 0;
   for (int j = 0; j < kKeyChars; ++j) {
     const uint64_t p = i + j;
@@ -98,10 +101,11 @@ __global__ void find_primary(const uint32_t* __restrict__ sa, uint64_t m, uint32
 
 // bitmaps and per-block counts of the $-removed BWT in 96-base blocks
 __global__ void bwt_blocks96(const uint8_t* __restrict__ T, const uint32_t* __restrict__ sa, uint32_t n,
-                             uint32_t primary, uint64_t nb, uint4* __restrict__ occ,
+                             const uint32_t* __restrict__ d_primary, uint64_t nb, uint4* __restrict__ occ,
                              uint32_t* __restrict__ bcnt) {
   const uint64_t b = blockIdx.x * 256ull + threadIdx.x;
   if (b >= nb) return;
+  const uint32_t primary = *d_primary;
   uint32_t bits[4][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
   uint32_t cnt[4] = {0, 0, 0, 0};
   for (uint32_t q = 0; q < gs::kBlockBases; ++q) {
@@ -118,10 +122,18 @@ __global__ void bwt_blocks96(const uint8_t* __restrict__ T, const uint32_t* __re
   }
 }
 
-__global__ void set_block_counts(const uint32_t* __restrict__ bcnt_scanned, uint64_t nb, uint4* __restrict__ occ) {
+// Counts before each block from one scan over the counts of all four bases
+// (base by base): a base's first value is what the bases before it have in
+// all, L2 of that base.  Thread 0 leaves L2[0..4] in out[0..4].
+__global__ void set_block_counts(const uint32_t* __restrict__ scanned, const uint32_t* __restrict__ bcnt, uint64_t nb,
+                                 uint4* __restrict__ occ, uint32_t* __restrict__ out) {
   const uint64_t b = blockIdx.x * 256ull + threadIdx.x;
   if (b >= nb) return;
-  for (uint32_t c = 0; c < 4; ++c) occ[b * 4 + c].x = bcnt_scanned[c * nb + b];
+  for (uint32_t c = 0; c < 4; ++c) occ[b * 4 + c].x = scanned[c * nb + b] - scanned[c * nb];
+  if (b == 0) {
+    for (uint32_t c = 0; c < 4; ++c) out[c] = scanned[c * nb];
+    out[4] = scanned[4 * nb - 1] + bcnt[4 * nb - 1];
+  }
 }
 
 __global__ void sample_sa(const uint32_t* __restrict__ sa, uint64_t n_sa, uint32_t intv, uint32_t* __restrict__ out) {
@@ -217,19 +229,31 @@ int build_sa(const uint8_t* dT, uint64_t n, hipStream_t st, Dev& D, uint32_t** s
   uint32_t *sa, *rank, *vA, *vB, *rows, *rows2;
   uint8_t* flag;
   uint64_t* d_count;
-  RC(D.alloc(&kA, m));
-  RC(D.alloc(&kB, m));
   RC(D.alloc(&sa, m));
-  RC(D.alloc(&rank, m));
-  RC(D.alloc(&vA, m));
-  RC(D.alloc(&vB, m));
-  RC(D.alloc(&rows, m));
-  RC(D.alloc(&rows2, m));
-  RC(D.alloc(&flag, m));
-  RC(D.alloc(&d_count, 1));
+  // one allocation for the sort's arrays: each one's release took 0.3 ms (5
+  // Mbp), after the sort's 2.7 ms
+  const uint64_t r8 = (8 * m + 255) & ~255ull, r4 = (4 * m + 255) & ~255ull, r1 = (m + 255) & ~255ull;
+  uint8_t* arena;
+  RC(D.alloc(&arena, 2 * r8 + 5 * r4 + r1 + 256));
+  uint8_t* at = arena;
+  auto carve = [&](uint64_t bytes) {
+    uint8_t* q = at;
+    at += bytes;
+    return q;
+  };
+  kA = (uint64_t*)carve(r8);
+  kB = (uint64_t*)carve(r8);
+  rank = (uint32_t*)carve(r4);
+  vA = (uint32_t*)carve(r4);
+  vB = (uint32_t*)carve(r4);
+  rows = (uint32_t*)carve(r4);
+  rows2 = (uint32_t*)carve(r4);
+  flag = carve(r1);
+  d_count = (uint64_t*)carve(256);  // [0] unresolved rows, [1] a code above 3
   Temp tmp;
   const double t0 = wall();
-  hipLaunchKernelGGL(make_keys, dim3(grid_for(m, 256)), dim3(256), 0, st, dT, n, kA, vA);
+  CK(hipMemsetAsync(d_count, 0, 16, st));
+  hipLaunchKernelGGL(make_keys, dim3(grid_for(m, 256)), dim3(256), 0, st, dT, n, kA, vA, d_count + 1);
   {
     rocprim::double_buffer<uint64_t> K(kA, kB);
     rocprim::double_buffer<uint32_t> V(vA, vB);
@@ -260,9 +284,11 @@ int build_sa(const uint8_t* dT, uint64_t n, hipStream_t st, Dev& D, uint32_t** s
     sb = tmp.cap;
     CK(rocprim::select(tmp.p, sb, it, flag, rows, d_count, (size_t)m, st));
   }
-  uint64_t u = 0;
-  CK(hipMemcpyAsync(&u, d_count, 8, hipMemcpyDeviceToHost, st));
+  uint64_t first[2] = {0, 0};
+  CK(hipMemcpyAsync(first, d_count, 16, hipMemcpyDeviceToHost, st));
   CK(hipStreamSynchronize(st));
+  if (first[1]) return GS_EINVAL;
+  uint64_t u = first[0];
   uint64_t H = kKeyChars;
   int rounds = 0;
   while (u > 0) {
@@ -301,15 +327,7 @@ int build_sa(const uint8_t* dT, uint64_t n, hipStream_t st, Dev& D, uint32_t** s
   CK(hipStreamSynchronize(st));
   *t_sort = wall() - t0;
   *rounds_out = rounds;
-  // keep only the suffix array
-  D.release(kA);
-  D.release(kB);
-  D.release(rank);
-  D.release(vA);
-  D.release(vB);
-  D.release(rows);
-  D.release(rows2);
-  D.release(flag);
+  D.release(arena);  // all but the suffix array
   *sa_out = sa;
   return GS_OK;
 }
@@ -389,60 +407,44 @@ extern "C" GS_API int gs_index_build(const uint8_t* codes, uint64_t n, uint32_t 
     Dev D;
     uint8_t* dT;
     if ((rc = D.alloc(&dT, n))) return fail(rc);
-    for (uint64_t i = 0; i < n; ++i)
-      if (codes[i] > 3) return fail(GS_EINVAL);
     if (hipMemcpyAsync(dT, codes, n, hipMemcpyHostToDevice, st) != hipSuccess) return fail(GS_EHIP);
     uint32_t* d_sa = nullptr;
     double t_sort = 0;
     int rounds = 0;
     if ((rc = build_sa(dT, n, st, D, &d_sa, &t_sort, &rounds))) return fail(rc);
     const double t1 = wall();
-    // primary, BWT blocks, counts, L2
-    uint32_t* d_prim;
+    // primary, BWT blocks, counts, L2: no wait before the last of them
     uint32_t* bcnt;
-    uint32_t* bscan;
     const uint64_t nb = X->n_blocks;
-    if ((rc = D.alloc(&d_prim, 1)) || (rc = D.alloc(&bcnt, 4 * nb)) || (rc = D.alloc(&bscan, 4 * nb)))
-      return fail(rc);
+    if ((rc = D.alloc(&bcnt, 8 * nb + 6))) return fail(rc);
+    uint32_t* const bscan = bcnt + 4 * nb;
+    uint32_t* const d_small = bscan + 4 * nb;  // primary, L2[0..4]
     if (hipMalloc(&X->occ, (nb + 1) * 4 * sizeof(uint4)) != hipSuccess) return fail(GS_ENOMEM);
     if (hipMalloc(&X->sa, X->n_sa * sizeof(uint32_t)) != hipSuccess) return fail(GS_ENOMEM);
     X->device_bytes = (nb + 1) * 4 * sizeof(uint4) + X->n_sa * sizeof(uint32_t);
-    hipLaunchKernelGGL(find_primary, dim3(grid_for(n + 1, 256)), dim3(256), 0, st, d_sa, n + 1, d_prim);
-    if (hipMemcpyAsync(&X->primary, d_prim, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-      return fail(GS_EHIP);
-    hipLaunchKernelGGL(bwt_blocks96, dim3(grid_for(nb, 256)), dim3(256), 0, st, dT, d_sa, (uint32_t)n, X->primary,
-                       nb, X->occ, bcnt);
+    hipLaunchKernelGGL(find_primary, dim3(grid_for(n + 1, 256)), dim3(256), 0, st, d_sa, n + 1, d_small);
+    hipLaunchKernelGGL(bwt_blocks96, dim3(grid_for(nb, 256)), dim3(256), 0, st, dT, d_sa, (uint32_t)n, d_small, nb,
+                       X->occ, bcnt);
     if (hipMemsetAsync(X->occ + nb * 4, 0, 4 * sizeof(uint4), st) != hipSuccess) return fail(GS_EHIP);
-    {
-      Temp tmp;
-      for (uint32_t c = 0; c < 4; ++c) {
-        size_t sb = 0;
-        if (rocprim::exclusive_scan(nullptr, sb, bcnt + c * nb, bscan + c * nb, 0u, (size_t)nb,
-                                    rocprim::plus<uint32_t>(), st) != hipSuccess)
-          return fail(GS_EHIP);
-        if ((rc = tmp.ensure(sb))) return fail(rc);
-        sb = tmp.cap;
-        if (rocprim::exclusive_scan(tmp.p, sb, bcnt + c * nb, bscan + c * nb, 0u, (size_t)nb,
-                                    rocprim::plus<uint32_t>(), st) != hipSuccess)
-          return fail(GS_EHIP);
-      }
-    }
-    hipLaunchKernelGGL(set_block_counts, dim3(grid_for(nb, 256)), dim3(256), 0, st, bscan, nb, X->occ);
+    Temp tmp;
+    size_t sb = 0;
+    if (rocprim::exclusive_scan(nullptr, sb, bcnt, bscan, 0u, (size_t)(4 * nb), rocprim::plus<uint32_t>(), st) !=
+        hipSuccess)
+      return fail(GS_EHIP);
+    if ((rc = tmp.ensure(sb))) return fail(rc);
+    sb = tmp.cap;
+    if (rocprim::exclusive_scan(tmp.p, sb, bcnt, bscan, 0u, (size_t)(4 * nb), rocprim::plus<uint32_t>(), st) !=
+        hipSuccess)
+      return fail(GS_EHIP);
+    hipLaunchKernelGGL(set_block_counts, dim3(grid_for(nb, 256)), dim3(256), 0, st, bscan, bcnt, nb, X->occ,
+                       d_small + 1);
     hipLaunchKernelGGL(sample_sa, dim3(grid_for(X->n_sa, 256)), dim3(256), 0, st, d_sa, X->n_sa, sa_intv, X->sa);
-    std::vector<uint32_t> tail(8);
-    if (hipMemcpyAsync(tail.data(), bscan + 0 * nb + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(tail.data() + 1, bscan + 1 * nb + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(tail.data() + 2, bscan + 2 * nb + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(tail.data() + 3, bscan + 3 * nb + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(tail.data() + 4, bcnt + 0 * nb + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(tail.data() + 5, bcnt + 1 * nb + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(tail.data() + 6, bcnt + 2 * nb + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipMemcpyAsync(tail.data() + 7, bcnt + 3 * nb + nb - 1, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
+    uint32_t h_small[6];
+    if (hipMemcpyAsync(h_small, d_small, 24, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
       return fail(GS_EHIP);
-    X->L2[0] = 0;
-    for (uint32_t c = 0; c < 4; ++c) X->L2[c + 1] = X->L2[c] + tail[c] + tail[4 + c];
+    X->primary = h_small[0];
+    for (uint32_t c = 0; c < 5; ++c) X->L2[c] = h_small[1 + c];
     if (X->L2[4] != n) return fail(GS_EINVAL);
     const double t2 = wall();
     if (write_prefix && (rc = write_files(write_prefix, X, d_sa, n, st, D))) return fail(rc);

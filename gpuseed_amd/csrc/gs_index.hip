@@ -6,6 +6,7 @@
 #include <string.h>
 #include <sys/time.h>
 
+#include <algorithm>
 #include <chrono>
 
 #include "gs_internal.h"
@@ -118,21 +119,22 @@ __global__ void repack_occ96(const uint32_t* __restrict__ bwt, uint32_t n, uint6
 
 // One level of the 13-mer table: entries of level i+1 from level i.  Entry p
 // after i characters depends on the low 2i bits of p; character i is applied
-// next; an empty interval is carried unchanged (the break at 2666-2668).
-__global__ void kmer_level(const DevIndex X, const uint2* __restrict__ prev, uint2* __restrict__ next,
-                           uint32_t level, uint64_t first, uint64_t end) {
-  const uint64_t t = first + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-  if (t >= end) return;
-  const uint64_t q = t & ((1ull << (2 * level)) - 1);
-  const uint32_t c = (uint32_t)(t >> (2 * level));
-  uint32_t l = 0, u = X.seq_len;
-  if (level > 0) {
-    const uint2 iv = prev[q];
-    l = iv.x;
-    u = iv.y;
+// next; an empty interval is carried unchanged (the break at 2666-2668).  A
+// thread makes the four entries of one of level i: their occurrence entries
+// share two 64-byte lines, and `prev` may be the last quarter of `next`, whose
+// slots only the thread that read them writes.
+__global__ void kmer_level(const DevIndex X, const uint2* prev, uint2* next, uint32_t level, uint64_t first,
+                           uint64_t end) {
+  const uint64_t q = first + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
+  if (q >= end) return;
+  const uint2 iv = prev[q];
+  uint2 out[4] = {iv, iv, iv, iv};
+  if (iv.x <= iv.y) {
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c) gs::extend(X, c, out[c].x, out[c].y);
   }
-  if (l <= u) gs::extend(X, c, l, u);
-  next[t] = make_uint2(l, u);
+#pragma unroll
+  for (uint32_t c = 0; c < 4; ++c) next[q | ((uint64_t)c << (2 * level))] = out[c];
 }
 
 // Presence bits of one extended-table entry: which of the 64 three-base
@@ -238,6 +240,19 @@ __global__ void pack_text(const uint8_t* __restrict__ text8, uint64_t n, uint32_
   text[w] = v;
 }
 
+// bases [first, first + count) of the packed text, a byte each, four per thread
+__global__ void __launch_bounds__(256) unpack_text(const uint32_t* __restrict__ text, uint64_t first, uint32_t count,
+                                                   uint32_t* __restrict__ out) {
+  const uint32_t i = 4 * (blockIdx.x * 256 + threadIdx.x);
+  if (i >= count) return;
+  uint32_t v = 0;
+  for (uint32_t q = 0; q < 4; ++q) {
+    const uint64_t pos = first + (i + q < count ? i + q : count - 1);
+    v |= ((text[pos >> 4] >> (2 * (pos & 15))) & 3u) << (8 * q);
+  }
+  out[i >> 2] = v;
+}
+
 // Pair table: the 18-base core at text position p (its index: the sum of
 // text[p + 17 - j] * 4^j) gets bit text[p + 18] (a base that follows it) and
 // bit 4 + text[p - 1] (a base that precedes it).  One thread per core; the
@@ -285,10 +300,21 @@ __global__ void tandem_rows(const DevIndex X, uint4* __restrict__ out) {
   }
 }
 
+// The first kKmerFirst levels at once: an entry's characters one after another.
+constexpr uint32_t kKmerFirst = 7;
+__global__ void kmer_first(const DevIndex X, uint2* __restrict__ out) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 1u << (2 * kKmerFirst)) return;
+  uint32_t l = 0, u = X.seq_len;
+  for (uint32_t i = 0; i < kKmerFirst; ++i)
+    if (l <= u) gs::extend(X, (t >> (2 * i)) & 3u, l, u);
+  out[t] = make_uint2(l, u);
+}
+
 inline unsigned grid_for(uint64_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// One table level in launches of at most launch_chunk() work-items (level
-// 16 has 2^32 entries).
+// One table level of 4 * cnt entries in launches of at most launch_chunk()
+// work-items (level 16 has 2^32 entries).
 void launch_level(const DevIndex& D, const uint2* prev, uint2* next, uint32_t level, uint64_t cnt,
                   hipStream_t st) {
   const uint64_t step = gs::launch_chunk();
@@ -317,30 +343,26 @@ void gs::index_acquire(gs_index* X) { X->refs.fetch_add(1, std::memory_order_rel
 
 int gs_build_kmer_table(gs_index* X) {
   const uint64_t full = 1ull << (2 * gs::kPrecalc);
-  uint2 *a = nullptr, *b = nullptr;
   if (hipMalloc(&X->kmer, full * sizeof(uint2)) != hipSuccess) return GS_ENOMEM;
   X->device_bytes += full * sizeof(uint2);
-  if (hipMalloc(&a, (full / 4) * sizeof(uint2)) != hipSuccess) return GS_ENOMEM;
-  if (hipMalloc(&b, (full / 4) * sizeof(uint2)) != hipSuccess) {
-    (void)hipFree(a);
-    return GS_ENOMEM;
-  }
   const DevIndex D = X->dev();
-  const uint2* prev = nullptr;
-  for (uint32_t lev = 0; lev < (uint32_t)gs::kPrecalc; ++lev) {
-    const uint64_t cnt = 1ull << (2 * (lev + 1));
-    uint2* next = lev + 1 == (uint32_t)gs::kPrecalc ? X->kmer : ((lev & 1) ? b : a);
-    launch_level(D, prev, next, lev, cnt, X->stream);
+  // the levels before the last in the table's first and last quarter by
+  // turns, the one before the last in its last (arrays of their own cost 0.9
+  // ms to allocate and release, more than the levels take at 5 Mbp)
+  static_assert(kKmerFirst < (uint32_t)gs::kPrecalc, "the last level is made from one before it");
+  uint2* const quarter[2] = {X->kmer + 3 * (full / 4), X->kmer};
+  uint2* prev = quarter[(gs::kPrecalc - 1 - kKmerFirst) & 1];
+  hipLaunchKernelGGL(kmer_first, dim3(grid_for(1u << (2 * kKmerFirst), 64)), dim3(64), 0, X->stream, D, prev);
+  for (uint32_t lev = kKmerFirst; lev < (uint32_t)gs::kPrecalc; ++lev) {
+    uint2* next = lev + 1 == (uint32_t)gs::kPrecalc ? X->kmer : quarter[(gs::kPrecalc - 2 - lev) & 1];
+    launch_level(D, prev, next, lev, 1ull << (2 * lev), X->stream);
     prev = next;
   }
-  hipError_t e = hipStreamSynchronize(X->stream);
-  (void)hipFree(a);
-  (void)hipFree(b);
-  if (e != hipSuccess) return GS_EHIP;
   // the tandem table (about 21 MB), from the occ entries alone
   const uint64_t tbytes = (uint64_t)gs::kTandemKeys * gs::kTandemRows * sizeof(uint4);
   if (hipMalloc(&X->tandem, tbytes) != hipSuccess) {
     X->tandem = nullptr;
+    (void)hipStreamSynchronize(X->stream);
     return GS_ENOMEM;
   }
   X->device_bytes += tbytes;
@@ -375,9 +397,9 @@ extern "C" GS_API int gs_index_set_kmer_len(gs_index* X, int len) {
   const DevIndex D = X->dev();
   const uint2* prev = X->kmer;
   for (int lev = gs::kPrecalc; lev < len && !rc; ++lev) {
-    const uint64_t cnt = 1ull << (2 * (lev + 1));
+    const uint64_t cnt = 1ull << (2 * lev);
     uint2*& next = levels[lev + 1 - 14];
-    if (hipMalloc(&next, cnt * sizeof(uint2)) != hipSuccess) {
+    if (hipMalloc(&next, 4 * cnt * sizeof(uint2)) != hipSuccess) {
       rc = GS_ENOMEM;
       break;
     }
@@ -614,13 +636,22 @@ extern "C" GS_API int gs_index_read_direct(const gs_index* X, uint32_t first, ui
   if (sa_out) GS_HIP(hipMemcpy(sa_out, X->sa_full + first, (size_t)count * 4, hipMemcpyDeviceToHost));
   if (isa_out) GS_HIP(hipMemcpy(isa_out, X->isa + first, (size_t)count * 4, hipMemcpyDeviceToHost));
   if (text_out && count) {
-    const uint64_t w0 = first >> 4, w1 = ((uint64_t)first + count + 15) >> 4;
-    std::vector<uint32_t> w(w1 - w0);
-    GS_HIP(hipMemcpy(w.data(), X->text + w0, w.size() * 4, hipMemcpyDeviceToHost));
-    for (uint32_t q = 0; q < count; ++q) {
-      const uint64_t pos = (uint64_t)first + q;
-      text_out[q] = (uint8_t)((w[(pos >> 4) - w0] >> (2 * (pos & 15))) & 3u);
+    // bytes from the packed text on the device (on the host, base by base,
+    // 3.5 ms for 5 Mbp), at most 64 M of them at a time
+    const uint32_t step = std::min<uint32_t>(count, 1u << 26);
+    uint32_t* bytes = nullptr;
+    if (hipMalloc(&bytes, (size_t)step + 4) != hipSuccess) return GS_ENOMEM;
+    bool ok = true;
+    for (uint64_t a = 0; ok && a < count; a += step) {
+      const uint32_t m = (uint32_t)std::min<uint64_t>(step, count - a);
+      hipLaunchKernelGGL(unpack_text, dim3(grid_for((m + 3) / 4, 256)), dim3(256), 0, X->stream, X->text,
+                         (uint64_t)first + a, m, bytes);
+      ok = hipGetLastError() == hipSuccess &&
+           hipMemcpyAsync(text_out + a, bytes, m, hipMemcpyDeviceToHost, X->stream) == hipSuccess &&
+           hipStreamSynchronize(X->stream) == hipSuccess;
     }
+    (void)hipFree(bytes);
+    if (!ok) return GS_EHIP;
   }
   return GS_OK;
 }

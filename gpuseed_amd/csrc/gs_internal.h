@@ -117,7 +117,7 @@ struct PersistParams {
   const uint64_t* task_off;
   const uint64_t* items;
   uint64_t n_items;
-  uint32_t n_reads, k, smem, seg_tasks;
+  uint32_t n_reads, n_long, k, smem, seg_tasks;
   uint4* cand;               // same candidate layout as the plain kernel
   uint32_t* nF;
   uint32_t* nR;
@@ -155,7 +155,7 @@ struct JoinParams {
   uint32_t* nF;
   uint32_t* nR;
   uint32_t n_long, k, smem, seg_tasks;
-  uint32_t n_reads, dyn_cap, split_tasks, pad;
+  uint32_t n_reads, dyn_cap;
 };
 
 constexpr uint32_t kSplitStream = 0xFFFFFFFFu;  // nF/nR of a whole-read stream left for join_whole
@@ -168,8 +168,15 @@ constexpr uint32_t kSplitStream = 0xFFFFFFFFu;  // nF/nR of a whole-read stream 
 // 3.1 Gbp index 1.62, 1.61, 1.68, 1.83; task ends 2, 4, 8: 1.42, 1.68, 2.07
 // and 1000 reads there 0.58, 0.85, 0.86.  In a launch of 1,000,000 reads all
 // of 16-32 idle lanes, 16-64 operations and 1-4 task ends gave 7.2-7.5.
+// kSplitTasksLong (launches from the queue, SMEM, some reads in segments):
+// 20,000 uneven reads on the 3.1 Gbp index with 2, 4, 8 and 12 task ends 3.41,
+// 3.26, 3.18, 3.47 ms, 60,000 6.69, 6.56, 6.35, 6.26, in MEM mode 3.88, 4.04,
+// 3.95, 3.96; 500,000 150 bp reads 3.97, 4.03, 4.38, 4.43.  kSplitTasksPlain
+// (a plain task has no shortcuts, and so more steps): with 1, 2 and 4 10,000
+// uneven reads on a 100 Mbp index 2.74, 2.89, 3.42 ms, 300,000 150 bp reads
+// 3.64, 3.66, 3.93.
 constexpr uint32_t kSplitWork = 64;
-constexpr uint32_t kSplitTasks = 2;
+constexpr uint32_t kSplitTasks = 2, kSplitTasksPlain = 1, kSplitTasksLong = 8;
 constexpr uint32_t kSplitIdle = 32;
 constexpr uint32_t kSplitIdleSmall = 24;
 // Pieces a launch can split off (36 bytes each): 8 per item, at least 65,536,

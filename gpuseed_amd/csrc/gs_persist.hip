@@ -117,6 +117,7 @@ struct PersistArgs {
   uint32_t* queue;
   uint64_t n_items;
   uint32_t k, smem, direct_min, dyn_cap, split_work, split_tasks, split_idle, refill_group, take, tandem;
+  uint32_t n_waves;
 };
 
 // Waves per SIMD the register allocation must allow: 4 for the 4-bit
@@ -127,10 +128,9 @@ struct PersistArgs {
 template <typename AT>
 constexpr int kMinWaves = std::is_same<AT, Nib>::value ? 4 : 1;
 
-// PLAIN is the plain kernel (gs_opts.kernel 0): one work item per lane in a
-// launch of as many lanes as items, no queue, and neither pair probes nor
-// direct runs nor tandem jumps.  It reads the batch's bytes instead of packed
-// codes, which its lanes convert as they fill their slots (once per lane).
+// PLAIN is the plain kernel (gs_opts.kernel 0): neither pair probes nor direct
+// runs nor tandem jumps.  It reads the batch's bytes instead of packed codes,
+// which its lanes convert as they fill their slots.
 template <typename AT, int LMAX, int BS, bool PLAIN>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kMinWaves<AT>)))
 seed_persistent(PersistArgs P) {
@@ -644,7 +644,7 @@ seed_persistent(PersistArgs P) {
         uint32_t base, cnt;
         if (P.take) {  // a small launch: this wave's share of the items, once
           cnt = P.take;
-          base = __builtin_amdgcn_readfirstlane((blockIdx.x * BS + threadIdx.x) >> 6) * cnt;
+          base = __builtin_amdgcn_readfirstlane((blockIdx.x * BS + threadIdx.x) >> 6);  // this wave's number
           drained = true;
         } else {
           cnt = (uint32_t)__popcll(needmask);
@@ -654,7 +654,10 @@ seed_persistent(PersistArgs P) {
           drained = (uint64_t)base + cnt >= n_items;
         }
         const uint32_t rank = (uint32_t)__popcll(needmask & ((1ull << lane) - 1ull));
-        const uint64_t it = (uint64_t)base + rank;
+        // A small launch's waves take items n_waves apart: the segments of a
+        // read that crosses a repeat are all slow, and next to each other.
+        uint64_t it = (uint64_t)base + rank;
+        if (P.take) it = base < P.n_waves ? base + (uint64_t)rank * P.n_waves : n_items;
         if (need && rank < cnt && it < n_items) fresh = load_main(it);
       }
     } else if (splitting) {
@@ -1365,6 +1368,7 @@ int launch_t(const gs::PersistParams& P, unsigned grid, hipStream_t st, hipEvent
   A.split_idle = gs::kSplitIdle;
   A.tandem = P.tandem;
   A.take = 0;
+  A.n_waves = 0;
   constexpr uint32_t kWaves = BS / 64;  // per workgroup
   if (P.n_items <= (uint64_t)grid * BS) {
     // Fewer items than lanes: each wave takes its share at once, and only as
@@ -1375,20 +1379,38 @@ int launch_t(const gs::PersistParams& P, unsigned grid, hipStream_t st, hipEvent
     // Kernel time with as many waves as fit against this: 10,000 100 bp reads
     // on a 1 Mbp index 1.05 -> 0.44 ms, 50,000 and 100,000 150 bp reads on a
     // 100 Mbp index 2.75 -> 1.31 and (plain kernel) 4.62 -> 2.05 ms, 60,000
-    // on the 3.1 Gbp index 2.72 -> 1.42 ms.
+    // on the 3.1 Gbp index 2.72 -> 1.42 ms.  A wave's items lie n_waves apart
+    // (next to each other: 3000 uneven reads on a 100 Mbp index 0.99 -> 0.91
+    // ms, 10,000 with the plain kernel 3.4 -> 2.9).  From the queue, with any
+    // number of waves, 3000 uneven reads take 1.06 ms and 100,000 150 bp reads
+    // 1.72 (here 1.65); at 130,000 the two are equal.
     const uint64_t simds = std::max(1u, 4 * compute_units());
     A.take = (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, (P.n_items + simds - 1) / simds));
-    const uint32_t used = (uint32_t)((P.n_items + A.take - 1) / A.take);
-    grid = (used + kWaves - 1) / kWaves;
+    A.n_waves = (uint32_t)((P.n_items + A.take - 1) / A.take);
+    grid = (A.n_waves + kWaves - 1) / kWaves;
     if (!grid) grid = 1;
     A.split_idle = gs::kSplitIdleSmall;
   } else {
+    // More: the waves of a grid that fills the chip take them from the queue,
+    // or half of those waves up to two items per lane and three quarters up to
+    // six.  Memory is saturated by then, more lanes only make each operation
+    // wait longer, and a launch ends with chains of operations; fewer lanes
+    // also leave more items in the queue to even them out.  Kernel ms with
+    // all, three quarters and half of the waves, 3.1 Gbp index: 200,000 reads
+    // of 150 bp (1.5 items per lane) 3.14, 2.64, 2.37; 300,000 3.43, 2.97,
+    // 3.09; 500,000 3.99, 3.93, 4.58; 1,000,000 6.38, 6.76, 8.37; 20,000 uneven
+    // reads (3.7) 3.63, 3.39, 3.58; 60,000 (11) 6.64, 6.73, 7.97.  Plain
+    // kernel, 100 Mbp index, a launch of one item per lane and three quarters:
+    // 300,000 reads 4.7 -> 3.65, 30,000 uneven reads 8.5 -> 5.1.
+    const uint64_t lanes = (uint64_t)grid * BS;
+    if (P.n_items < 2 * lanes)
+      grid = (grid + 1) / 2;
+    else if (P.n_items < 6 * lanes)
+      grid = (3 * grid + 3) / 4;
     if (!A.split_work) A.split_work = gs::kSplitWork;
-    if (PLAIN) {  // one item per lane
-      A.take = 64;
-      grid = (unsigned)((P.n_items + BS - 1) / BS);
-    }
   }
+  if (!A.split_tasks)
+    A.split_tasks = PLAIN ? gs::kSplitTasksPlain : (!A.take && P.n_long && P.smem ? gs::kSplitTasksLong : gs::kSplitTasks);
   if (e0 && hipEventRecord(e0, st) != hipSuccess) return GS_EHIP;
   hipLaunchKernelGGL((seed_persistent<AT, LMAX, BS, PLAIN>), dim3(grid), dim3(BS), 0, st, A);
   if (hipGetLastError() != hipSuccess) return GS_EHIP;

@@ -1659,6 +1659,7 @@ static int enqueue_extension(gs_batch* B, const SeedParams& S, int kernel, unsig
   PP.items = B->items.as<uint64_t>();
   PP.n_items = B->n_items;
   PP.n_reads = S.n_reads;
+  PP.n_long = B->n_long;
   PP.k = S.k;
   PP.smem = S.smem;
   PP.seg_tasks = B->seg_tasks;
@@ -1676,7 +1677,7 @@ static int enqueue_extension(gs_batch* B, const SeedParams& S, int kernel, unsig
   PP.wmeta = B->wmeta.as<uint4>();
   PP.wlink = B->wlink.as<uint32_t>();
   PP.dyn_cap = B->dyn_cap;
-  PP.split_tasks = B->opts.split_tasks ? B->opts.split_tasks : gs::kSplitTasks;
+  PP.split_tasks = B->opts.split_tasks;         // 0: by the launch's size
   PP.split_work = 64u * B->opts.split_work;  // 0: by the launch's size
   // tandem jumps read the index's tandem table
   const bool tandem = B->opts.tandem != 0xFFFF && B->X->tandem;
@@ -1702,8 +1703,6 @@ static int enqueue_extension(gs_batch* B, const SeedParams& S, int kernel, unsig
   J.wlink = PP.wlink;
   J.n_reads = S.n_reads;
   J.dyn_cap = PP.dyn_cap;
-  J.split_tasks = PP.split_tasks;
-  J.pad = 0;
   int rc = GS_OK;
   if (kernel)  // the plain kernel reads the bytes
     rc = gs::launch_pack_codes(S.bases, S.offs, S.lens, PP.code_off, S.n_reads, J.long_reads, B->n_long,

@@ -268,8 +268,8 @@ typedef struct {
                        interval is larger get no positions                      */
   uint32_t batch_bases; /* MEM look-ahead stays inside batches closed at this
                        many bases (seed_gen.cu:2814, 2955); 0 = 1,000,000     */
-  int kernel;       /* 0: plain kernel (the drop-in): one work item per lane, no
-                          pair probes, direct runs or tandem jumps;
+  int kernel;       /* 0: plain kernel (the drop-in): no pair probes, direct
+                          runs or tandem jumps;
                        1: batched persistent kernel, 8-bit size records;
                        2: batched persistent kernel, 16-bit size records;
                        3: batched persistent kernel, 4-bit size records (a
@@ -283,7 +283,9 @@ typedef struct {
                        exhausted, an item that has used split_work memory
                        operations hands half of its task ends to an idle
                        lane of its wave while at least 2 * split_tasks
-                       remain, 1..64 (0 = 2); 0xFFFF: no splitting           */
+                       remain, 1..64 (0: 1 in the plain kernel, 8 where a
+                       large SMEM launch holds reads in segments, else 2);
+                       0xFFFF: no splitting                                  */
   uint16_t split_work;  /* in units of 64 memory operations, 1..0xFFFE (0 = 1,
                        and none in a launch of fewer items than lanes)       */
   uint16_t direct_min;  /* batched kernels on an index with gs_index_set_direct:

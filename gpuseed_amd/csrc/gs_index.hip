@@ -660,6 +660,8 @@ static void free_index(gs_index* X) {
   if (!X) return;
   if (X->work) gs::batch_free(X->work);
   X->work = nullptr;
+  if (X->locate) gs::batch_free(X->locate);
+  X->locate = nullptr;
   (void)hipFree(X->occ);
   (void)hipFree(X->sa);
   (void)hipFree(X->kmer);

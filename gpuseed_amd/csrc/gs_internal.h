@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <mutex>
 #include <utility>
 #include <vector>
 
@@ -45,6 +46,8 @@ struct gs_index {
   double t_read = 0, t_upload = 0, t_repack = 0, t_table = 0, t_sa = 0, t_write = 0, t_ext = 0, t_direct = 0;
   int sa_rounds = 0;
   gs_batch* work = nullptr;  // gs_seed's batch, kept for the next call (its buffers only grow)
+  std::mutex locate_mu;
+  gs_batch* locate = nullptr;  // gs_index_locate's pinned chunks (two of at most 64 MB)
   // Lifetime: the caller's handle holds one reference, every batch and
   // server made on the index one more; gs_index_close drops the caller's
   // and the device structures are freed with the last one, so a batch or

@@ -1,10 +1,11 @@
 // Persistent extension kernel (the batched form of the seeding path).
 //
-// Same stream procedure and output as seed_streams in gs_seed.hip (the plain
-// one-stream-per-lane kernel), restructured for throughput on gfx950:
-//  * a fixed grid that fills the chip; every lane pulls work items from a
-//    device queue (one atomic per wave refill, leader lane + ballot) and
-//    starts the next one as soon as its current one ends;
+// Same stream procedure and output as seed_streams in gs_seed.hip (one stream
+// per lane), restructured for throughput on gfx950:
+//  * a grid that fills the chip, or part of it where there are few items per
+//    lane (launch_t); every lane pulls work items from a device queue (one
+//    atomic per wave refill, leader lane + ballot) and starts the next one as
+//    soon as its current one ends;
 //  * reads are pre-packed to 4-bit codes of both virtual strands by
 //    pack_codes, so a refill is a few 16-byte loads and LDS stores;
 //  * a lane's LDS slot holds its item's codes (4 bits per base) and its size
@@ -32,8 +33,8 @@
 //    settle the SMEM filter at their boundaries, as for the segments of long
 //    reads: pieces are chained in task order.
 //  * a launch of fewer items than lanes gives every wave its share of them
-//    at once (one item per wave at first, if there are fewer than waves) and
-//    splits them from the start.
+//    at once (one item per wave at first, if there are fewer than waves; a
+//    wave's items lie apart) and splits them from the start.
 #include <algorithm>
 #include <type_traits>
 
@@ -575,7 +576,7 @@ seed_persistent(PersistArgs P) {
   // lanes (why: a launch ended with its slowest items, alone in their waves
   // at 2-4 us per operation; 1,000,000 150 bp reads on the 3.1 Gbp index
   // spent 12 of 18 ms so, 64 reads on a 100 Mbp index all of their 2.4 ms;
-  // with this, 7.4 and 0.25 ms): each of the first n busy lanes that have used split_work memory
+  // with this, 7.4 and 0.25 ms, 6.4 and 0.16 with the steps as they are now): each of the first n busy lanes that have used split_work memory
   // operations since they started or last split, and still have at least
   // 2 * split_tasks task ends after the current one, gives the lower half of
   // them to an idle lane, as a piece linked right after its own tasks (ahead

@@ -131,7 +131,14 @@ constexpr int kMinWaves = std::is_same<AT, Nib>::value ? 4 : 1;
 
 // PLAIN is the plain kernel (gs_opts.kernel 0): neither pair probes nor direct
 // runs nor tandem jumps.  It reads the batch's bytes instead of packed codes,
-// which its lanes convert as they fill their slots.
+// which its lanes convert as they fill their slots.  Its size records have 16
+// bits: without those shortcuts only pruning ends the tasks of a read in a
+// repeat, and a record that saturates never prunes.  Whole calls in ms with 4,
+// 8 and 16 bits, 3 Mbp text: 50,000 MEM reads of 150 bp in 30 exact copies
+// 5.6, 1.7, 1.8, in 600 copies 6.2, 5.8, 2.0; 30 reads of 20 kbp in 30 copies
+// 285, 64, 33.  Their slots leave 6 waves per CU where 4 bits leave 16, which
+// costs launches that need them: 100 Mbp index, 100,000 SMEM reads 3.8 -> 4.0
+// ms, 1,000,000 23.0 -> 26.1, 3000 uneven reads 1.96 in both, 30,000 8.5 -> 10.1.
 template <typename AT, int LMAX, int BS, bool PLAIN>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kMinWaves<AT>)))
 seed_persistent(PersistArgs P) {
@@ -221,6 +228,8 @@ seed_persistent(PersistArgs P) {
   int rout = 0;
   uint4* out = nullptr;
   uint32_t gcodes = 0;  // the stream's first 16-byte code chunk (a batch has fewer than 2^32)
+  const uint8_t* bytes = nullptr;  // PLAIN: the read's bytes (kept, not looked up: codes left of the slot wait
+                                   // for one load, not two; 30 reads of 20 kbp in repeats 292 -> 250 ms)
   uint32_t n_table = 0, n_occ = 0, n_direct = 0, n_tandem = 0;  // this lane's memory operations
   // Tandem jumps.  In a stretch [tR, ..) of period tp (code(z) == code(z + tp)
   // <= 3 for z >= tR up to the stretch's end), read[y, e) for tR <= y < e
@@ -250,7 +259,6 @@ seed_persistent(PersistArgs P) {
     const int32_t j = i - w0;
     if (j >= 0) return slot_code(j);
     if constexpr (PLAIN) {
-      const uint8_t* bytes = C->bases + C->offs[r];
       return strand ? gs::code_rev(bytes[L - 1 - (uint32_t)i]) : gs::code_fwd(bytes[i]);
     }
     const uint32_t w = reinterpret_cast<const uint32_t*>(P.codes + gcodes + (uint32_t)(i >> 5))[(i >> 3) & 3];
@@ -520,7 +528,7 @@ seed_persistent(PersistArgs P) {
       cw[CW + q] = v.z;
     };
     if constexpr (PLAIN) {
-      const uint8_t* bytes = C->bases + C->offs[r];
+      bytes = C->bases + C->offs[r];
 #pragma unroll 1
       for (uint32_t c = c0; c < c1; ++c) put(c - c0, slot_chunk(gs::pack_chunk(bytes, L, strand, c)));
     } else {
@@ -608,6 +616,8 @@ seed_persistent(PersistArgs P) {
     const int32_t g_emin = __shfl(e_min, from), g_w0 = __shfl(w0, from);
     const uint32_t g_push = __shfl(n_push, from), g_link = __shfl(link, from), g_codes = __shfl(gcodes, from);
     const uint64_t g_out = __shfl((uint64_t)out, from);
+    uint64_t g_bytes = 0;
+    if constexpr (PLAIN) g_bytes = __shfl((uint64_t)bytes, from);
     if (give) {
       link = id0 + rank;
       e_min += (int32_t)n_push;
@@ -620,6 +630,7 @@ seed_persistent(PersistArgs P) {
     w0 = g_w0;
     gcodes = g_codes;
     out = reinterpret_cast<uint4*>(g_out);
+    if constexpr (PLAIN) bytes = reinterpret_cast<const uint8_t*>(g_bytes);
     link = g_link;
     kind = 2;
     item = id0 + rank;
@@ -1393,21 +1404,23 @@ int launch_t(const gs::PersistParams& P, unsigned grid, hipStream_t st, hipEvent
     A.split_idle = gs::kSplitIdleSmall;
   } else {
     // More: the waves of a grid that fills the chip take them from the queue,
-    // or half of those waves up to two items per lane and three quarters up to
-    // six.  Memory is saturated by then, more lanes only make each operation
-    // wait longer, and a launch ends with chains of operations; fewer lanes
-    // also leave more items in the queue to even them out.  Kernel ms with
-    // all, three quarters and half of the waves, 3.1 Gbp index: 200,000 reads
-    // of 150 bp (1.5 items per lane) 3.14, 2.64, 2.37; 300,000 3.43, 2.97,
-    // 3.09; 500,000 3.99, 3.93, 4.58; 1,000,000 6.38, 6.76, 8.37; 20,000 uneven
-    // reads (3.7) 3.63, 3.39, 3.58; 60,000 (11) 6.64, 6.73, 7.97.  Plain
-    // kernel, 100 Mbp index, a launch of one item per lane and three quarters:
-    // 300,000 reads 4.7 -> 3.65, 30,000 uneven reads 8.5 -> 5.1.
-    const uint64_t lanes = (uint64_t)grid * BS;
+    // but at most 8 per CU up to two items per lane of 16 waves per CU, and at
+    // most 12 up to six.  Memory is saturated by then, more lanes only make
+    // each operation wait longer, and a launch ends with chains of operations;
+    // fewer lanes also leave more items in the queue to even them out.  Kernel
+    // ms with 16, 12 and 8 waves, 3.1 Gbp index: 200,000 reads of 150 bp (1.5
+    // items per lane) 3.14, 2.64, 2.37; 300,000 3.43, 2.97, 3.09; 500,000 3.99,
+    // 3.93, 4.58; 1,000,000 6.38, 6.76, 8.37; 20,000 uneven reads (3.7) 3.63,
+    // 3.39, 3.58; 60,000 (11) 6.64, 6.73, 7.97.  In waves, not in parts of the
+    // grid: wide records leave a CU 10 or 6 waves, of which half is too few
+    // (16 bits, calls on a 100 Mbp index with 3 and with 6 waves: 200,000 reads
+    // 6.5 and 5.7, 3000 uneven reads 2.22 and 1.84).
+    const unsigned cus = std::max(1u, compute_units());
+    const uint64_t lanes = 16ull * 64 * cus;
     if (P.n_items < 2 * lanes)
-      grid = (grid + 1) / 2;
+      grid = std::min(grid, 8 * cus / kWaves);
     else if (P.n_items < 6 * lanes)
-      grid = (3 * grid + 3) / 4;
+      grid = std::min(grid, 12 * cus / kWaves);
     if (!A.split_work) A.split_work = gs::kSplitWork;
   }
   if (!A.split_tasks)
@@ -1460,7 +1473,7 @@ int launch_join(const JoinParams& J, hipStream_t st) {
 // Workgroups that fill every CU at the kernel's occupancy (LDS slots bound it).
 int persistent_grid(int variant, int wg, unsigned* grid) {
   constexpr int L = kPersistLmax;
-  if (variant < 0) return grid_t<Nib, L, 128, true>(grid);
+  if (variant < 0) return grid_t<uint16_t, L, 128, true>(grid);
   switch (variant * 1000 + (wg ? wg : 128)) {
     case 64: return grid_t<uint8_t, L, 64>(grid);
     case 128: return grid_t<uint8_t, L, 128>(grid);
@@ -1480,7 +1493,7 @@ int launch_persistent(const PersistParams& P, int variant, int wg, unsigned grid
   if (!grid) return GS_EINVAL;
   if (!P.counters) return GS_EINVAL;  // its buffer also holds the launch's PersistCold
   constexpr int L = kPersistLmax;
-  if (variant < 0) return launch_t<Nib, L, 128, true>(P, grid, st, e0, e1);
+  if (variant < 0) return launch_t<uint16_t, L, 128, true>(P, grid, st, e0, e1);
   switch (variant * 1000 + (wg ? wg : 128)) {
     case 64: return launch_t<uint8_t, L, 64>(P, grid, st, e0, e1);
     case 128: return launch_t<uint8_t, L, 128>(P, grid, st, e0, e1);

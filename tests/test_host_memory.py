@@ -1,0 +1,81 @@
+"""What the library does where memory is short or refused, and what it
+allocates where it says it allocates nothing.  CPU only: the library runs in a
+child process on a stand-in for the HIP runtime (fake_hip.c) whose kernels do
+nothing, so that calls end without results and only their allocations, copies
+and return codes are looked at."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.join(HERE, "..")
+pytestmark = pytest.mark.skipif(shutil.which("gcc") is None, reason="gcc not found")
+
+PRELUDE = """
+import ctypes as C, sys
+F = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+F.fake_held.restype = F.fake_calls.restype = C.c_uint64
+F.fake_limit.argtypes = [C.c_int, C.c_uint64, C.c_uint64]
+F.fake_chain_rows.argtypes = [C.c_uint64]
+DEVICE, PINNED, ANY = 0, 1, 2**64 - 1
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+import gpuseed_amd as g
+TEXT = 600_000
+
+def index():
+    return g.Index(sys.argv[3])
+
+def reads(n, length):
+    return (np.frombuffer(b"ACGT", np.uint8)[np.random.default_rng(n).integers(0, 4, n * length)].copy(),
+            np.arange(n, dtype=np.uint64) * length, np.full(n, length, np.uint32))
+
+def rc_of(f, *a, **kw):
+    try:
+        f(*a, **kw)
+        return 0
+    except g.GsError as e:
+        return e.rc
+"""
+
+
+@pytest.fixture(scope="module")
+def child(tmp_path_factory):
+    """Runs a program on the stand-in; its output."""
+    d = tmp_path_factory.mktemp("fake")
+    shim = str(d / "libfake_hip.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-pthread", "-I/opt/rocm/include", "-o", shim,
+                    os.path.join(HERE, "fake_hip.c")], check=True, stdout=subprocess.PIPE, stderr=subprocess.PIPE)
+    import gpuseed_amd
+    prefix = str(d / "idx")
+    gpuseed_amd.build_index_host(np.random.default_rng(1).integers(0, 4, 600_000, dtype=np.uint8), 7, prefix)
+
+    def run(program):
+        p = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(program), shim, ROOT, prefix],
+                           stdout=subprocess.PIPE, stderr=subprocess.PIPE, timeout=300)
+        assert p.returncode == 0, p.stderr.decode()[-3000:]
+        return p.stdout.decode().split()
+
+    return run
+
+
+def test_reading_text_needs_no_device_memory(child):
+    """Short ranges allocate nothing; long ones do without where there is none."""
+    out = child("""
+        X = index()
+        F.fake_chain_rows(TEXT + 1)
+        X.set_direct(True)
+        before = F.fake_calls(DEVICE)
+        X.read_text(5, 1000)
+        X.read_direct(0, 100)
+        print(F.fake_calls(DEVICE) - before)
+        F.fake_limit(DEVICE, F.fake_held(DEVICE), ANY)
+        print(rc_of(X.read_text, 0, TEXT), rc_of(X.read_direct, 3, TEXT - 3))
+        print(rc_of(X.set_kmer_len, 13))
+    """)
+    assert out == ["0", "0", "0", "0"]

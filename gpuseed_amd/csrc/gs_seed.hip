@@ -2236,12 +2236,13 @@ constexpr int kNoAllocDevices = 64;
 static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
 
 // Small inputs and results of a call go through pinned memory that is set up
-// with the scratch array (larger ones are copied from and to the caller's
-// arrays), behind the call's totals.
+// with the scratch array, behind the call's totals.  Larger ones, and all of
+// them where that memory could not be had, are copied from and to the caller's
+// arrays.
 constexpr size_t kNoAllocStage = 1u << 20, kNoAllocTotals = 256;
 
 std::mutex g_scratch_mu;
-char* g_scratch_stage[kNoAllocDevices];  // pinned, kNoAllocTotals + kNoAllocStage bytes
+char* g_scratch_stage[kNoAllocDevices];  // pinned, kNoAllocTotals + kNoAllocStage bytes (null: none yet)
 void* g_scratch_ptr[kNoAllocDevices];  // device address of `scratch` on each device (null: not looked up)
 int g_scratch_rc[kNoAllocDevices];     // the lookup's result once it has run
 
@@ -2281,20 +2282,22 @@ inline uint64_t align256(uint64_t v) { return (v + 255) & ~255ull; }
 int gs::noalloc_setup(int device) {
   if (device < 0 || device >= kNoAllocDevices) return GS_EINVAL;
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (g_scratch_ptr[device]) return GS_OK;
-  if (g_scratch_rc[device]) return g_scratch_rc[device];
-  void* p = nullptr;
-  if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) {
-    g_scratch_rc[device] = GS_EHIP;
-    return GS_EHIP;
+  if (!g_scratch_ptr[device]) {
+    if (g_scratch_rc[device]) return g_scratch_rc[device];
+    void* p = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) {
+      g_scratch_rc[device] = GS_EHIP;
+      return GS_EHIP;
+    }
+    g_scratch_ptr[device] = p;
   }
-  void* stage = nullptr;
-  if (hipHostMalloc(&stage, kNoAllocTotals + kNoAllocStage, hipHostMallocDefault) != hipSuccess) {
-    g_scratch_rc[device] = GS_EHIP;
-    return GS_EHIP;
+  if (!g_scratch_stage[device]) {
+    void* stage = nullptr;
+    if (hipHostMalloc(&stage, kNoAllocTotals + kNoAllocStage, hipHostMallocDefault) == hipSuccess)
+      g_scratch_stage[device] = static_cast<char*>(stage);
+    else
+      (void)hipGetLastError();  // calls do without; the next index on the device asks again
   }
-  g_scratch_stage[device] = static_cast<char*>(stage);
-  g_scratch_ptr[device] = p;
   return GS_OK;
 }
 
@@ -2356,9 +2359,8 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
                  o_toff = take(8 * nr1), o_batch = take(4 * nr1), o_cand = take(16 * (2 * tasks + 1)),
                  o_nF = take(4 * nr1), o_nR = take(4 * nr1), o_ns = take(4 * nr1), o_np = take(4 * nr1),
                  o_soff = take(8 * nr1), o_poff = take(8 * nr1), o_spare = take(8 * (nr1 / kScanTile + 2)),
-                 o_tot = take(16) /* unused */, o_queue = take(16), o_counters = take(gs::kCounterBytes + gs::kColdBytes);
+                 o_tot = take(16), o_queue = take(16), o_counters = take(gs::kCounterBytes + gs::kColdBytes);
   (void)o_spare;
-  (void)o_tot;
   const uint64_t common = at;
   const uint64_t o_code_off = take(8 * nr1), o_long = long_scratch ? take(4 * (span + 16)) : 0;
   if (short_batched) {
@@ -2429,10 +2431,13 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
     B.wlink.view(base + o_wlink, 8 * nr1);
     if (n_long) B.seg_link.view(base + o_seg_link, 4 * n_items);
   }
-  uint64_t* const h_tot = reinterpret_cast<uint64_t*>(stage);
-  stage += kNoAllocTotals;
+  // the totals: written to pinned memory by the scan, else copied
+  uint64_t sums[2] = {0, 0};
+  uint64_t* const h_tot = stage ? reinterpret_cast<uint64_t*>(stage) : sums;
   h_tot[0] = h_tot[1] = 0;
-  B.h_tot = h_tot;
+  B.h_tot = stage ? h_tot : reinterpret_cast<uint64_t*>(base + o_tot);
+  const size_t stage_bytes = stage ? kNoAllocStage : 0;
+  if (stage) stage += kNoAllocTotals;
   B.bases.view(base + o_bases, span + 32);
   B.offs.view(base + o_offs, 8 * nr1);
   B.lens.view(base + o_lens, 4 * nr1);
@@ -2458,7 +2463,7 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   in.add(nullptr, B.bases.p, span + sizeof kZeros);
   in.add(nullptr, B.offs.p, 8ull * n);
   in.add(nullptr, B.lens.p, 4ull * n);
-  if (in.total <= kNoAllocStage) {
+  if (in.total <= stage_bytes) {
     if (span) memcpy(stage, bases + lo, span);
     memcpy(stage + span, kZeros, sizeof kZeros);
     if (n) memcpy(stage + in.part[1].at, offsets, 8ull * n);
@@ -2497,6 +2502,7 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   fill_params(&B, S, Q);
   if ((rc = enqueue_extension(&B, S, kernel, pgrid, st))) return rc;
   if ((rc = enqueue_counts(&B, Q, st))) return rc;
+  if (n && !stage) GS_HIP(hipMemcpyAsync(sums, B.h_tot, sizeof sums, hipMemcpyDeviceToHost, st));
   GS_HIP(hipStreamSynchronize(st));
   const uint64_t n_seeds = n ? h_tot[0] : 0, n_pos = n ? h_tot[1] : 0;
   out->n_seeds = n_seeds;
@@ -2520,7 +2526,7 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   P.add(out->read_pos_off, B.poff.p, 8 * nr1);
   P.add(out->seeds, B.seeds.p, sizeof(gs_seed_rec) * n_seeds);
   P.add(out->pos, B.rows.p, 4 * n_pos);
-  const bool staged = P.total <= kNoAllocStage;
+  const bool staged = P.total <= stage_bytes;
   if (staged) {
     if ((rc = P.launch_gather(0, P.total, stage, st))) return rc;
   } else {

@@ -79,3 +79,19 @@ def test_reading_text_needs_no_device_memory(child):
         print(rc_of(X.set_kmer_len, 13))
     """)
     assert out == ["0", "0", "0", "0"]
+
+
+def test_noalloc_does_without_pinned_memory(child):
+    """Its pinned megabyte is refused when the index is opened, then to be had."""
+    out = child("""
+        small, large = reads(20, 150), reads(20000, 150)
+        F.fake_limit(PINNED, ANY, 4096)
+        X = index()
+        for r in (small, large):
+            print(rc_of(g.seed_noalloc, X, r, 100, 100, k=19, smem=True, kernel=3))
+        held = F.fake_held(PINNED)
+        F.fake_limit(PINNED, ANY, ANY)
+        with index() as Y:
+            print(F.fake_held(PINNED) - held >= 1 << 20, rc_of(g.seed_noalloc, X, small, 100, 100, k=19, kernel=0))
+    """)
+    assert out == ["0", "0", "True", "0"]

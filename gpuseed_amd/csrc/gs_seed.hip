@@ -1208,6 +1208,14 @@ static size_t stage_chunk(size_t total) {
   return std::min(total, std::max(kStageChunkMin, std::min(kStageChunk, (total / 4 + 4095) & ~(size_t)4095)));
 }
 
+// B's pinned chunks for `nch` chunks of `ch` bytes; false if there is no pinned
+// memory for them.
+static bool have_chunks(gs_batch* B, size_t ch, size_t nch) {
+  if (!B->st_a.ensure(ch) && (nch < 2 || !B->st_b.ensure(ch))) return true;
+  (void)hipGetLastError();  // not an error of the call
+  return false;
+}
+
 static void destroy_batch(gs_batch* B) {
   if (!B) return;
   free_graph(B);
@@ -1365,10 +1373,10 @@ int gs::batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_
   // at most as many tasks as bases and code chunks as 32-base spans (+1)
   const uint64_t items = 2 * (reads + bases / seg_tasks + 1);
   const uint32_t dyn = gs::piece_cap(items);
-  int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, dyn);
-  if (!rc) {  // the pinned chunks of staged uploads
+  const int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, dyn);
+  if (!rc) {  // the pinned chunks of staged uploads, which do without where there are none
     const size_t up = bases + 12 * reads + 1024, ch = stage_chunk(up);
-    if (B->st_a.ensure(ch) || (ch < up && B->st_b.ensure(ch))) rc = GS_ENOMEM;
+    (void)have_chunks(B, ch, ch < up ? 2 : 1);
   }
   return rc;
 }
@@ -1413,6 +1421,16 @@ struct UploadParts {
     source(p, bytes, to.total);
     to.add(nullptr, device, bytes);
   }
+  // every source by itself, from where it lies
+  bool copy(hipStream_t st) const {
+    bool ok = true;
+    for (const Source& s : from)
+      to.each(s.at, s.at + s.bytes, [&](const FetchParts::Part& p, size_t o, size_t len, size_t at) {
+        ok = ok && hipMemcpyAsync(static_cast<char*>(const_cast<void*>(p.src)) + o, s.p + (at - s.at), len,
+                                  hipMemcpyHostToDevice, st) == hipSuccess;
+      });
+    return ok;
+  }
   // bytes [a, z) of the sources to dst
   void fill(size_t a, size_t z, char* dst) const {
     size_t lo = 0, hi = from.size();  // the first source that ends past a
@@ -1436,13 +1454,14 @@ struct UploadParts {
 // rate.  Up to kScatterMax one launch reads them all (launch_scatter: a call
 // of 10,000 reads 102 -> 70 us); larger ones are copied array by array, which
 // reads host memory faster than that kernel (45 MB: 1.1 ms against 1.4).
+// Without pinned memory the sources are copied from where they lie.
 constexpr size_t kScatterMax = 2u << 20;
 static int staged_upload(gs_batch* B, const UploadParts& U) {
   hipStream_t st = B->stream;
   const size_t total = U.to.total;
   if (!total) return GS_OK;
   const size_t ch = stage_chunk(total), nch = (total + ch - 1) / ch;
-  if (B->st_a.ensure(ch) || (nch > 1 && B->st_b.ensure(ch))) return GS_ENOMEM;
+  if (!have_chunks(B, ch, nch)) return U.copy(st) ? GS_OK : GS_EHIP;
   for (auto& e : B->cev)
     if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return GS_EHIP;
   char* stage[2] = {static_cast<char*>(B->st_a.p), static_cast<char*>(B->st_b.p)};
@@ -1977,12 +1996,18 @@ extern "C" GS_API int gs_batch_replay(gs_batch* B, gs_batch_stats* stats) {
 // of chunk c+1 runs while chunk c is copied out, on several threads when it
 // is large.  Pageable destinations otherwise go through the runtime's own
 // staging at a fraction of the link's rate (and one array after another: a
-// call of 1000 reads waited six times).
+// call of 1000 reads waited six times).  They do where there is no pinned
+// memory; the caller waits for the stream.
 static int staged_d2h(gs_batch* B, const FetchParts& P) {
   if (!P.total) return GS_OK;
   hipStream_t st = B->stream;
   const size_t ch = stage_chunk(P.total), nch = (P.total + ch - 1) / ch;
-  if (B->st_a.ensure(ch) || (nch > 1 && B->st_b.ensure(ch))) return GS_ENOMEM;
+  if (!have_chunks(B, ch, nch)) {
+    for (int i = 0; i < P.n; ++i)
+      if (hipMemcpyAsync(P.part[i].dst, P.part[i].src, P.part[i].bytes, hipMemcpyDeviceToHost, st) != hipSuccess)
+        return GS_EHIP;
+    return GS_OK;
+  }
   for (auto& e : B->cev)
     if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return GS_EHIP;
   char* stage[2] = {static_cast<char*>(B->st_a.p), static_cast<char*>(B->st_b.p)};

@@ -40,6 +40,13 @@ for n, length in ((1, 150), (300, 150), (60, 700), (20000, 150)):
         name = "%d-%d-%d-" % (n, length, smem)
         if what == "noalloc":
             keep(name, g.seed_noalloc(X, reads, **kw))
+        elif what == "seed":
+            keep(name, g.seed(X, arrays=reads, **kw))
+        elif what == "batch":
+            b = g.Batch(X, reads, **kw)
+            b.run()
+            keep(name, b.fetch())
+            b.close()
 print("refused", F.no_pinned_refused() if shim else 0, flush=True)
 np.savez(out, **res)
 X.close()
@@ -70,7 +77,7 @@ def run(setting, what, shim):
     return np.load(out), refused
 
 
-@pytest.mark.parametrize("what", ["noalloc"])
+@pytest.mark.parametrize("what", ["noalloc", "seed", "batch"])
 def test_without_pinned_memory(setting, what):
     want, _ = run(setting, what, "")
     got, refused = run(setting, what, setting[1])

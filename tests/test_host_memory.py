@@ -95,3 +95,20 @@ def test_noalloc_does_without_pinned_memory(child):
             print(F.fake_held(PINNED) - held >= 1 << 20, rc_of(g.seed_noalloc, X, small, 100, 100, k=19, kernel=0))
     """)
     assert out == ["0", "0", "True", "0"]
+
+
+def test_batches_do_without_pinned_memory(child):
+    """Calls, batches and servers, of one chunk and of several."""
+    out = child("""
+        F.fake_limit(PINNED, ANY, 4096)
+        X = index()
+        for r in (reads(1, 150), reads(20, 150), reads(100_000, 150)):
+            print(rc_of(g.seed, X, arrays=r, k=19, smem=True, kernel=3))
+            b = g.Batch(X, r, k=19, smem=False, batch_bases=1000)
+            b.run()
+            print(len(b.fetch().pos))
+            b.close()
+        g.Server(X, k=19, round_bases=100_000).close()
+        print(F.fake_held(PINNED) < 8192)
+    """)
+    assert out == ["0"] * 6 + ["True"]

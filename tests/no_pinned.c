@@ -12,7 +12,9 @@ void no_pinned_limit(size_t bytes) { limit = bytes; }
 int no_pinned_refused(void) { return refused; }
 
 hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) {
-  hipError_t (*real)(void**, size_t, unsigned) = dlsym(RTLD_NEXT, "hipHostMalloc");
+  static hipError_t (*real)(void**, size_t, unsigned);
+  Dl_info hip;  /* the runtime's library, found by another of its functions */
+  if (!real && dladdr((void*)hipHostFree, &hip)) real = dlsym(dlopen(hip.dli_fname, RTLD_LAZY), "hipHostMalloc");
   if (n > limit || !real) {
     ++refused;
     return hipErrorOutOfMemory;

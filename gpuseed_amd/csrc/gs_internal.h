@@ -47,7 +47,7 @@ struct gs_index {
   int sa_rounds = 0;
   gs_batch* work = nullptr;  // gs_seed's batch, kept for the next call (its buffers only grow)
   std::mutex locate_mu;
-  gs_batch* locate = nullptr;  // gs_index_locate's pinned chunks (two of at most 64 MB)
+  gs_batch* locate = nullptr;  // gs_index_locate's pinned chunks (two of at most 80 MB)
   // Lifetime: the caller's handle holds one reference, every batch and
   // server made on the index one more; gs_index_close drops the caller's
   // and the device structures are freed with the last one, so a batch or

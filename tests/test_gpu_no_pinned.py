@@ -40,6 +40,8 @@ for n, length in ((1, 150), (300, 150), (60, 700), (20000, 150)):
         name = "%d-%d-%d-" % (n, length, smem)
         if what == "noalloc":
             keep(name, g.seed_noalloc(X, reads, **kw))
+        elif what == "locate":
+            res[name + "pos"] = X.locate(rng.integers(0, len(codes) + 3, n * length, dtype=np.uint32))
         elif what == "seed":
             keep(name, g.seed(X, arrays=reads, **kw))
         elif what == "batch":
@@ -77,7 +79,7 @@ def run(setting, what, shim):
     return np.load(out), refused
 
 
-@pytest.mark.parametrize("what", ["noalloc", "seed", "batch"])
+@pytest.mark.parametrize("what", ["noalloc", "seed", "batch", "locate"])
 def test_without_pinned_memory(setting, what):
     want, _ = run(setting, what, "")
     got, refused = run(setting, what, setting[1])

@@ -112,3 +112,15 @@ def test_batches_do_without_pinned_memory(child):
         print(F.fake_held(PINNED) < 8192)
     """)
     assert out == ["0"] * 6 + ["True"]
+
+
+def test_locate_does_without_pinned_memory(child):
+    out = child("""
+        F.fake_limit(PINNED, ANY, 1024)
+        X = index()
+        for n in (1, 1000, 5_000_000):
+            rows = np.arange(n, dtype=np.uint32)
+            print(rc_of(X.locate, rows))
+        print(np.array_equal(X.locate(rows), rows))
+    """)
+    assert out == ["0", "0", "0", "True"]

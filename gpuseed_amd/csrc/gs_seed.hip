@@ -2142,7 +2142,9 @@ int gs_batch_set_tuning(gs_batch* B, int kernel, int wg, int walk_rows) {
 // of a 100 Mbp index 2.53 -> 1.29 ms, of which walks 0.67).  Calls on one index
 // follow each other, as their walks did on its stream before (8 threads, 5
 // calls of 1,000,000 rows each: 24.0 -> 18.1 ms in all).  Without pinned
-// memory the rows are copied to a device buffer and back.
+// memory the rows are copied to a device buffer and back; so they are where
+// `out` starts inside the rows, whose later chunks its first ones would
+// overwrite before they are read.
 extern "C" GS_API int gs_index_locate(gs_index* X, const uint32_t* rows, uint64_t n, uint32_t* out) {
   if (!X || (n && (!rows || !out))) return GS_EINVAL;
   if (!n) return GS_OK;
@@ -2152,7 +2154,8 @@ extern "C" GS_API int gs_index_locate(gs_index* X, const uint32_t* rows, uint64_
   gs_batch* B = X->locate;  // only its pinned chunks and their events
   const size_t total = 4 * n, ch = stage_chunk(total);
   const uint64_t nch = (total + ch - 1) / ch;
-  if (!have_chunks(B, ch, nch)) {
+  const uintptr_t r0 = (uintptr_t)rows, o0 = (uintptr_t)out;
+  if ((o0 > r0 && o0 - r0 < total) || !have_chunks(B, ch, nch)) {
     uint32_t* d = nullptr;
     if (hipMalloc(&d, total) != hipSuccess) return GS_ENOMEM;
     bool ok = hipMemcpyAsync(d, rows, total, hipMemcpyHostToDevice, X->stream) == hipSuccess;

@@ -124,3 +124,19 @@ def test_locate_does_without_pinned_memory(child):
         print(np.array_equal(X.locate(rows), rows))
     """)
     assert out == ["0", "0", "0", "True"]
+
+
+@pytest.mark.parametrize("shift", [1, 2_097_152, 3_000_000, 5_000_000, -1, -3_000_000])
+def test_locate_where_rows_and_positions_overlap(child, shift):
+    """The stand-in's walks leave the rows as they are."""
+    out = child("""
+        shift, n = %d, 9_000_000
+        X = index()
+        both = np.arange(n + abs(shift), dtype=np.uint32)
+        rows, at = both[max(0, -shift):][:n], both[max(0, shift):][:n]
+        want = rows.copy()
+        u32 = C.POINTER(C.c_uint32)
+        print(g.lib().gs_index_locate(X.h, rows.ctypes.data_as(u32), n, at.ctypes.data_as(u32)))
+        print(np.array_equal(at, want))
+    """ % shift)
+    assert out == ["0", "True"]

@@ -230,26 +230,35 @@ int build_sa(const uint8_t* dT, uint64_t n, hipStream_t st, Dev& D, uint32_t** s
   uint8_t* flag;
   uint64_t* d_count;
   RC(D.alloc(&sa, m));
-  // one allocation for the sort's arrays: each one's release took 0.3 ms (5
-  // Mbp), after the sort's 2.7 ms
+  // one allocation for the sort's arrays (each one's release took 0.3 ms at 5
+  // Mbp, after the sort's 2.7 ms), or one each where there is no block for all
   const uint64_t r8 = (8 * m + 255) & ~255ull, r4 = (4 * m + 255) & ~255ull, r1 = (m + 255) & ~255ull;
-  uint8_t* arena;
-  RC(D.alloc(&arena, 2 * r8 + 5 * r4 + r1 + 256));
+  uint8_t* arena = nullptr;
+  if (D.alloc(&arena, 2 * r8 + 5 * r4 + r1 + 256)) {
+    (void)hipGetLastError();  // not an error of the build
+    arena = nullptr;
+  }
+  uint8_t* arrays[9];
+  int n_arrays = 0;
   uint8_t* at = arena;
-  auto carve = [&](uint64_t bytes) {
-    uint8_t* q = at;
-    at += bytes;
-    return q;
-  };
-  kA = (uint64_t*)carve(r8);
-  kB = (uint64_t*)carve(r8);
-  rank = (uint32_t*)carve(r4);
-  vA = (uint32_t*)carve(r4);
-  vB = (uint32_t*)carve(r4);
-  rows = (uint32_t*)carve(r4);
-  rows2 = (uint32_t*)carve(r4);
-  flag = carve(r1);
-  d_count = (uint64_t*)carve(256);  // [0] unresolved rows, [1] a code above 3
+  for (uint64_t bytes : {r8, r8, r4, r4, r4, r4, r4, r1, (uint64_t)256}) {
+    uint8_t*& q = arrays[n_arrays++];
+    if (arena) {
+      q = at;
+      at += bytes;
+    } else {
+      RC(D.alloc(&q, bytes));
+    }
+  }
+  kA = (uint64_t*)arrays[0];
+  kB = (uint64_t*)arrays[1];
+  rank = (uint32_t*)arrays[2];
+  vA = (uint32_t*)arrays[3];
+  vB = (uint32_t*)arrays[4];
+  rows = (uint32_t*)arrays[5];
+  rows2 = (uint32_t*)arrays[6];
+  flag = arrays[7];
+  d_count = (uint64_t*)arrays[8];  // [0] unresolved rows, [1] a code above 3
   Temp tmp;
   const double t0 = wall();
   CK(hipMemsetAsync(d_count, 0, 16, st));
@@ -327,7 +336,11 @@ int build_sa(const uint8_t* dT, uint64_t n, hipStream_t st, Dev& D, uint32_t** s
   CK(hipStreamSynchronize(st));
   *t_sort = wall() - t0;
   *rounds_out = rounds;
-  D.release(arena);  // all but the suffix array
+  // keep only the suffix array
+  if (arena)
+    D.release(arena);
+  else
+    for (uint8_t* q : arrays) D.release(q);
   *sa_out = sa;
   return GS_OK;
 }

@@ -1,6 +1,7 @@
 """Calls on a device whose host refuses pinned memory beyond a page: they
-copy from and to the caller's arrays instead.  Exact, against the same calls in
-a process that has it."""
+copy from and to the caller's arrays instead; and a build that gets no block
+for all of its sort's arrays.  Exact, against the same calls in a process that
+has the memory."""
 import os
 import shutil
 import subprocess
@@ -19,7 +20,10 @@ shim, root, prefix, what, out = sys.argv[1:]
 if shim:
     F = C.CDLL(shim, mode=C.RTLD_GLOBAL)
     F.no_pinned_limit.argtypes = [C.c_size_t]
-    F.no_pinned_limit(4096)
+    F.no_device_between.argtypes = [C.c_size_t, C.c_size_t]
+    F.no_pinned_limit(4096 if what != "build" else 1 << 40)
+    if what == "build":
+        F.no_device_between(5_000_000, 15_000_000)  # the sort's arrays together: 11.1 MB, the largest 2.4
 sys.path.insert(0, root)
 import numpy as np
 import gpuseed_amd as g
@@ -29,7 +33,13 @@ res = {}
 def keep(name, r):
     res.update({name + k: getattr(r, k) for k in ("read_nseeds", "read_npos", "read_seed_off", "read_pos_off", "pos")})
     res[name + "seeds"] = r.seeds.view(np.uint32)
-X = g.Index(prefix)
+if what == "build":
+    X = g.Index(codes=np.concatenate([codes[:150_000], codes[:150_000]]), sa_intv=7)
+    X.set_direct(True)
+    res["occ"] = X.read_occ(0, X.info().n_blocks)
+    res["sa"], res["isa"], res["pos"] = X.read_direct(0, 300_000)
+else:
+    X = g.Index(prefix)
 for n, length in ((1, 150), (300, 150), (60, 700), (20000, 150)):
     at = rng.integers(0, len(codes) - length, n)
     buf = np.frombuffer(b"ACGT", np.uint8)[codes[at[:, None] + np.arange(length)]].reshape(-1).copy()
@@ -79,7 +89,7 @@ def run(setting, what, shim):
     return np.load(out), refused
 
 
-@pytest.mark.parametrize("what", ["noalloc", "seed", "batch", "locate"])
+@pytest.mark.parametrize("what", ["noalloc", "seed", "batch", "locate", "build"])
 def test_without_pinned_memory(setting, what):
     want, _ = run(setting, what, "")
     got, refused = run(setting, what, setting[1])

@@ -140,3 +140,18 @@ def test_locate_where_rows_and_positions_overlap(child, shift):
         print(np.array_equal(at, want))
     """ % shift)
     assert out == ["0", "True"]
+
+
+def test_build_takes_its_sort_arrays_in_pieces(child):
+    """No block of the sort's 37 bytes per base can be had, but smaller ones
+    can.  The stand-in sorts nothing, so the build fails later on, with an
+    index that does not fit its text."""
+    out = child("""
+        codes = np.zeros(1_000_000, np.uint8)
+        print(rc_of(g.Index, codes=codes) == g.GS_EINVAL)
+        F.fake_limit(DEVICE, ANY, 20_000_000)
+        print(rc_of(g.Index, codes=codes) == g.GS_EINVAL)
+        F.fake_limit(DEVICE, 20_000_000, ANY)
+        print(rc_of(g.Index, codes=codes) == -2, F.fake_held(DEVICE))
+    """)
+    assert out == ["True", "True", "True", "0"]

@@ -990,9 +990,12 @@ struct DevBuf {
   T* as() const {
     return reinterpret_cast<T*>(p);
   }
-  ~DevBuf() {
+  void release() {
     if (p && own) (void)hipFree(p);
+    p = nullptr;
+    cap = 0;
   }
+  ~DevBuf() { release(); }
 };
 
 inline uint64_t scan_ntiles(uint64_t n) { return (n + kScanTile - 1) / kScanTile; }
@@ -1365,6 +1368,17 @@ static int ensure_buffers(gs_batch* B, uint64_t span, uint64_t n, uint64_t tasks
   return GS_OK;
 }
 
+// Where the device has no room for the pieces of work splitting, the batch
+// runs without it, as with split_tasks 0xFFFF (large batches did without by
+// default once, so a batch that fitted then still does).
+static bool give_up_splitting(gs_batch* B) {
+  if (!B->dyn_cap) return false;
+  (void)hipGetLastError();  // not an error of the call
+  B->dyn_cap = 0;
+  for (auto* b : {&B->dyn_items, &B->dyn_meta, &B->dyn_link, &B->wmeta, &B->wlink}) b->release();
+  return true;
+}
+
 int gs::batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_tasks) {
   if (!B) return GS_EINVAL;
   if (hipSetDevice(B->X->device) != hipSuccess) return GS_EHIP;
@@ -1533,8 +1547,8 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P, bool wait) {
   const uint64_t n = P.n_reads;
   const bool split_on = P.opts.split_tasks != 0xFFFF;
   B->dyn_cap = split_on ? gs::piece_cap(B->n_items) : 0u;
-  if (ensure_buffers(B, B->span, n, B->tasks, B->code_chunks, B->n_items, B->n_long, B->dyn_cap))
-    return GS_ENOMEM;
+  while (ensure_buffers(B, B->span, n, B->tasks, B->code_chunks, B->n_items, B->n_long, B->dyn_cap))
+    if (!give_up_splitting(B)) return GS_ENOMEM;
   hipStream_t st = B->stream;
   if (hipEventRecord(B->lev[0], st) != hipSuccess) return GS_EHIP;
   const bool one = P.offs.empty();
@@ -1806,8 +1820,10 @@ static int run_pipeline(gs_batch* B, int kernel, bool kev) {
   B->n_seeds = B->h_tot[0];
   B->n_pos = B->h_tot[1];
   const void *seeds0 = B->seeds.p, *rows0 = B->rows.p;
-  if (B->seeds.ensure(sizeof(gs_seed_rec) * (B->n_seeds + 1)) || B->rows.ensure(4 * (B->n_pos + 1)))
-    return GS_ENOMEM;
+  while (B->seeds.ensure(sizeof(gs_seed_rec) * (B->n_seeds + 1)) || B->rows.ensure(4 * (B->n_pos + 1))) {
+    if (!give_up_splitting(B)) return GS_ENOMEM;
+    free_graph(B);  // it splits
+  }
   if (B->graph && (B->seeds.p != seeds0 || B->rows.p != rows0)) free_graph(B);  // it wrote the old buffers
   fill_params(B, S, Q);
   GS_HIP(hipEventRecord(B->ev[3], st));

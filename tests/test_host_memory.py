@@ -155,3 +155,36 @@ def test_build_takes_its_sort_arrays_in_pieces(child):
         print(rc_of(g.Index, codes=codes) == -2, F.fake_held(DEVICE))
     """)
     assert out == ["True", "True", "True", "0"]
+
+
+def test_batches_do_without_room_for_split_off_pieces(child):
+    """No room for the pieces when the batch is made, or for its results
+    beside them."""
+    out = child("""
+        X = index()
+        r = reads(50_000, 150)
+        start = F.fake_held(DEVICE)
+        def made(limit, **kw):
+            F.fake_limit(DEVICE, limit, ANY)
+            rc, held = 0, 0
+            try:
+                b = g.Batch(X, r, k=19, **kw)
+                held = F.fake_held(DEVICE) - start
+                b.run()
+                b.run()
+                b.fetch()
+                b.close()
+            except g.GsError as e:
+                rc = e.rc
+            return rc, held
+        rc, bare = made(ANY, split_tasks=g.NO_SPLIT)
+        rc2, full = made(ANY)
+        print(rc, rc2, full > bare + 2_000_000)
+        room = 2048  # for the results, which are empty here
+        for limit in (bare + room, bare + 1_000_000, (bare + full) // 2, full - 1, full):
+            rc, held = made(start + limit)
+            print(rc, held <= limit)
+        rc, _ = made(start + bare // 2)
+        print(rc)
+    """)
+    assert out == ["0", "0", "True"] + ["0", "True"] * 5 + ["-2"]

@@ -1387,7 +1387,9 @@ int gs::batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_
   // at most as many tasks as bases and code chunks as 32-base spans (+1)
   const uint64_t items = 2 * (reads + bases / seg_tasks + 1);
   const uint32_t dyn = gs::piece_cap(items);
-  const int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, dyn);
+  int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, dyn);
+  // MEM: the first reads of the reference batches, at most every read
+  if (!rc && B->cuts.ensure(4 * (reads + 1))) rc = GS_ENOMEM;
   if (!rc) {  // the pinned chunks of staged uploads, which do without where there are none
     const size_t up = bases + 12 * reads + 1024, ch = stage_chunk(up);
     (void)have_chunks(B, ch, ch < up ? 2 : 1);

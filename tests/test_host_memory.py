@@ -188,3 +188,19 @@ def test_batches_do_without_room_for_split_off_pieces(child):
         print(rc)
     """)
     assert out == ["0", "0", "True"] + ["0", "True"] * 5 + ["-2"]
+
+
+def test_served_mem_rounds_allocate_no_more_than_smem_rounds(child):
+    """More reference batches than the plan's launch holds: their list has its
+    room from the start, as everything else but the results."""
+    out = child("""
+        X = index()
+        r = reads(2000, 150)
+        for smem in (True, False):
+            with g.Server(X, k=19, smem=smem, batch_bases=1000, round_bases=1_000_000, workers=1) as S:
+                before = F.fake_calls(DEVICE)
+                for _ in range(3):
+                    S.wait(S.submit(r))
+                print(F.fake_calls(DEVICE) - before)
+    """)
+    assert out == ["2", "2"]  # seed records and rows

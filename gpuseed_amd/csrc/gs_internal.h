@@ -223,6 +223,35 @@ __host__ __device__ inline uint32_t n_segments(uint32_t L, uint32_t k, uint32_t 
   return (ntask + seg_tasks - 1) / seg_tasks;
 }
 
+__host__ __device__ __forceinline__ bool read_is_long(uint32_t L, uint32_t k, uint32_t nseg) {
+  return nseg > 1 || (L > kPersistLmax && L >= k);
+}
+
+// What the reads of a batch need, added up read by read.
+struct ReadSums {
+  uint64_t tasks = 0, chunks = 0, whole = 0, items = 0, n_long = 0;  // items: those of long reads' segments
+  void add(uint32_t L, uint32_t k, uint32_t seg_tasks) {
+    tasks += L >= k ? L - k + 1 : 0;
+    chunks += 2 * (uint64_t)((L + 31ull) / 32);
+    const uint32_t nseg = n_segments(L, k, seg_tasks);
+    if (read_is_long(L, k, nseg)) {
+      ++n_long;
+      items += 2ull * nseg;
+    } else {
+      whole += 2ull * nseg;
+    }
+  }
+};
+
+// The sizes that a batch's device buffers follow from: bytes of its reads,
+// reads, task slots per strand, 16-byte code chunks, work items, reads in
+// segments, reference batches that need a list, room for split-off pieces.
+struct BatchSizes {
+  uint64_t span, n, tasks, chunks, items, n_long, cuts;
+  uint32_t dyn_cap;
+};
+uint64_t batch_bytes(const BatchSizes& z);  // all of them, outputs excluded
+
 int launch_pack_codes(const uint8_t* bases, const uint64_t* offs, const uint32_t* lens, const uint64_t* code_off,
                       uint32_t n_reads, const uint32_t* long_reads, uint32_t n_long, uint4* codes, hipStream_t st);
 // variant -1: the plain kernel (wg ignored), 0: 8-bit size records, 1: 16-bit

@@ -826,10 +826,6 @@ __global__ void zero_bytes(uint8_t* __restrict__ p, uint32_t n) {
 // segment at most seg_tasks, so the last items a persistent kernel hands
 // out are the small ones.
 
-__host__ __device__ __forceinline__ bool read_is_long(uint32_t L, uint32_t k, uint32_t nseg) {
-  return nseg > 1 || (L > gs::kPersistLmax && L >= k);
-}
-
 // The rest of a batch's plan, from the reads' lengths: task and code-chunk
 // offsets, the reads' offsets rebased onto the uploaded bytes, the
 // reference-batch ids that MEM's row skip needs, and the work items (null
@@ -866,7 +862,7 @@ __device__ __forceinline__ bool plan_counts(const PlanParams& P, uint64_t i, uin
   if (i >= P.n) return false;
   L = P.lens[i];
   const uint32_t nseg = gs::n_segments(L, P.k, P.seg_tasks);
-  const bool lng = read_is_long(L, P.k, nseg);
+  const bool lng = gs::read_is_long(L, P.k, nseg);
   c[0] = L >= P.k ? L - P.k + 1 : 0u;
   c[1] = 2u * (L / 32u + (L % 32u ? 1u : 0u));
   c[lng ? 3 : 2] = 2u * nseg;
@@ -1279,7 +1275,8 @@ int gs::plan_add(BatchPlan& P, const char* bases, const uint64_t* offsets, const
   const uint32_t batch_bases = P.opts.batch_bases ? P.opts.batch_bases : 1000000u;
   // a group starts a reference batch of its own
   if (P.n_reads) P.cuts.push_back((uint32_t)P.n_reads);
-  uint64_t lo = UINT64_MAX, hi = 0, acc = 0, tasks = 0, chunks = 0, whole = 0, items = 0, n_long = 0;
+  uint64_t lo = UINT64_MAX, hi = 0, acc = 0;
+  ReadSums sum;
   bool closed = false;  // the read before this one closed its reference batch
   for (uint64_t i = r0; i < r1; ++i) {
     const uint32_t L = lens[i];
@@ -1289,26 +1286,18 @@ int gs::plan_add(BatchPlan& P, const char* bases, const uint64_t* offsets, const
     if (closed) acc = 0;
     lo = std::min(lo, offsets[i]);
     hi = std::max(hi, offsets[i] + L);
-    tasks += L >= k ? L - k + 1 : 0;
-    chunks += 2 * (uint64_t)((L + 31ull) / 32);
-    const uint32_t nseg = gs::n_segments(L, k, P.seg_tasks);
-    if (read_is_long(L, k, nseg)) {
-      ++n_long;
-      items += 2ull * nseg;
-    } else {
-      whole += 2ull * nseg;
-    }
+    sum.add(L, k, P.seg_tasks);
   }
   if (hi < lo) lo = hi = 0;
   if (hi > lo) P.pieces.push_back({bases + lo, hi - lo});
   P.groups.push_back({offsets + r0, lens + r0, r1 - r0, lo, P.span});
   P.span += hi - lo;
   P.n_reads += r1 - r0;
-  P.tasks += tasks;
-  P.code_chunks += chunks;
-  P.n_whole += whole;
-  P.n_items += whole + items;
-  P.n_long += n_long;
+  P.tasks += sum.tasks;
+  P.code_chunks += sum.chunks;
+  P.n_whole += sum.whole;
+  P.n_items += sum.whole + sum.items;
+  P.n_long += sum.n_long;
   return P.n_items > 0xF0000000ull ? GS_ERANGE : GS_OK;
 }
 
@@ -1326,11 +1315,13 @@ void gs::plan_finish(BatchPlan& P, bool copy) {
   }
 }
 
-uint64_t gs::plan_device_bytes(const BatchPlan& P) {
-  const uint64_t nr1 = P.n_reads + 1;
-  return (P.span + 32) + 16 * (P.code_chunks + 1) + 16 * (2 * P.tasks + 1) + 8 * P.n_items +
-         (P.n_long ? 16 * P.n_items : 0) + 12 * P.n_long + nr1 * (8 * 5 + 4 * 7);
+static gs::BatchSizes plan_sizes(const gs::BatchPlan& P) {
+  const bool list = !P.opts.smem && P.cuts.size() > kInlineCuts;
+  return {P.span, P.n_reads, P.tasks, P.code_chunks, P.n_items, P.n_long, list ? P.cuts.size() : 0,
+          P.opts.split_tasks != 0xFFFF ? gs::piece_cap(P.n_items) : 0u};
 }
+
+uint64_t gs::plan_device_bytes(const BatchPlan& P) { return batch_bytes(plan_sizes(P)); }
 
 static int batch_events(gs_batch* B) {
   if (!B->stream && hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking) != hipSuccess) return GS_EHIP;
@@ -1346,26 +1337,61 @@ static int batch_events(gs_batch* B) {
   return GS_OK;
 }
 
-// Device buffers of a batch of `span` bases, n reads, `tasks` task slots per
-// strand, `code_chunks` 16-byte code chunks, n_items work items (n_long of
-// them long reads) and room for dyn_cap split-off pieces; buffers only grow.
-static int ensure_buffers(gs_batch* B, uint64_t span, uint64_t n, uint64_t tasks, uint64_t code_chunks,
-                          uint64_t n_items, uint64_t n_long, uint32_t dyn_cap) {
-  const uint64_t nr1 = n + 1;
-  if (B->codes.ensure(16 * (code_chunks + 1)) || B->code_off.ensure(8 * nr1) ||
-      B->items.ensure(8 * (n_items + 1)) || B->long_reads.ensure(4 * (n_long + 1)) ||
-      B->item0.ensure(8 * (n_long + 1)) || B->seg_meta.ensure(n_long ? 16 * n_items : 16) ||
-      B->bases.ensure(span + 32) || B->offs.ensure(8 * nr1) || B->lens.ensure(4 * nr1) ||
-      B->toff.ensure(8 * nr1) || B->batch.ensure(4 * nr1) || B->cand.ensure(16 * (2 * tasks + 1)) ||
-      B->nF.ensure(4 * nr1) || B->nR.ensure(4 * nr1) || B->ns.ensure(4 * nr1) || B->np.ensure(4 * nr1) ||
-      B->soff.ensure(8 * nr1) || B->poff.ensure(8 * nr1) || B->tiles.ensure(scan_tile_bytes(n)) ||
-      B->queue.ensure(16) || B->counters.ensure(gs::kCounterBytes + gs::kColdBytes) ||
-      B->seg_link.ensure(n_long ? 4 * n_items : 16) ||
-      (dyn_cap &&
-       (B->dyn_items.ensure(16ull * dyn_cap) || B->dyn_meta.ensure(16ull * dyn_cap) ||
-        B->dyn_link.ensure(4ull * dyn_cap) || B->wmeta.ensure(32 * nr1) || B->wlink.ensure(8 * nr1))))
-    return GS_ENOMEM;
+// f(buffer, bytes) for the device buffers of a batch, those of work splitting
+// last; stops where it returns something else than 0.
+template <typename F>
+static int each_buffer(const gs::BatchSizes& z, F&& f) {
+  const uint64_t nr1 = z.n + 1;
+  const struct {
+    DevBuf gs_batch::*buf;
+    uint64_t bytes;
+  } all[] = {
+      {&gs_batch::codes, 16 * (z.chunks + 1)},
+      {&gs_batch::code_off, 8 * nr1},
+      {&gs_batch::items, 8 * (z.items + 1)},
+      {&gs_batch::long_reads, 4 * (z.n_long + 1)},
+      {&gs_batch::item0, 8 * (z.n_long + 1)},
+      {&gs_batch::seg_meta, z.n_long ? 16 * z.items : 16},
+      {&gs_batch::seg_link, z.n_long ? 4 * z.items : 16},
+      {&gs_batch::bases, z.span + 32},
+      {&gs_batch::offs, 8 * nr1},
+      {&gs_batch::lens, 4 * nr1},
+      {&gs_batch::toff, 8 * nr1},
+      {&gs_batch::batch, 4 * nr1},
+      {&gs_batch::cuts, 4 * z.cuts},
+      {&gs_batch::cand, 16 * (2 * z.tasks + 1)},
+      {&gs_batch::nF, 4 * nr1},
+      {&gs_batch::nR, 4 * nr1},
+      {&gs_batch::ns, 4 * nr1},
+      {&gs_batch::np, 4 * nr1},
+      {&gs_batch::soff, 8 * nr1},
+      {&gs_batch::poff, 8 * nr1},
+      {&gs_batch::tiles, scan_tile_bytes(z.n)},
+      {&gs_batch::queue, 16},
+      {&gs_batch::counters, gs::kCounterBytes + gs::kColdBytes},
+      {&gs_batch::dyn_items, 16ull * z.dyn_cap},
+      {&gs_batch::dyn_meta, 16ull * z.dyn_cap},
+      {&gs_batch::dyn_link, 4ull * z.dyn_cap},
+      {&gs_batch::wmeta, z.dyn_cap ? 32 * nr1 : 0},
+      {&gs_batch::wlink, z.dyn_cap ? 8 * nr1 : 0},
+  };
+  for (const auto& b : all)
+    if (const int rc = f(b.buf, b.bytes)) return rc;
   return GS_OK;
+}
+
+uint64_t gs::batch_bytes(const BatchSizes& z) {
+  uint64_t sum = 0;
+  each_buffer(z, [&](DevBuf gs_batch::*, uint64_t bytes) {
+    sum += bytes;
+    return 0;
+  });
+  return sum;
+}
+
+// B's device buffers for these sizes; they only grow.
+static int ensure_buffers(gs_batch* B, const gs::BatchSizes& z) {
+  return each_buffer(z, [&](DevBuf gs_batch::*buf, uint64_t bytes) { return (B->*buf).ensure(bytes); });
 }
 
 // Where the device has no room for the pieces of work splitting, the batch
@@ -1386,10 +1412,9 @@ int gs::batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_
   // every read and long-read segment is an item of each strand; a read has
   // at most as many tasks as bases and code chunks as 32-base spans (+1)
   const uint64_t items = 2 * (reads + bases / seg_tasks + 1);
-  const uint32_t dyn = gs::piece_cap(items);
-  int rc = ensure_buffers(B, bases, reads, bases, 2 * (bases / 32 + reads), items, reads, dyn);
-  // MEM: the first reads of the reference batches, at most every read
-  if (!rc && B->cuts.ensure(4 * (reads + 1))) rc = GS_ENOMEM;
+  // (and its reference batches are no more than the reads)
+  const int rc = ensure_buffers(
+      B, {bases, reads, bases, 2 * (bases / 32 + reads), items, reads, reads, gs::piece_cap(items)});
   if (!rc) {  // the pinned chunks of staged uploads, which do without where there are none
     const size_t up = bases + 12 * reads + 1024, ch = stage_chunk(up);
     (void)have_chunks(B, ch, ch < up ? 2 : 1);
@@ -1547,10 +1572,12 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P, bool wait) {
   B->n_seeds = B->n_pos = 0;
   B->ran = false;
   const uint64_t n = P.n_reads;
-  const bool split_on = P.opts.split_tasks != 0xFFFF;
-  B->dyn_cap = split_on ? gs::piece_cap(B->n_items) : 0u;
-  while (ensure_buffers(B, B->span, n, B->tasks, B->code_chunks, B->n_items, B->n_long, B->dyn_cap))
+  BatchSizes z = plan_sizes(P);
+  B->dyn_cap = z.dyn_cap;
+  while (ensure_buffers(B, z)) {
     if (!give_up_splitting(B)) return GS_ENOMEM;
+    z.dyn_cap = 0;
+  }
   hipStream_t st = B->stream;
   if (hipEventRecord(B->lev[0], st) != hipSuccess) return GS_EHIP;
   const bool one = P.offs.empty();
@@ -1580,7 +1607,6 @@ int gs::batch_load(gs_batch* B, const BatchPlan& P, bool wait) {
       if (PP.n_cuts <= kInlineCuts) {
         std::copy(P.cuts.begin(), P.cuts.end(), PP.cut);
       } else {
-        if (B->cuts.ensure(4 * P.cuts.size())) return GS_ENOMEM;
         PP.cuts = B->cuts.as<uint32_t>();
         if (hipMemcpyAsync(B->cuts.p, P.cuts.data(), 4 * P.cuts.size(), hipMemcpyHostToDevice, st) != hipSuccess)
           return GS_EHIP;
@@ -2391,7 +2417,7 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
     tasks += L >= k ? L - k + 1 : 0;
     chunks += 2 * ((L + 31) / 32);
     const uint32_t nseg = gs::n_segments(L, k, seg_tasks);
-    if (read_is_long(L, k, nseg))
+    if (gs::read_is_long(L, k, nseg))
       ++n_long;
     else
       n_whole += 2ull * nseg;

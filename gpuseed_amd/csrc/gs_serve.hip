@@ -151,21 +151,42 @@ std::unique_ptr<Round> plan_round(gs_server* S) {
   const uint64_t cap_max = S->o.round_bases * (uint64_t)S->o.round_growth;
   const uint64_t cap = grown < S->o.round_bases ? S->o.round_bases : (grown > cap_max ? cap_max : grown);
   const uint64_t mem_cap = S->o.budget_bytes / (uint64_t)(S->o.workers + 1);
-  uint64_t bases = 0, est = 0;
-  // device bytes of a chunk, an upper bound of what plan_device_bytes adds:
-  // bytes, codes, two candidate slots per task, work items and per-read arrays
-  auto chunk_bytes = [](uint64_t b, uint64_t reads) { return b * (1 + 1 + 32 + 24 + 4) + reads * 160; };
+  uint64_t bases = 0;
+  // the round's sizes with one more chunk: what plan_add will add, with as many
+  // reference batches as there can be
+  gs::BatchSizes size{};
+  const uint32_t k = (uint32_t)S->o.opts.k, seg_tasks = S->o.opts.seg_tasks;
+  const uint32_t batch_bases = S->o.opts.batch_bases ? S->o.opts.batch_bases : 1000000u;
+  auto with_chunk = [&](const Request* q, uint64_t end, uint64_t b) {
+    gs::ReadSums sum;
+    uint64_t lo = UINT64_MAX, hi = 0;
+    for (uint64_t i = q->next_read; i < end; ++i) {
+      sum.add(q->lens[i], k, seg_tasks);
+      lo = std::min(lo, q->offs[i]);
+      hi = std::max(hi, q->offs[i] + q->lens[i]);
+    }
+    gs::BatchSizes z = size;
+    z.span += hi - lo;
+    z.n += end - q->next_read;
+    z.tasks += sum.tasks;
+    z.chunks += sum.chunks;
+    z.items += sum.whole + sum.items;
+    z.n_long += sum.n_long;
+    if (!S->o.opts.smem) z.cuts += b / batch_bases + 1;
+    z.dyn_cap = S->o.opts.split_tasks != 0xFFFF ? gs::piece_cap(z.items) : 0u;
+    return z;
+  };
   auto add = [&](Request* q, uint64_t end) -> bool {
     if (end <= q->next_read) return true;
     uint64_t b = 0;
     for (uint64_t i = q->next_read; i < end; ++i) b += q->lens[i];
-    const uint64_t e = chunk_bytes(b, end - q->next_read);
-    if (!R->chunks.empty() && est + e > mem_cap) return false;  // over the budget: a later round
+    const gs::BatchSizes z = with_chunk(q, end, b);
+    if (!R->chunks.empty() && gs::batch_bytes(z) > mem_cap) return false;  // over the budget: a later round
     if (n_reads + (end - q->next_read) > 0x7FFFFFFFull) return false;
     const uint64_t at = n_reads;
     n_reads += end - q->next_read;
     bases += b;
-    est += e;
+    size = z;
     q->sched_bases += b;
     auto piece = std::make_shared<Request::Piece>();
     q->pieces.push_back(piece);

@@ -204,3 +204,40 @@ def test_served_mem_rounds_allocate_no_more_than_smem_rounds(child):
                 print(F.fake_calls(DEVICE) - before)
     """)
     assert out == ["2", "2"]  # seed records and rows
+
+
+@pytest.mark.parametrize("opts", ["seg_tasks=64", "seg_tasks=1", "seg_tasks=64, smem=False, batch_bases=2000",
+                                  "seg_tasks=5, split_tasks=g.NO_SPLIT"])
+@pytest.mark.parametrize("n,length", [(20_000, 150), (300, 4000)])
+def test_a_round_s_device_bytes_are_those_it_allocates(child, opts, n, length):
+    """peak_round_bytes against the buffers of a batch of the same reads (each
+    allocated with a quarter and 256 bytes of headroom)."""
+    out = child("""
+        X = index()
+        r = reads(%d, %d)
+        kw = dict(dict(k=19, smem=True, kernel=3), **dict(%s))
+        before = F.fake_held(DEVICE)
+        b = g.Batch(X, r, **kw)
+        held = F.fake_held(DEVICE) - before
+        b.close()
+        with g.Server(X, workers=1, round_bases=10_000_000, **kw) as S:
+            S.wait(S.submit(r))
+            peak = S.stats().peak_round_bytes
+        print(0 <= held - 1.25 * peak <= 40 * 256, held, peak)
+    """ % (n, length, opts))
+    assert out[0] == "True", out
+
+
+@pytest.mark.parametrize("seg_tasks", [1, 3, 64])
+def test_rounds_stay_within_their_budget(child, seg_tasks):
+    out = child("""
+        X = index()
+        with g.Server(X, budget_bytes=16_000_000, workers=1, round_bases=1_000_000, k=19, smem=True, batch_bases=5000,
+                      seg_tasks=%d) as S:
+            rs = [reads(5, 2000 + i) for i in range(100)] + [reads(1000, 100 + i) for i in range(5)]
+            for t in [S.submit(r) for r in rs]:
+                S.wait(t)
+            st = S.stats()
+            print(st.peak_round_bytes <= 8_000_000, st.peak_round_bytes > 4_000_000, st.peak_round_bytes, st.n_rounds)
+    """ % seg_tasks)
+    assert out[:2] == ["True", "True"], out

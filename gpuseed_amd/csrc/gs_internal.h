@@ -120,7 +120,7 @@ struct PersistParams {
   const uint64_t* task_off;
   const uint64_t* items;
   uint64_t n_items;
-  uint32_t n_reads, n_long, k, smem, seg_tasks;
+  uint32_t n_long, k, smem, seg_tasks;
   uint4* cand;               // same candidate layout as the plain kernel
   uint32_t* nF;
   uint32_t* nR;
@@ -161,7 +161,7 @@ struct JoinParams {
   uint32_t n_reads, dyn_cap;
 };
 
-constexpr uint32_t kSplitStream = 0xFFFFFFFFu;  // nF/nR of a whole-read stream left for join_whole
+constexpr uint32_t kSplitStream = 0xFFFFFFFFu;  // nF/nR of a whole-read stream left for join_whole_wave/thread
 // Work splitting (take_pieces): a lane gives half of its task ends away after
 // kSplitWork memory operations (at once in a launch of fewer items than
 // lanes), while it has at least 2 * kSplitTasks of them left, and once
@@ -176,8 +176,8 @@ constexpr uint32_t kSplitStream = 0xFFFFFFFFu;  // nF/nR of a whole-read stream 
 // 3.26, 3.18, 3.47 ms, 60,000 6.69, 6.56, 6.35, 6.26, in MEM mode 3.88, 4.04,
 // 3.95, 3.96; 500,000 150 bp reads 3.97, 4.03, 4.38, 4.43.  kSplitTasksPlain
 // (a plain task has no shortcuts, and so more steps): with 1, 2 and 4 10,000
-// uneven reads on a 100 Mbp index 2.74, 2.89, 3.42 ms, 300,000 150 bp reads
-// 3.64, 3.66, 3.93.
+// uneven reads on a 100 Mbp index 2.60, 2.71, 3.20 ms, 300,000 150 bp reads
+// 4.32, 4.41, 4.59.
 constexpr uint32_t kSplitWork = 64;
 constexpr uint32_t kSplitTasks = 2, kSplitTasksPlain = 1, kSplitTasksLong = 8;
 constexpr uint32_t kSplitIdle = 32;
@@ -300,7 +300,8 @@ uint64_t plan_device_bytes(const BatchPlan& P);  // device buffers the plan need
 gs_batch* batch_new(gs_index* X, bool hold = true);
 int batch_load(gs_batch* B, const BatchPlan& P, bool wait = true);
 // Grows B's device buffers for any plan of at most `bases` bases and `reads`
-// reads, so that loading such plans allocates (and synchronises) nothing.
+// reads, so that loading such plans allocates (and synchronises) nothing (but
+// tries again for pinned chunks that it could not have).
 int batch_reserve(gs_batch* B, uint64_t bases, uint64_t reads, uint32_t seg_tasks);
 void batch_free(gs_batch* B);
 

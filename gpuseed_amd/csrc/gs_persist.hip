@@ -1389,13 +1389,14 @@ int launch_t(const gs::PersistParams& P, unsigned grid, hipStream_t st, hipEvent
     // waves: the kernel is bound by the instructions that its waves issue, so
     // that a second wave on a SIMD costs more than lanes that share one.
     // Kernel time with as many waves as fit against this: 10,000 100 bp reads
-    // on a 1 Mbp index 1.05 -> 0.44 ms, 50,000 and 100,000 150 bp reads on a
-    // 100 Mbp index 2.75 -> 1.31 and (plain kernel) 4.62 -> 2.05 ms, 60,000
-    // on the 3.1 Gbp index 2.72 -> 1.42 ms.  A wave's items lie n_waves apart
-    // (next to each other: 3000 uneven reads on a 100 Mbp index 0.99 -> 0.91
-    // ms, 10,000 with the plain kernel 3.4 -> 2.9).  From the queue, with any
-    // number of waves, 3000 uneven reads take 1.06 ms and 100,000 150 bp reads
-    // 1.72 (here 1.65); at 130,000 the two are equal.
+    // on a 1 Mbp index 1.05 -> 0.44 ms, 50,000 150 bp reads on a 100 Mbp index
+    // 2.75 -> 1.31 ms, 60,000 on the 3.1 Gbp index 2.72 -> 1.42 ms.  A wave's
+    // items lie n_waves apart (next to each other: 3000 uneven reads on a 100
+    // Mbp index 0.99 -> 0.91 ms).  From the queue, with any number of waves,
+    // 3000 uneven reads take 1.06 ms and 100,000 150 bp reads 1.72 (here 1.65);
+    // at 130,000 the two are equal.  Shares for more waves than fit at once are
+    // no gain (plain kernel, 6 waves per CU, 100,000 reads: calls of 3.3 ms from
+    // the queue, 3.9 so).
     const uint64_t simds = std::max(1u, 4 * compute_units());
     A.take = (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, (P.n_items + simds - 1) / simds));
     A.n_waves = (uint32_t)((P.n_items + A.take - 1) / A.take);

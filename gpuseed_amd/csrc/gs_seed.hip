@@ -1240,10 +1240,10 @@ static void destroy_batch(gs_batch* B) {
 }
 
 // ---- host plan of a batch -----------------------------------------------------
-// Everything gs_batch_create derives on the CPU: the byte pieces to upload, the
-// offsets rebased onto them, task offsets, reference-batch ids, code chunks and
-// the persistent kernel's work items.  A plan can hold several groups of reads
-// (one per request of a server round); batch ids never span two groups.
+// What gs_batch_create derives on the CPU: the byte pieces to upload, the sizes
+// of everything else and the first reads of the reference batches; the rest
+// follows on the device (launch_plan).  A plan can hold several groups of
+// reads (one per request of a server round); batch ids never span two groups.
 
 int gs::plan_check(const gs_opts* o) {
   if (!o) return GS_EINVAL;
@@ -1722,7 +1722,6 @@ static int enqueue_extension(gs_batch* B, const SeedParams& S, int kernel, unsig
   PP.task_off = S.task_off;
   PP.items = B->items.as<uint64_t>();
   PP.n_items = B->n_items;
-  PP.n_reads = S.n_reads;
   PP.n_long = B->n_long;
   PP.k = S.k;
   PP.smem = S.smem;
@@ -2308,10 +2307,9 @@ extern "C" GS_API void gs_result_free(gs_result* r) {
 // ---- gs_seed_noalloc: the same pipeline without any allocation --------------
 // Every device buffer of the call is a slice of `scratch`, a file-scope array
 // that each GPU holds from the library's load to the end of the process.  The
-// host side keeps no vectors either: the task map, code-chunk offsets, work
-// items and reference-batch ids that gs_batch_create plans on the CPU are
-// computed on the device from the uploaded offsets and lengths.  Calls on
-// one GPU share its array, so calls that overlap on one GPU race.
+// host side keeps no vectors either: where the list of reference batches is
+// long, the device finds them (noalloc_batch_ids).  Calls on one GPU share its
+// array, so calls that overlap on one GPU race.
 
 namespace {
 
@@ -2431,7 +2429,9 @@ extern "C" GS_API int gs_seed_noalloc(gs_index* X, const char* bases, const uint
   // its first layout: reads of at most 160 bases with a batched kernel need
   // their codes and two work items each, every other call the plain kernel
   // seed_streams, which needs none, but for reads of more than 256 bases a
-  // size record per base and strand; the outputs come after that.
+  // size record per base and strand; the outputs come after that.  (o_spare held
+  // the tile totals of an earlier scan; it stays, so that the largest call that
+  // fits is the same.)
   uint64_t at = 0;
   auto take = [&](uint64_t bytes) {
     const uint64_t o = at;

@@ -226,7 +226,9 @@ GS_API int gs_index_read_pairs(const gs_index* idx, uint64_t first, uint64_t cou
  * them, row primary+1 behaviour included (locate_seeds_gpu with
  * bwt_inv_psi_gpu, seed_gen.cu:455-484, 668-684); rows past seq_len and row
  * 0 give 0xFFFFFFFF.  From the full suffix array when the index has the
- * direct-extension structures, else by the sampled-suffix-array walk. */
+ * direct-extension structures, else by the sampled-suffix-array walk.  `rows`
+ * and `out` may be one array or overlap.  Calls on one index follow each
+ * other. */
 GS_API int gs_index_locate(gs_index* idx, const uint32_t* rows, uint64_t n, uint32_t* out);
 /* Rows [first, first+count) of the full suffix array and positions
  * [first, first+count) of its inverse and of the text (one code 0..3 per
@@ -269,23 +271,22 @@ typedef struct {
   uint32_t batch_bases; /* MEM look-ahead stays inside batches closed at this
                        many bases (seed_gen.cu:2814, 2955); 0 = 1,000,000     */
   int kernel;       /* 0: plain kernel (the drop-in): no pair probes, direct
-                          runs or tandem jumps;
+                          runs or tandem jumps, 16-bit size records;
                        1: batched persistent kernel, 8-bit size records;
                        2: batched persistent kernel, 16-bit size records;
                        3: batched persistent kernel, 4-bit size records (a
                           smaller LDS slot, so more waves per CU)             */
-  uint32_t seg_tasks; /* batched kernels: reads longer than 160 bases are cut
-                       into work items of this many task ends, 1..112
-                       (0 = 64)                                               */
+  uint32_t seg_tasks; /* reads longer than 160 bases are cut into work items of
+                       this many task ends, 1..112 (0 = 64)                   */
   uint16_t wg;        /* batched kernels: workgroup size 64, 128 or 256 (0 = 128) */
   uint16_t walk_rows; /* suffix-array walk: rows per thread 1, 2 or 4 (0 = 1) */
-  uint16_t split_tasks; /* batched kernels: once a launch's work queue is
-                       exhausted, an item that has used split_work memory
-                       operations hands half of its task ends to an idle
-                       lane of its wave while at least 2 * split_tasks
-                       remain, 1..64 (0: 1 in the plain kernel, 8 where a
-                       large SMEM launch holds reads in segments, else 2);
-                       0xFFFF: no splitting                                  */
+  uint16_t split_tasks; /* once a launch's work queue is exhausted, an item
+                       that has used split_work memory operations hands half
+                       of its task ends to an idle lane of its wave while at
+                       least 2 * split_tasks remain, 1..64 (0: 1 in the plain
+                       kernel, 8 where a large SMEM launch holds reads in
+                       segments, else 2); 0xFFFF: no splitting; a batch whose
+                       device has no room for the pieces runs without it too */
   uint16_t split_work;  /* in units of 64 memory operations, 1..0xFFFE (0 = 1,
                        and none in a launch of fewer items than lanes)       */
   uint16_t direct_min;  /* batched kernels on an index with gs_index_set_direct:
@@ -341,11 +342,11 @@ GS_API void gs_result_free(gs_result* res);
  * buffers do not fit the array returns GS_ERANGE (about 7 million bases of
  * 150 bp reads per call; candidates take 32 bytes per base); so does a call
  * whose seeds or positions exceed seeds_cap or pos_cap, with n_seeds and
- * n_pos set to what it needs.  Output equals gs_seed's.  The persistent
- * kernel runs when every read fits its 160-base window (opts->kernel 1..3),
- * else the plain kernel.  Calls on one GPU share the array: calls that
- * overlap on one GPU race.  Runs on the index's stream.  No counterpart in
- * the reference. */
+ * n_pos set to what it needs.  Output equals gs_seed's.  The kernel that
+ * gs_seed would run runs where its work items fit the array too, else
+ * one stream per lane (the same output, later).  Calls on one GPU share the
+ * array: calls that overlap on one GPU race.  Runs on the index's stream.  No
+ * counterpart in the reference. */
 typedef struct {
   uint32_t* read_nseeds;   /* [n_reads]                                       */
   uint32_t* read_npos;     /* [n_reads]                                       */

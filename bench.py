@@ -619,10 +619,12 @@ def main():
         log("one batch host to host: gs_seed %.1f ms, graph replay %.1f ms (%.0f reads/s)" %
             (e2e["drop_in_call_ms"], e2e["graph_replay_ms"], e2e["graph_reads_per_s"]))
 
-    # random-access ceiling of this GPU (16-byte dependent requests, 8 GiB)
-    rr = g.roofline_random(8 << 30, line_bytes=16, mode=1, inflight=1, grid=2048, iters=512, reps=3)
-    r_max = rr.lines_per_s
-    log("random-access ceiling: %.1f G requests/s" % (r_max / 1e9))
+    # random access on this GPU, dependent 16-byte requests: over 8 GiB, all
+    # from HBM (a mix of smaller and larger tables can pass that rate), and
+    # over 64 MiB, from the last-level cache, which none has passed
+    r_hbm, r_max = (g.roofline_random(size, line_bytes=16, mode=1, inflight=1, grid=2048, iters=512, reps=3).lines_per_s
+                    for size in (8 << 30, 64 << 20))
+    log("random access: %.1f G requests/s over 8 GiB, %.1f over 64 MiB" % (r_hbm / 1e9, r_max / 1e9))
 
     cpu = None
     nproc, avail = host_cpus()
@@ -675,9 +677,9 @@ def main():
         # every request that misses L2 moves one 128-byte line from HBM: the
         # kernel's own request count over the timed launches times the L2
         # miss share rocprofv3 measured on this workload, against the
-        # measured ceiling of dependent random 16-byte requests (all misses)
+        # highest rate of dependent random 16-byte requests (64 MiB)
         ra = {"requests_per_read_model": req_per_read, "requests_per_read_issued": issued,
-              "measured_ceiling_requests_per_s": r_max}
+              "measured_ceiling_requests_per_s": r_max, "probe_8gib_requests_per_s": r_hbm}
         if sample_counts:
             sc = sample_counts
             ra["requests_per_read_issued_on_model_sample"] = (sc["table"] + sc["occ"] + sc["direct"] + sc["tandem"]) / sc["reads"]
